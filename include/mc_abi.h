@@ -255,16 +255,14 @@ int mc_align_movie(mc_context ctx, const mc_movie_desc *movie, const mc_params *
  * B-factor, precision form and noise window form a group, whatever their
  * transform sizes; a group is split into sub-batches whose resident spectra
  * and pair-stage buffers fit in device memory (MC_BATCH_MEM_MB, default 60%
- * of the free memory).  In a sub-batch, stage 1 runs per movie; the pair
- * column pass of every movie on the default column kernel is one persistent
- * launch sequence across sizes (a plan table, one record per movie), the
- * others keep per-movie launches; the row pass and the peak search run once
+ * of the free memory).  In a sub-batch, stage 1 and the pair column pass run
+ * per movie; the row pass and the peak search run once
  * per transform size; the drift model runs per movie on the host; each
  * align-to-sum round of the movies still iterating (all sizes) is one HIP
  * graph, captured once and replayed while that set of movies is unchanged;
  * the final sums run per movie.  Every movie gets bit for bit the results
- * mc_align_movie would give it: alone, a movie runs the same kernels (the
- * default column kernel with its one plan), and the row pass's summation
+ * mc_align_movie would give it: alone, a movie runs the same kernels, and the
+ * row pass's summation
  * order depends on n only.  The ms_* fields of its report are those of its
  * sub-batch.  The movies' frame buffers must all be resident. */
 typedef struct {
@@ -294,9 +292,9 @@ int mc_align_batch(mc_context ctx, const mc_batch_item *items, int count,
  *            1024 to 8192, the radix plan of its FFT (balanced, reversed
  *            order, radix-8 chain) x its LDS index padding (one float2 per
  *            16, or none);
- *   pair stage (FP32 form): column kernel (M=128, M=128 with next-item
- *            prefetch, M-generic, M=128 at 4 waves per SIMD) and row kernel
- *            (FP32 MFMA with 4 or 8 waves per pair, vector ALU).
+ *   pair stage (FP32 form): row kernel (FP32 MFMA with 4 or 8 waves per
+ *            pair, vector ALU); the column pass has one kernel per size,
+ *            whose time is reported.
  * Each candidate runs once untimed and 3 times timed (minimum kept); the
  * context's resident spectra are overwritten, so the stage entry points need
  * mc_load_frames again afterwards.  With
@@ -304,21 +302,20 @@ int mc_align_batch(mc_context ctx, const mc_batch_item *items, int count,
  * ({"arch", "cus", "nu", "n", "dtype", "box", "precision", "r2c", "chunk",
  * "cols", "rows"}); mc_tune_load reads the lines of the same device type
  * back (later lines win).  Without tuning, the defaults are 4x512 (4x256
- * below 4096), 192 MB of row-pass scratch per launch, the M=128 column
- * pass (the batched plan kernel up to n = 3840, the 4-wave kernel at 4096,
- * the plain one above) and the streaming FP32 MFMA row kernel. */
+ * below 4096), 192 MB of row-pass scratch per launch and the streaming FP32
+ * MFMA row kernel. */
 typedef struct {
   int r2c_variant;        /* 1: 4x256, 2: 2x256, 3: 4x512; +8: persistent
                              column pass with register twiddles           */
   int chunk_frames;       /* frames per stage-1 launch                      */
-  int pair_cols_variant;  /* 0: M=128, 1: M=128 + prefetch, 2: M-generic,
-                             3: M=128 at 4 waves per SIMD                 */
+  int pair_cols_variant;  /* 0 (cache files may hold 0 to 3: the codes of former
+                             column kernels; all run the same one)        */
   int pair_rows_variant;  /* 0: FP32 MFMA streaming (box <= 96), 1: vector
                              ALU, 2: FP32 MFMA through LDS (8 waves),
                              3: FP32 MFMA through LDS (4 waves)             */
   float ms_stage1[2][4][4]; /* [column pass: per column, persistent]
                                [row shape][chunk 1, 2, 4, 8]; 0 = not run  */
-  float ms_pair_cols[4];  /* 0 = not run                                    */
+  float ms_pair_cols[4];  /* [0]: the column pass; the others 0             */
   float ms_pair_rows[4];
   int cols_plan;          /* per-column pass of stage 1: radix plan cols_plan/2
                              (0 balanced, 1 reversed order, 2 radix-8 chain)

@@ -92,7 +92,7 @@ struct mc_context_s {
   int device = 0;
   hipStream_t st = nullptr;
   DevBuf spec, rt, rowsum, fill, padP, pairs_d, tbuf, box, boxpart, peaks, shifts, image, tmp, means,
-      sum2img, wk, gpart, gout, jobs, tmax, fsc, disp, plans;
+      sum2img, wk, gpart, gout, jobs, tmax, fsc, disp;
   int graph_captures = 0, graph_replays = 0;
   // autotuned launch shapes (mc_autotune / mc_tune_load)
   struct Tune {
@@ -1218,20 +1218,16 @@ static void use_group(mc_context_s* c, const SizeGroup& g) {
 struct PairSpan {
   int gi = 0, np = 0;
   size_t po = 0, to = 0;
-  int cols = mc::PAIR_COLS_AUTO, body = -1;
+  int cols = mc::PAIR_COLS_AUTO;
 };
 struct PairPlan {
   std::vector<PairSpan> sp;
   size_t np = 0;
-  long long items[2] = {0, 0};  // plan-kernel items of each register class
-  int nplans[2] = {0, 0};       // class-0 table, then the class-1 table
   float bfactor = 0.f;
   int box = 0, wnoise = 0, precision = 0;
 };
 
-// Reserves the pair buffers and uploads pairs (host slot pairs, span by span)
-// and the column-pass plan table.  With more than one span the spans that
-// the plan kernel covers run as one launch sequence (mc::PairColsPlan).
+// Reserves the pair buffers and uploads pairs (host slot pairs, span by span).
 static int pairs_prepare(mc_context_s* c, const std::vector<SizeGroup>& gs, PairPlan& L,
                          const std::vector<int>& slots) {
   size_t np = 0, tel = 0, part = 0, pscr = 0;
@@ -1245,10 +1241,6 @@ static int pairs_prepare(mc_context_s* c, const std::vector<SizeGroup>& gs, Pair
     gnp[q.gi] += q.np;
     const mc_context_s::Tune* tn = pair_tune(c, n, L.box, L.precision);
     q.cols = tn ? tn->cols : mc::PAIR_COLS_AUTO;
-    // several movies: the default-variant ones share one plan table (a
-    // single movie runs the same plan kernel with its plan passed by value)
-    q.body = (L.precision == MC_PREC_FP32 && L.sp.size() > 1)
-                 ? mc::pair_cols_plan_body(n, L.box, q.cols) : -1;
   }
   for (size_t g = 0; g < gs.size(); g++) {
     part = std::max(part, mc::pair_rows_part_elems((int)gnp[g], gs[g].n, L.box));
@@ -1264,52 +1256,17 @@ static int pairs_prepare(mc_context_s* c, const std::vector<SizeGroup>& gs, Pair
   HIP_TRY(c->peaks.ensure(sizeof(double) * (3 * np + pscr + 1)));
   HIP_TRY(hipMemcpyAsync(c->pairs_d.p, slots.data(), sizeof(int) * slots.size(), hipMemcpyHostToDevice,
                          c->st));
-  std::vector<mc::PairColsPlan> plans[2];
-  for (int k = 0; k < 2; k++) L.items[k] = 0;
-  for (const PairSpan& q : L.sp) {
-    if (q.body < 0 || q.np == 0) continue;
-    const SizeGroup& g = gs[q.gi];
-    const int k = mc::pair_cols_plan_class(q.body);
-    mc::PairColsPlan pl;
-    pl.spectra = c->spec.as<float2>() + g.off;
-    pl.pairs = c->pairs_d.as<int2>() + q.po;
-    pl.wxy = mc::pair_weights(g.n, L.bfactor);
-    pl.tw = mc::twiddles(g.n);
-    if (!pl.wxy || !pl.tw) return set_err(MC_ERR_DEVICE, "pair tables for n %d", g.n);
-    pl.tbuf = c->tbuf.as<float2>() + q.to;
-    pl.spec_stride = g.stride;
-    pl.item0 = L.items[k];
-    pl.npairs = q.np;
-    pl.box = L.box;
-    pl.body = q.body;
-    plans[k].push_back(pl);
-    L.items[k] += (long long)q.np * (g.n / 2 + 1);
-  }
-  for (int k = 0; k < 2; k++) L.nplans[k] = (int)plans[k].size();
-  plans[0].insert(plans[0].end(), plans[1].begin(), plans[1].end());
-  if (!plans[0].empty()) {
-    HIP_TRY(c->plans.ensure(sizeof(mc::PairColsPlan) * plans[0].size()));
-    HIP_TRY(hipMemcpyAsync(c->plans.p, plans[0].data(), sizeof(mc::PairColsPlan) * plans[0].size(),
-                           hipMemcpyHostToDevice, c->st));
-    // the host vector goes out of scope: the copy must have read it
-    HIP_TRY(hipStreamSynchronize(c->st));
-  }
   return MC_OK;
 }
 
-// Column pass (plan kernel and per-span launches), then the row pass and the
-// peak search per size group.  Results: peaks (3 doubles per pair, span
+// Column pass per span, then the row pass and the peak search per size group.  Results: peaks (3 doubles per pair, span
 // order) and box maps.  Capturable.
 static int pairs_launch(mc_context_s* c, const std::vector<SizeGroup>& gs, const PairPlan& L) {
   const int box = L.box;
   {
     KScope ks(c, MC_KT_PAIR_COLS);
-    for (int k = 0; k < 2; k++)
-      if (L.nplans[k] > 0)
-        HIP_TRY(mc::launch_pair_cols_plans(c->plans.as<mc::PairColsPlan>() + (k ? L.nplans[0] : 0),
-                                           L.nplans[k], L.items[k], k, c->st));
     for (const PairSpan& q : L.sp) {
-      if (q.body >= 0 || q.np == 0) continue;
+      if (q.np == 0) continue;
       const SizeGroup& g = gs[q.gi];
       float* tmax = L.precision == MC_PREC_MFMA_HILO ? c->tmax.as<float>() + q.to / box : nullptr;
       HIP_TRY(mc::launch_pair_cols(c->spec.as<float2>() + g.off, g.stride,
@@ -1419,8 +1376,7 @@ struct GroupTimes {
 // of any transform sizes, whose spectra fit together in device memory
 // (callers order them by size): stage 1 per movie into its size group's
 // region, then one pair stage over every pair of every movie (the column
-// pass as one plan-kernel launch sequence across sizes when there are
-// several movies), the host drift model per movie, align-to-sum rounds over
+// pass per movie, row pass and peak search per size), the host drift model per movie, align-to-sum rounds over
 // the movies still iterating (one graph replay per round), and the final sum
 // per movie.
 static int align_group(mc_context_s* c, std::vector<MovieRun*>& rs, bool use_graph,
@@ -1945,27 +1901,17 @@ extern "C" int mc_autotune(mc_context ctx, const mc_movie_desc* m, const mc_para
                          hipMemcpyHostToDevice, c->st));
   int bcol = mc::PAIR_COLS_AUTO, brow = mc::PAIR_ROWS_AUTO;
   if (p->precision == MC_PREC_FP32) {
-    best = 1e30f;
-    for (int v = 0; v < mc::PAIR_COLS_VARIANTS; v++) {
-      if (v != mc::PAIR_COLS_GENERIC && !(n >= 512 && box <= 128)) continue;
+    {  // one column kernel per size: its time is reported
       float ms = 0;
       MC_TRY(time_min(c, reps, &ms, [&] {
         const hipError_t e = mc::launch_pair_cols(slot(c, 0), c->spec_stride,
                                                   c->pairs_d.as<int2>(), r.P, n, p->bfactor, box,
                                                   c->tbuf.as<float2>(), c->tmax.as<float>(),
-                                                  p->precision, v, c->st);
+                                                  p->precision, bcol, c->st);
         return e == hipSuccess ? MC_OK : set_err(MC_ERR_DEVICE, "pair columns: %s", hipGetErrorString(e));
       }));
-      tr.ms_pair_cols[v] = ms;
-      if (ms < best) {
-        best = ms;
-        bcol = v;
-      }
+      tr.ms_pair_cols[bcol] = ms;
     }
-    // The default variant is the plan kernel that mc_align_batch shares across
-    // movies: it is kept unless another one is more than 2% faster.
-    if (tr.ms_pair_cols[mc::PAIR_COLS_AUTO] > 0 && tr.ms_pair_cols[mc::PAIR_COLS_AUTO] <= 1.02f * best)
-      bcol = mc::PAIR_COLS_AUTO;
     best = 1e30f;
     for (int v = 0; v < mc::PAIR_ROWS_VARIANTS; v++) {
       if (v != mc::PAIR_ROWS_VALU && box > 96) continue;

@@ -43,6 +43,46 @@ MC_DEV float2 buf_ld2(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
   return make_float2(v.x, v.y);
 }
 
+// 16 bytes per lane: the vector L1 delivers 64 B/clk to 16-byte loads and 32
+// to 8- and 4-byte ones (measured: 35 against 19 TB/s out of L2).
+MC_DEV float4 buf_ld4(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  typedef float f4v __attribute__((ext_vector_type(4)));
+  const f4v v = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+  return make_float4(v.x, v.y, v.z, v.w);
+}
+
+MC_DEV void buf_st2(__amdgpu_buffer_rsrc_t r, int voff, float2 v) {
+  typedef unsigned u2v __attribute__((ext_vector_type(2)));
+  __builtin_amdgcn_raw_buffer_store_b64(u2v{__float_as_uint(v.x), __float_as_uint(v.y)}, r, voff, 0, 0);
+}
+
+// ------------------------------------------------- cross-lane and LDS order
+// swap32: the upper 32 lanes of a change places with the lower 32 lanes of b.
+// swap16: the odd rows of 16 lanes of a with the even rows of b.
+MC_DEV void swap32(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+MC_DEV void swap16(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+// LDS accesses before it are ordered before those after it, among the lanes
+// of a wave (the LDS pipe keeps a wave's order, so this costs nothing) ...
+MC_DEV void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+// ... and among the waves of a workgroup; global loads stay in flight.
+MC_DEV void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // twiddle e^{S * 2 pi i e / N} from a table t[e] = e^{+2 pi i e / N}
 template <int S> MC_DEV float2 twid(const float2* t, int e) {
   float2 w = t[e];
@@ -87,19 +127,20 @@ template <int S> MC_DEV void dft8(float2* v) {
   v[7] = csub(e3, o3);
 }
 
-template <int S> MC_DEV void dft16(float2* v) {
-  // 16 = 4 x 4: X[k1 + 4 k2] = sum_n2 W4^{n2 k2} W16^{n2 k1} sum_n1 v[n2 + 4 n1] W4^{n1 k1}
+// 16 = 4 x 4: X[k1 + 4 k2] = sum_n2 W4^{n2 k2} W16^{n2 k1} sum_n1 x[n2 + 4 n1] W4^{n1 k1}.
+// dft16_rest takes v[r] = x[r] + x[r + 8] and v[r + 8] = x[r] - x[r + 8], r < 8.
+template <int S> MC_DEV void dft16_rest(float2* v) {
   const float c1 = 0.92387953251128675613f;  // cos(pi/8)
   const float s1 = 0.38268343236508977173f;  // sin(pi/8)
   const float c2 = 0.70710678118654752440f;
   float2 a[4][4];
 #pragma unroll
   for (int n2 = 0; n2 < 4; n2++) {
-    a[n2][0] = v[n2];
-    a[n2][1] = v[n2 + 4];
-    a[n2][2] = v[n2 + 8];
-    a[n2][3] = v[n2 + 12];
-    dft4<S>(a[n2][0], a[n2][1], a[n2][2], a[n2][3]);
+    const float2 t0 = v[n2], t1 = v[n2 + 8], t2 = v[n2 + 4], t3 = mul_si<S>(v[n2 + 12]);
+    a[n2][0] = cadd(t0, t2);
+    a[n2][2] = csub(t0, t2);
+    a[n2][1] = cadd(t1, t3);
+    a[n2][3] = csub(t1, t3);
   }
   // twiddles W16^{n2 k1}, exponent e = n2*k1 in {0..9}
   // W16^1 = (c1, S s1), ^2 = (c2, S c2), ^3 = (s1, S c1), ^4 = S i,
@@ -122,6 +163,16 @@ template <int S> MC_DEV void dft16(float2* v) {
     v[k1 + 8] = b2;
     v[k1 + 12] = b3;
   }
+}
+
+template <int S> MC_DEV void dft16(float2* v) {
+#pragma unroll
+  for (int r = 0; r < 8; r++) {
+    const float2 a = v[r], b = v[r + 8];
+    v[r] = cadd(a, b);
+    v[r + 8] = csub(a, b);
+  }
+  dft16_rest<S>(v);
 }
 
 // X[k] = sum_n v[n] W3^{S n k}: W3 = -1/2 + S i sqrt(3)/2.
@@ -226,8 +277,47 @@ template <int S> MC_DEV void dft11(float2* v) {
   v[0] = x0;
 }
 
+// DFT_16 of w[r] v[r] (real weights): the weights go into the additions of the
+// first radix-2 layer, w_a a +- w_b b, instead of 32 products before it.
+template <int S> MC_DEV void dft16w(float2* v, const float* w) {
+#pragma unroll
+  for (int r = 0; r < 8; r++) {
+    const float2 a = v[r], b = cscale(v[r + 8], w[r + 8]);
+    v[r] = make_float2(fmaf(w[r], a.x, b.x), fmaf(w[r], a.y, b.y));
+    v[r + 8] = make_float2(fmaf(w[r], a.x, -b.x), fmaf(w[r], a.y, -b.y));
+  }
+  dft16_rest<S>(v);
+}
+
+// DFT of length N1 N2 (coprime) without twiddles: inputs n = N2 n1 + N1 n2
+// mod N, outputs k = k1 mod N1 = k2 mod N2.
+template <int R, int S> MC_DEV void dft(float2* v);
+template <int N1, int N2, int S> MC_DEV void dft_pfa(float2* v) {
+  constexpr int N = N1 * N2;
+  float2 a[N1][N2];
+#pragma unroll
+  for (int n1 = 0; n1 < N1; n1++) {
+#pragma unroll
+    for (int n2 = 0; n2 < N2; n2++) a[n1][n2] = v[(N2 * n1 + N1 * n2) % N];
+    dft<N2, S>(a[n1]);
+  }
+  float2 b[N2][N1];
+#pragma unroll
+  for (int k2 = 0; k2 < N2; k2++) {
+#pragma unroll
+    for (int n1 = 0; n1 < N1; n1++) b[k2][n1] = a[n1][k2];
+    dft<N1, S>(b[k2]);
+  }
+#pragma unroll
+  for (int k = 0; k < N; k++) v[k] = b[k % N2][k % N1];
+}
+
 template <int R, int S> MC_DEV void dft(float2* v) {
   if constexpr (R == 2) dft2<S>(v);
+  else if constexpr (R == 6) dft_pfa<2, 3, S>(v);
+  else if constexpr (R == 10) dft_pfa<2, 5, S>(v);
+  else if constexpr (R == 12) dft_pfa<4, 3, S>(v);
+  else if constexpr (R == 14) dft_pfa<2, 7, S>(v);
   else if constexpr (R == 3) dft3<S>(v);
   else if constexpr (R == 4) dft4<S>(v);
   else if constexpr (R == 5) dft5<S>(v);
@@ -235,7 +325,7 @@ template <int R, int S> MC_DEV void dft(float2* v) {
   else if constexpr (R == 11) dft11<S>(v);
   else if constexpr (R == 8) dft8<S>(v);
   else if constexpr (R == 16) dft16<S>(v);
-  else static_assert(R == 2 || R == 3 || R == 4 || R == 5 || R == 7 || R == 8 || R == 11 || R == 16, "radix");
+  else static_assert(R == 2, "radix");
 }
 
 // ------------------------------------------- direct DFT of an odd length

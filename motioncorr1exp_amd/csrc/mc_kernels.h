@@ -9,11 +9,11 @@ namespace mc {
 // Grid of a persistent kernel on the current device: CUs x resident
 // workgroups per CU (occupancy query), a multiple of 8 so that every XCD
 // gets the same share (workgroup b runs on XCD b % 8), at least 8.
-template <class K> inline int persistent_grid(K kernel, int nt) {
+template <class K> inline int persistent_grid(K kernel, int nt, size_t lds = 0) {
   int dev = 0, cus = 256, per = 1;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, nt, 0) != hipSuccess || per < 1)
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, nt, lds) != hipSuccess || per < 1)
     per = 1;
   const int g = (cus * per) / 8 * 8;
   return g < 8 ? 8 : g;
@@ -103,49 +103,27 @@ hipError_t launch_spectrum_to_image(const float2* spec, int n, float scale, floa
 // stage of the column pass and the row pass as FP16 hi/lo MFMA products
 // (tmax: npairs*(n/2+1) floats of column maxima, written by the column pass
 // and read by the row pass).
-// Plain-form variants (the hi/lo form has one kernel per pass):
-//   column pass: AUTO = the M = 128 persistent kernel (n >= 512, box <= 128),
-//   M128_PF = the same with next-item register prefetch (fewer resident
-//   workgroups), GENERIC = the M-generic persistent kernel, M128_W4 = M = 128
-//   compiled for 4 waves per SIMD (128 VGPRs); row pass: AUTO = FP32 MFMA
+// The column pass has one kernel per size and form (`variant` is one of the
+// codes that tuning files may hold; all run it).  Row-pass variants of the plain
+// form: AUTO = FP32 MFMA
 //   streaming each wave's kx range from memory (box <= 96; from n = 2048
 //   the kx range is also split over workgroups, a count set by n alone, whose
 //   partial maps go to `part`, pair_rows_part_elems(npairs, n, box) floats,
 //   and are added in order), VALU = register-tiled vector ALU kernel, MFMA8 / MFMA4 = FP32
 //   MFMA staged through LDS with 8 / 4 waves per (pair, 32-row block).
-enum { PAIR_COLS_AUTO = 0, PAIR_COLS_M128_PF = 1, PAIR_COLS_GENERIC = 2, PAIR_COLS_M128_W4 = 3,
-       PAIR_COLS_VARIANTS = 4 };
+enum { PAIR_COLS_AUTO = 0, PAIR_COLS_VARIANTS = 4 };
 enum { PAIR_ROWS_AUTO = 0, PAIR_ROWS_VALU = 1, PAIR_ROWS_MFMA8 = 2, PAIR_ROWS_MFMA4 = 3,
        PAIR_ROWS_VARIANTS = 4 };
 bool pair_form_supported(int precision, int n, int box);
 hipError_t launch_pair_cols(const float2* spectra, size_t spec_stride, const int2* pairs,
                             int npairs, int n, float bfactor, int box, float2* tbuf,
                             float* tmax, int precision, int variant, hipStream_t st);
-// One movie of a batched column pass: its (pair, kx) items are the global
-// indices [item0, item0 + npairs (n/2+1)), kx major; plans are listed in
-// increasing item0.
-struct PairColsPlan {
-  const float2* spectra;  // the movie's slot 0
-  const int2* pairs;      // movie-local slot pairs
-  const float* wxy;       // pair_weights(n, B-factor)
-  const float2* tw;       // twiddles(n)
-  float2* tbuf;           // T columns of the movie's pairs, [pair][kx][box]
-  unsigned long long spec_stride;
-  long long item0;
-  int npairs, box;
-  int body;               // pair_cols_plan_body(n, box, variant)
-};
-// The plan-kernel body launch_pair_cols(n, box, variant) runs at precision 0:
-// the default variant (PAIR_COLS_AUTO) of the M = 128 decimation at n in
-// [512, 3840] and box <= 128; -1 for other variants and sizes, which keep
-// their own kernels (the default at 4096 is the 4-wave M = 128 kernel).
-int pair_cols_plan_body(int n, int box, int variant);
-// Register class of a body: 0 runs at 4 workgroups per CU, 1 at 2.  A plan
-// table holds the movies of one class; each class is its own launch sequence.
-int pair_cols_plan_class(int body);
-const float* pair_weights(int n, float bfactor);
-hipError_t launch_pair_cols_plans(const PairColsPlan* plans, int nplans, long long items, int cls,
-                                  hipStream_t st);
+// The FP32 column pass (mc_cols.hip; wxy: the weight table of mc_pair.hip), and
+// the kx segments of a persistent column-pass launch sequence.
+hipError_t launch_pair_cols_fp32(const float2* spectra, size_t spec_stride, const int2* pairs,
+                                 int npairs, const float* wxy, int n, int box, float2* tbuf,
+                                 hipStream_t st);
+int col_segments(int npairs, int H, int grid);
 size_t pair_rows_part_elems(int npairs, int n, int box);
 hipError_t launch_pair_rows(const float2* tbuf, const float* tmax, int npairs, int n, int box,
                             float* boxmaps, float* part, int precision, int variant,

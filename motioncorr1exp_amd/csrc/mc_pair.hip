@@ -8,12 +8,9 @@
 // read back (FindShift, cufunc.cu:398-407).  Here the product, the weight
 // and the inverse restricted to the box are fused:
 //
-//  k_pair_cols : one (pair, kx) per workgroup.  The product X[ky] is formed
-//    on the fly from the two spectra columns (contiguous in the [kx][ky]
-//    layout), decimated ky = a + A b (A = n/M), transformed by A inverse
-//    M-point FFTs in LDS, and combined as
-//      T[r] = sum_a e^{2 pi i a R_r/n} Y_a[R_r mod M],  R_r = (n-box)/2 + r,
-//    which equals the column inverse at the box rows (M >= box).
+//  column pass : T[r], the column inverse at the box rows R_r = (n-box)/2 + r
+//    of the product formed on the fly from the two spectra columns (mc_cols.hip;
+//    k_pair_cols here at some sizes and boxes).
 //  k_pair_rows : one pair per workgroup: C[r][c] = sum_kx a_kx Re(T[kx][r]
 //    e^{2 pi i kx R_c/n}) with a_0 = a_{n/2} = 1, a_kx = 2 (the C2R row
 //    transform with the DC/Nyquist projection): a real GEMM with K =
@@ -47,10 +44,6 @@ typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 // HBM once into that XCD's L2 and reused by all pairs.  Per-workgroup
 // constants (M-point twiddles in LDS; ky weights, combine twiddles in
 // registers) are loaded once.
-//
-// The per-item arithmetic of each column pass lives in a body struct
-// (ColGen, ColM128) shared by the single-movie kernels and the batched plan
-// kernel, so a pair's T column has the same FP32 operations in both.
 //
 // ColGen: generic decimated pass, A = N/M inverse M-point FFTs in LDS
 // (fft_lds_t; M any Stockham length), combine by lane groups of SP lanes
@@ -210,320 +203,9 @@ __global__ __launch_bounds__(NT) void k_pair_cols(const float2* __restrict__ spe
   }
 }
 
-// Specialised column pass for M = 128 (box <= 128), n >= 512, NT = 256:
-//  stage 0 (radix 16 over b): the 16 inputs X[a + A(j + 8r)] of butterfly
-//    (a, j) are loaded straight from the two spectra (coalesced over a),
-//    multiplied and weighted in registers, transformed and written to LDS;
-//  stage 1 (radix 8, Ns = 16): reads and writes the same 8 LDS slots per
-//    butterfly, so it runs in place without a barrier; its 7 twiddles depend
-//    only on tid % 16 and stay in registers;
-//  combine: SP adjacent lanes share one output row and reduce with xor
-//    shuffles (no LDS round trip).
-// WYG (for the 128-VGPR cap of 4 workgroups per CU): the stage-0 weights are
-// re-read per item (L1-resident, coalesced) instead of held in 16 registers,
-// and the stage-1 twiddles come from a 128-entry LDS table, which frees 16
-// more VGPRs.  The values, and so the results, are the same either way.
-template <int N, int SP, bool WYG>
-struct ColM128 {
-  static constexpr int NN = N;
-  static constexpr int NT = 256;
-  static constexpr int M = 128;
-  static constexpr int A = N / M;
-  static constexpr int H = N / 2 + 1;
-  static constexpr int PB = 4;
-  static constexpr int TS = lds_len<PB>(M) | 1;
-  static constexpr int NB0 = A * 8;  // stage-0 butterflies
-  static constexpr int P0 = (NB0 + NT - 1) / NT;
-  static constexpr int NB1 = A * 16;  // stage-1 butterflies
-  static constexpr int P1 = (NB1 + NT - 1) / NT;
-  static constexpr int AS = A / SP;
-  static constexpr int LDS = A * TS + (WYG ? M : 0);  // float2 elements
-  static_assert(NT % 16 == 0 && A % SP == 0, "shape");
-  float2* buf;
-  float2* tw128;
-  float wy[P0][16];
-  float2 t1[8];
-  float2 ctw[AS];
-  int cr, ch, Rm, tid;
-  bool cact;
-
-  // Loads the workgroup constants (the LDS twiddle table is complete after
-  // the first barrier of the first item).
-  MC_DEV void init(float2* lds, const float* __restrict__ wxy, const float2* __restrict__ tw,
-                   int box, int tid_) {
-    tid = tid_;
-    buf = lds;
-    tw128 = lds + A * TS;
-    // stage-0 element weights (fixed per thread)
-#pragma unroll
-    for (int p = 0; p < P0; p++) {
-      const int q = tid + p * NT;
-      const int a = q % A, j = q / A;
-#pragma unroll
-      for (int r = 0; r < 16; r++) wy[p][r] = (!WYG && q < NB0) ? wxy[H + a + A * (j + 8 * r)] : 0.f;
-    }
-    // stage-1 twiddles W_128^{k r}, k = tid % 16 (inverse sign)
-    if constexpr (WYG) {
-      for (int i = tid; i < M; i += NT) tw128[i] = tw[i * (N / M)];
-    } else {
-#pragma unroll
-      for (int r = 0; r < 8; r++) t1[r] = tw[((tid % 16) * r * (N / M)) % N];
-    }
-    // combine: lane group (SP lanes) per output row
-    const int ori = (N - box) / 2;
-    cr = tid / SP;
-    ch = tid % SP;
-    cact = cr < box;
-    const int R = ori + (cact ? cr : 0);
-    Rm = R & (M - 1);
-#pragma unroll
-    for (int i = 0; i < AS; i++) ctw[i] = tw[((i * SP + ch) * R) % N];
-  }
-  // Raw stage-0 inputs of one item: the two spectrum columns at bin kx.
-  // (As buffer loads, with the column base in scalar registers, the loop
-  // issues 28 fewer VALU instructions per item at the same speed, but the
-  // pass fetched 13% more bytes past L2, so these stay global loads.)
-  MC_DEV void fetch(float2 (&ra)[P0][16], float2 (&rb)[P0][16], const float2* sa,
-                    const float2* sb) const {
-#pragma unroll
-    for (int pp = 0; pp < P0; pp++) {
-      const int q = tid + pp * NT;
-      if (NB0 % NT == 0 || q < NB0) {
-        const int a = q % A, j = q / A;
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int e = a + A * (j + 8 * r);
-          ra[pp][r] = sa[e];
-          rb[pp][r] = sb[e];
-        }
-      }
-    }
-  }
-  // Stage 0 from the fetched registers into LDS (no barrier).  The column
-  // weight is left to finish(): the transform is linear, so scaling its
-  // box outputs by wx replaces 16 products per lane.
-  MC_DEV void stage0(const float2 (&ra)[P0][16], const float2 (&rb)[P0][16],
-                     const float* __restrict__ wxy) {
-#pragma unroll
-    for (int pp = 0; pp < P0; pp++) {
-      const int q = tid + pp * NT;
-      if (NB0 % NT == 0 || q < NB0) {
-        const int a = q % A, j = q / A;
-        float2 v[16];
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const float w = WYG ? wxy[H + a + A * (j + 8 * r)] : wy[pp][r];
-          v[r] = cscale(cmulc(ra[pp][r], rb[pp][r]), w);
-        }
-        dft16<1>(v);
-#pragma unroll
-        for (int r = 0; r < 16; r++) buf[a * TS + lix_at<PB, 1, 16>(lix<PB>(16 * j), 16 * j, r)] = v[r];
-      }
-    }
-  }
-  // Stage 1 and the combine into tout[0, box), scaled by the column weight
-  // wx; ends with a barrier (buf is rewritten by the next item's stage 0).
-  MC_DEV void finish(float2* tout, float wx) {
-    __syncthreads();
-    // ---- stage 1 in place (radix 8, Ns = 16)
-#pragma unroll
-    for (int pp = 0; pp < P1; pp++) {
-      const int q = tid + pp * NT;
-      if (NB1 % NT == 0 || q < NB1) {
-        const int a = q / 16, j = q % 16;
-        float2 v[8];
-#pragma unroll
-        for (int r = 0; r < 8; r++) v[r] = buf[a * TS + lix_at<PB, 16>(lix<PB>(j), j, r)];
-#pragma unroll
-        for (int r = 1; r < 8; r++)
-          v[r] = cmul(v[r], WYG ? tw128[((tid % 16) * r) % M] : t1[r]);
-        dft8<1>(v);
-#pragma unroll
-        for (int r = 0; r < 8; r++) buf[a * TS + lix_at<PB, 16>(lix<PB>(j), j, r)] = v[r];
-      }
-    }
-    __syncthreads();
-    // ---- combine T[R] = sum_a e^{2 pi i a R/N} Y_a[R mod M]
-    float2 acc = make_float2(0.f, 0.f);
-#pragma unroll
-    for (int i = 0; i < AS; i++) acc = cadd(acc, cmul(ctw[i], buf[(i * SP + ch) * TS + lix<PB>(Rm)]));
-#pragma unroll
-    for (int o = 1; o < SP; o <<= 1) {
-      acc.x += __shfl_xor(acc.x, o);
-      acc.y += __shfl_xor(acc.y, o);
-    }
-    if (cact && ch == 0) tout[cr] = cscale(acc, wx);
-    __syncthreads();
-  }
-  // One whole item (no prefetch).
-  MC_DEV void item(const float2* a, const float2* b, const float* __restrict__ wxy, float wx,
-                   float2* tout) {
-    float2 ra[P0][16], rb[P0][16];
-    fetch(ra, rb, a, b);
-    stage0(ra, rb, wxy);
-    finish(tout, wx);
-  }
-};
-
-// A launch covers the bins kx in [kxb, kxb + nkx) of every pair.  With PF
-// (software pipeline) the raw spectrum values of the next item are loaded
-// into registers while the current item goes through stage 1 and the
-// combine, so the global-load latency overlaps LDS work (at the cost of 64
-// more VGPRs, i.e. one workgroup less per CU).
-template <int N, int SP, bool PF, int MINW>
-__global__ __launch_bounds__(256, (N <= 4096 ? MINW : 1)) void k_pair_cols_m128(const float2* __restrict__ spectra,
-                                                        size_t spec_stride,
-                                                        const int2* __restrict__ pairs,
-                                                        int npairs,
-                                                        const float* __restrict__ wxy, int box,
-                                                        float2* __restrict__ tbuf,
-                                                        const float2* __restrict__ tw,
-                                                        int kxb, int nkx) {
-  typedef ColM128<N, SP, (MINW >= 4)> B;
-  __shared__ float2 lds[B::LDS];
-  B b;
-  b.init(lds, wxy, tw, box, threadIdx.x);
-  const int xcd = blockIdx.x % 8, lid = blockIdx.x / 8, nper = gridDim.x / 8;
-  const long long items = (long long)npairs * nkx;
-  const long long i0 = items * xcd / 8, i1 = items * (xcd + 1) / 8;
-  float2 ra[B::P0][16], rb[B::P0][16];
-  auto fetch = [&](long long it) {
-    const int kx = kxb + (int)(it / npairs), p = (int)(it % npairs);
-    const int2 pr = pairs[p];
-    b.fetch(ra, rb, spectra + (size_t)pr.x * spec_stride + (size_t)kx * N,
-            spectra + (size_t)pr.y * spec_stride + (size_t)kx * N);
-  };
-  if (PF && i0 + lid < i1) fetch(i0 + lid);
-  for (long long it = i0 + lid; it < i1; it += nper) {
-    const int kx = kxb + (int)(it / npairs), p = (int)(it % npairs);
-    if (!PF) fetch(it);
-    b.stage0(ra, rb, wxy);
-    if (PF && it + nper < i1) fetch(it + nper);
-    b.finish(tbuf + ((size_t)p * B::H + kx) * box, wxy[kx]);
-  }
-}
-
-// ------------------------------------------- batched (plan) column pass
-// One persistent launch over the column-pass items of one movie or of many
-// movies of different transform sizes (the default column pass of the M = 128
-// decimation).  Movie m's items are the global indices [item0_m, item0_m +
-// npairs_m (n_m/2+1)), kx major, pair minor; a plan table lists the movies in
-// increasing item0 (one movie: the plan is passed by value).  A launch covers
-// the global range [g0, g1), split over the XCDs as in the single-movie
-// kernels; a workgroup runs consecutive items of one movie with that movie's
-// body (ColM128 at its n) and sets the body up again when its next item
-// belongs to the next movie.  Bodies are keyed n | SP << 14.  A movie alone
-// and a movie in a batch run the same machine code for its items, so its T
-// columns are bitwise the same (two builds of one body may contract
-// multiply-adds differently, so this is a property of the code, not of the
-// source).
-// The items [it, stop) (step nper) of one movie.  The movie's pointers are
-// parameters with __restrict__ so that, as in the single-movie kernels, its
-// uniform reads (pair slots, column weight) are scalar loads.
-template <class B>
-MC_DEV long long plan_items(const float2* __restrict__ spectra, size_t spec_stride,
-                            const int2* __restrict__ pairs, int np, const float* __restrict__ wxy,
-                            const float2* __restrict__ tw, float2* __restrict__ tbuf, long long it,
-                            long long li0, long long stop, int nper, int box, float2* lds,
-                            int tid) {
-  constexpr int N = B::NN;
-  constexpr int H = N / 2 + 1;
-  B b;
-  __syncthreads();  // the previous body's LDS reads are done
-  b.init(lds, wxy, tw, box, tid);
-  // a movie has fewer than 2^31 items: kx and pair advance incrementally
-  const int li = (int)li0;
-  int kx = li / np, p = li - kx * np;
-  const int dkx = nper / np, dp = nper - dkx * np;
-  for (; it < stop; it += nper) {
-    const int2 pr = pairs[p];
-    b.item(spectra + (size_t)pr.x * spec_stride + (size_t)kx * N,
-           spectra + (size_t)pr.y * spec_stride + (size_t)kx * N, wxy, wxy[kx],
-           tbuf + ((size_t)p * H + kx) * box);
-    kx += dkx;
-    p += dp;
-    if (p >= np) {
-      p -= np;
-      kx++;
-    }
-  }
-  return it;
-}
-
-constexpr int plan_key(int n, int sp) { return n | (sp << 14); }
-constexpr int kPlanLds = ColM128<3840, 2, true>::LDS;  // the largest body arena (float2)
-// The LDS arena of the plan kernels, shared by all bodies.
-__shared__ float2 plan_lds[kPlanLds];
-
-// Runs the items [it, stop) of plan pl with body B.  The thread index comes
-// in through an opaque move made here, once per plan: the values a body
-// derives from it are then computed per plan rather than hoisted to the
-// kernel entry, where those of every body would be live at once.  The box
-// comes from the plan record for the same reason.
-template <class B>
-MC_DEV long long plan_run(const PairColsPlan& pl, long long it, long long stop, int nper) {
-  int tid = threadIdx.x;
-  asm volatile("v_mov_b32 %0, %1" : "=v"(tid) : "v"(tid));
-  return plan_items<B>(pl.spectra, pl.spec_stride, pl.pairs, pl.npairs, pl.wxy, pl.tw, pl.tbuf, it,
-                       it - pl.item0, stop, nper, pl.box, plan_lds, tid);
-}
-
-// Two register classes: ColM128 at n <= 1536 fits the 128-VGPR cap of 4
-// workgroups per CU and runs in k_pair_cols_plan<4>; at 1920..3840 it needs
-// 150-180 VGPRs and runs in k_pair_cols_plan<2>.  At n = 4096 the body needs
-// 120-125 VGPRs alone and spills inside the plan kernel, so movies of that
-// size take k_pair_cols_m128<4096, SP, false, 4> (single and batched alike).
-constexpr bool plan_wide(int n) { return n >= 1920 && n < 4096; }
-
-template <int MINW>
-__global__ __launch_bounds__(256, MINW) void k_pair_cols_plan(PairColsPlan one,
-                                                              const PairColsPlan* __restrict__ plans,
-                                                              int nplans, long long g0,
-                                                              long long g1) {
-  const int xcd = blockIdx.x % 8, lid = blockIdx.x / 8, nper = gridDim.x / 8;
-  const long long tot = g1 - g0;
-  const long long x1 = g0 + tot * (xcd + 1) / 8;
-  long long it = g0 + tot * xcd / 8 + lid;
-  if (it >= x1) return;
-  if (!plans) nplans = 1;
-  auto plan = [&](int i) -> PairColsPlan { return plans ? plans[i] : one; };
-  // the movie of the first item (binary search), then forward as `it` grows
-  int lo = 0, hi = nplans - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) / 2;
-    if (plan(mid).item0 <= it) lo = mid;
-    else hi = mid - 1;
-  }
-  int pi = lo;
-  while (it < x1) {
-    while (pi + 1 < nplans && plan(pi + 1).item0 <= it) pi++;
-    const PairColsPlan pl = plan(pi);
-    const long long end = pi + 1 < nplans ? plan(pi + 1).item0 : x1;
-    const long long stop = end < x1 ? end : x1;
-    switch (pl.body) {
-// A key of the other class is never in this class's table; it is skipped.
-#define MC_PLAN_M(NN, SPV)                                                                   \
-  case plan_key(NN, SPV):                                                             \
-    if constexpr (plan_wide(NN) == (MINW == 2))                                              \
-      it = plan_run<ColM128<NN, SPV, true>>(pl, it, stop, nper);                            \
-    else                                                                                     \
-      it += (stop - it + nper - 1) / nper * nper;                                            \
-    break;
-      MC_PLAN_M(512, 4) MC_PLAN_M(512, 2) MC_PLAN_M(768, 2) MC_PLAN_M(1024, 4) MC_PLAN_M(1024, 2)
-      MC_PLAN_M(1280, 2) MC_PLAN_M(1536, 4) MC_PLAN_M(1536, 2) MC_PLAN_M(1920, 1)
-      MC_PLAN_M(2048, 4) MC_PLAN_M(2048, 2) MC_PLAN_M(2560, 4) MC_PLAN_M(2560, 2)
-      MC_PLAN_M(3072, 4) MC_PLAN_M(3072, 2) MC_PLAN_M(3840, 2)
-#undef MC_PLAN_M
-      default:  // not reached: the host admits only the keys above
-        it += (stop - it + nper - 1) / nper * nper;
-        break;
-    }
-    // `it` is now the workgroup's first item at or past `stop`
-  }
-}
-
 // ----------------------------------------------- MFMA FP16 hi/lo form
-// Same decimated pruned inverse as k_pair_cols_m128, with its first DFT
+// The pruned inverse of a column (T of mc_cols.hip), decimated ky = a + A b
+// (A = n/128) into 128-point transforms and a combine, with their first DFT
 // stage (16 points, stride 8A in ky) run on the matrix cores.  With
 // ky = c + 8A b1 (c in [0, 8A), b1 in [0, 16)) the stage is the complex
 // product Z[k1][c] = sum_b1 e^{2 pi i b1 k1/16} X[c + 8A b1], i.e. the real
@@ -1259,42 +941,6 @@ static hipError_t pair_cols_t(const float2* spectra, size_t spec_stride, const i
   return hipGetLastError();
 }
 
-// kx segments of a persistent column-pass launch: about 128 items per
-// workgroup each, at most 8.  Within one launch the workgroups of an XCD
-// drift apart as they go, and the frame columns of the kx values in flight
-// outgrow its L2; a new launch lines them up again (3838x3710x40: 3.09 ms in
-// one launch, 2.93 in four).
-static int col_segments(int npairs, int H, int grid) {
-  const long long per_wg = (long long)npairs * H / std::max(1, grid);
-  return (int)std::max(1LL, std::min(8LL, (per_wg + 64) / 128));
-}
-
-template <int N, int SP>
-static hipError_t pair_cols_m128(const float2* spectra, size_t spec_stride, const int2* pairs,
-                                 int npairs, const float* wxy, int box, float2* tbuf, int mode,
-                                 hipStream_t st) {
-  const float2* tw = twiddles(N);
-  if (!tw) return hipErrorOutOfMemory;
-  static const int g1 = persistent_grid(k_pair_cols_m128<N, SP, true, 1>, 256);
-  static const int g0 = persistent_grid(k_pair_cols_m128<N, SP, false, 1>, 256);
-  static const int g4 = persistent_grid(k_pair_cols_m128<N, SP, false, 4>, 256);
-  const int H = N / 2 + 1;
-  const int S = col_segments(npairs, H, mode == 1 ? g1 : (mode == 2 ? g4 : g0));
-  for (int sgi = 0; sgi < S; sgi++) {
-    const int kxb = H * sgi / S, nkx = H * (sgi + 1) / S - kxb;
-    if (mode == 1)
-      hipLaunchKernelGGL((k_pair_cols_m128<N, SP, true, 1>), dim3(g1), dim3(256), 0, st, spectra,
-                         spec_stride, pairs, npairs, wxy, box, tbuf, tw, kxb, nkx);
-    else if (mode == 2)
-      hipLaunchKernelGGL((k_pair_cols_m128<N, SP, false, 4>), dim3(g4), dim3(256), 0, st,
-                         spectra, spec_stride, pairs, npairs, wxy, box, tbuf, tw, kxb, nkx);
-    else
-      hipLaunchKernelGGL((k_pair_cols_m128<N, SP, false, 1>), dim3(g0), dim3(256), 0, st,
-                         spectra, spec_stride, pairs, npairs, wxy, box, tbuf, tw, kxb, nkx);
-  }
-  return hipGetLastError();
-}
-
 template <int N, int SP>
 static hipError_t pair_cols_mfma(const float2* spectra, size_t spec_stride, const int2* pairs,
                                  int npairs, const float* wxy, int box, float2* tbuf,
@@ -1312,75 +958,12 @@ static hipError_t pair_cols_mfma(const float2* spectra, size_t spec_stride, cons
   return hipGetLastError();
 }
 
-template <int N>
-static hipError_t pair_cols_n(const float2* spectra, size_t spec_stride, const int2* pairs,
-                              int npairs, const float* wxy, int box, float2* tbuf, int variant,
-                              hipStream_t st) {
-  if constexpr (N >= 512) {
-    if (variant != PAIR_COLS_GENERIC) {
-      // the default at 4096 (no plan body there) is the 4-workgroup kernel
-      const bool w4 = variant == PAIR_COLS_M128_W4 || (variant == PAIR_COLS_AUTO && N == 4096);
-      const int mode = variant == PAIR_COLS_M128_PF ? 1 : (w4 ? 2 : 0);
-      if constexpr ((N / 128) % 4 == 0) {
-        if (box <= 64)
-          return pair_cols_m128<N, 4>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, mode, st);
-      }
-      if constexpr ((N / 128) % 2 == 0) {
-        if (box <= 128)
-          return pair_cols_m128<N, 2>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, mode, st);
-      } else {
-        if (box <= 128)
-          return pair_cols_m128<N, 1>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, mode, st);
-      }
-    }
-  }
-  // the generic pass at M = 128: first stage (radix 8 of plan 1, 8 x 16) in
-  // registers on the loaded products
-  if constexpr (N % 512 == 0) {
-    if (box <= 64)
-      return pair_cols_t<N, 128, 4, true, 1>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st);
-  }
-  if constexpr (N % 256 == 0) {
-    if (box <= 128)
-      return pair_cols_t<N, 128, 2, true, 1>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st);
-  }
-  if constexpr (N % 128 == 0) {
-    if (box <= 128)
-      return pair_cols_t<N, 128, 1, true, 1>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st);
-  }
-  if constexpr (N % 256 == 0) {
-    if (box <= 256)
-      return pair_cols_t<N, 256, 1>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st);
-  }
-  if constexpr (N == 64) {
-    if (box <= 64)
-      return pair_cols_t<64, 64, 1>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st);
-  }
-  return hipErrorInvalidValue;
-}
-
-// Sizes of the decimated column pass (n = 128 A, and 64); other even sizes
-// take the chirp-z column pass (mc_czt.hip).
-static bool pair_cols_decimated(int n) {
-  switch (n) {
-    case 64: case 128: case 256: case 512: case 1024: case 2048: case 4096: case 8192:
-    case 768: case 1536: case 3072: case 6144: case 1280: case 2560: case 5120: case 1920:
-    case 3840:
-      return true;
-    default:
-      return false;
-  }
-}
-
 bool pair_form_supported(int precision, int n, int box) {
   if (precision == 0) return box >= 1 && box <= n && box <= 256 && n >= 64 && n <= 8192 && n % 2 == 0;
   // the hi/lo column kernel needs 32-column blocks of 8 n/128 columns
   if (precision == 1) return n >= 512 && n <= 8192 && n % 512 == 0 && box >= 1 && box <= 96;
   return false;
 }
-
-static hipError_t plan_launches(const PairColsPlan& one, const PairColsPlan* plans, int nplans,
-                                long long items, int cls, hipStream_t st);
 
 hipError_t launch_pair_cols(const float2* spectra, size_t spec_stride, const int2* pairs,
                             int npairs, int n, float bfactor, int box, float2* tbuf,
@@ -1411,84 +994,21 @@ hipError_t launch_pair_cols(const float2* spectra, size_t spec_stride, const int
     // the default square crop of a 5760 x 4092 K3 frame: n = 132 * 31,
     // decimated into 31 inverse 132-point FFTs (radix 4, 3, 11)
     return pair_cols_t<4092, 132, 2, true>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st);
-  if (!pair_cols_decimated(n))
-    return launch_pair_cols_czt(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, st);
-  const int body = pair_cols_plan_body(n, box, variant);
-  if (body >= 0) {  // the default: the plan kernel with this one movie
-    PairColsPlan one{};
-    one.spectra = spectra;
-    one.pairs = pairs;
-    one.wxy = wxy;
-    one.tw = twiddles(n);
-    if (!one.tw) return hipErrorOutOfMemory;
-    one.tbuf = tbuf;
-    one.spec_stride = spec_stride;
-    one.item0 = 0;
-    one.npairs = npairs;
-    one.box = box;
-    one.body = body;
-    return plan_launches(one, nullptr, 1, (long long)npairs * (n / 2 + 1),
-                         pair_cols_plan_class(body), st);
+  if (box > 128) {
+    switch (n) {
+#define MC_COLS_256(NN) \
+  case NN: return pair_cols_t<NN, 256, 1>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st);
+      MC_COLS_256(256) MC_COLS_256(512) MC_COLS_256(768) MC_COLS_256(1024) MC_COLS_256(1280)
+      MC_COLS_256(1536) MC_COLS_256(2048) MC_COLS_256(2560) MC_COLS_256(3072) MC_COLS_256(3840)
+      MC_COLS_256(4096) MC_COLS_256(5120) MC_COLS_256(6144) MC_COLS_256(8192)
+#undef MC_COLS_256
+      default: break;
+    }
+    if (n % 128 == 0) return hipErrorInvalidValue;  // multiples of 128 take such boxes at 256 only
   }
-  switch (n) {
-    case 64: return pair_cols_n<64>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 128: return pair_cols_n<128>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 256: return pair_cols_n<256>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 512: return pair_cols_n<512>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 1024: return pair_cols_n<1024>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 2048: return pair_cols_n<2048>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 4096: return pair_cols_n<4096>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 8192: return pair_cols_n<8192>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 768: return pair_cols_n<768>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 1536: return pair_cols_n<1536>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 3072: return pair_cols_n<3072>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 6144: return pair_cols_n<6144>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 1280: return pair_cols_n<1280>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 2560: return pair_cols_n<2560>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 5120: return pair_cols_n<5120>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 1920: return pair_cols_n<1920>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    case 3840: return pair_cols_n<3840>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, variant, st);
-    default: return hipErrorInvalidValue;
-  }
-}
-
-int pair_cols_plan_body(int n, int box, int variant) {
-  if (variant != PAIR_COLS_AUTO) return -1;
-  if (box < 1 || box > 128 || n < 512 || n >= 4096 || n % 128 != 0 || !pair_cols_decimated(n))
-    return -1;
-  const int A = n / 128;
-  return plan_key(n, (A % 4 == 0 && box <= 64) ? 4 : (A % 2 == 0 ? 2 : 1));
-}
-
-int pair_cols_plan_class(int body) { return plan_wide(body & 0x3fff) ? 1 : 0; }
-
-const float* pair_weights(int n, float bfactor) { return weights(n, bfactor); }
-
-// Launches of about 128 items per workgroup (see col_segments) over a plan
-// table (plans != nullptr) or the one plan `one`.
-static hipError_t plan_launches(const PairColsPlan& one, const PairColsPlan* plans, int nplans,
-                                long long items, int cls, hipStream_t st) {
-  if (items <= 0) return hipSuccess;
-  static const int g4 = persistent_grid(k_pair_cols_plan<4>, 256);
-  static const int g2 = persistent_grid(k_pair_cols_plan<2>, 256);
-  const int grid = cls ? g2 : g4;
-  const long long per_wg = items / grid;
-  const long long S = std::max(1LL, (per_wg + 64) / 128);
-  for (long long s = 0; s < S; s++) {
-    const long long a = items * s / S, b = items * (s + 1) / S;
-    if (cls)
-      hipLaunchKernelGGL(k_pair_cols_plan<2>, dim3(grid), dim3(256), 0, st, one, plans, nplans, a, b);
-    else
-      hipLaunchKernelGGL(k_pair_cols_plan<4>, dim3(grid), dim3(256), 0, st, one, plans, nplans, a, b);
-  }
-  return hipGetLastError();
-}
-
-hipError_t launch_pair_cols_plans(const PairColsPlan* plans, int nplans, long long items, int cls,
-                                  hipStream_t st) {
-  if (nplans <= 0) return hipSuccess;
-  PairColsPlan none{};
-  return plan_launches(none, plans, nplans, items, cls, st);
+  if (n == 64)
+    return pair_cols_t<64, 64, 1>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st);
+  return launch_pair_cols_fp32(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, st);
 }
 
 hipError_t launch_pair_rows(const float2* tbuf, const float* tmax, int npairs, int n, int box,

@@ -1,0 +1,60 @@
+"""The pair stage's column pass (mc_cols.hip) at the sizes where it can go
+wrong: transform sizes whose share per wave is full, ragged or a fraction of
+a wave, one to eight waves per item, boxes from 16 to the largest, odd ones
+and both sides of 96 among them.  Box maps of random spectra set directly,
+against the FP64 cross power and inverse of the same spectra by numpy
+(cufunc.cu:343-370, DFAlign.cu:897, cufunc.cu:398-407).
+
+Bound: the map is a sum of n^2/2 products by FP32 transforms of length n and
+a sum over n/2 bins, whose rounding errors add as random terms: about
+2^-24 sqrt(2 log2 n + 2) of the map's root mean square per point for the
+transforms and as much again for the sum, 7e-7 at n = 8192 with peaks of five
+standard deviations; 2e-6 of the map's maximum holds all of it."""
+import numpy as np
+import pytest
+
+import motioncorr1exp_amd as mc
+
+pytestmark = pytest.mark.gpu
+
+
+def reference_box(a, b, n, bfactor, box):
+    """Central box of irfft2(a conj(b) z) / normalisation in FP64 (rows by FFT,
+    box columns by direct sums)."""
+    kx = np.arange(n // 2 + 1)
+    y = np.where(np.arange(n) < n // 2, np.arange(n), np.arange(n) - n)
+    m = -0.5 * bfactor / n / n
+    z = np.exp(m * (kx[None, :] ** 2 + y[:, None] ** 2)) * (1 - 2 * ((kx[None, :] + y[:, None]) % 2))
+    o = (n - box) // 2
+    t = np.fft.ifft(a * np.conj(b) * z / (n * (n // 2 + 1)), axis=0, norm="forward")[o:o + box]
+    w = np.full(n // 2 + 1, 2.0)
+    w[0] = w[-1] = 1.0
+    e = np.exp(2j * np.pi * ((kx[:, None] * (o + np.arange(box))[None, :]) % n) / n)
+    return ((t * w) @ e).real
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = mc.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("n,box", [
+    (128, 16), (128, 128), (256, 96), (256, 127), (512, 33), (512, 96), (512, 128), (768, 95),
+    (1024, 64), (1024, 97), (1280, 96), (1280, 126), (1536, 17), (1920, 96), (2048, 96),
+    (2560, 128), (3072, 70), (3840, 96), (3840, 128), (4096, 96), (5120, 96), (6144, 111),
+    (8192, 96), (8192, 128)])
+def test_box_maps_match_fp64(ctx, n, box):
+    F = 3
+    rng = np.random.default_rng(n + box)
+    spec = np.fft.rfft2(rng.standard_normal((F, n, n))).astype(np.complex64)
+    ctx.set_spectra(spec.view(np.float32))
+    pairs = np.array([(0, 1), (0, 2), (2, 1), (1, 1)], np.int32)
+    _, _, maps = ctx.pair_shifts(pairs, 150.0, box, want_boxes=True)
+    worst = 0.0
+    for q, (a, b) in enumerate(pairs):
+        ref = reference_box(spec[a].astype(np.complex128), spec[b].astype(np.complex128), n, 150.0, box)
+        worst = max(worst, float(np.abs(maps[q] - ref).max() / np.abs(ref).max()))
+    print("n %d box %d: max error / max %.3g" % (n, box, worst), flush=True)
+    assert worst < 2e-6
