@@ -204,6 +204,188 @@ __global__ __launch_bounds__(512, 4) void k_pair_cols64(
   }
 }
 
+// Any other even n = R0 A, R0 a divisor of n out of 16, 14, 12, 10, 8 and 6.
+// ky = xi + A r, r < R0: per xi an R0-point DFT over r in registers, times
+// e^{2 pi i xi kappa/n}, giving z_xi[kappa]; then with the rows
+// ori + r' = base + R0 g + kappa (base: the multiple of R0 at or below ori; the
+// columns kappa < c = ori - base take the next group, by a factor
+// e^{2 pi i xi R0/n} folded into their twiddle)
+//   T = sum_xi f_g(xi) z_xi[kappa],  f_g(xi) = e^{2 pi i xi (base + R0 g)/n},
+// on v_mfma_f32_16x16x4: rows (g, re | im), eight groups per tile, columns
+// kappa, four xi per instruction.  The real and imaginary parts of z are
+// multiplied by the same rows and combined at the end.  R0 <= 8 fills the 16
+// columns with two sets of xi (lanes l and l + 32, xi and xi + 1), whose sums
+// differ by one factor per group.
+// The contraction costs 8 n box/R0 multiply-adds per item on units twice as
+// fast as the vector ALU; the chirp-z pass it replaces takes two transforms of
+// the next power of two above n + box: 1854, box 96, 78 pairs: 0.36 ms against
+// 0.83; 3710, 253 pairs: 3.9 against 5.0 for its decimated pass (53 FFTs of 70
+// points with five barriers per item); 4092, 55 pairs: 0.99 against 1.20.
+// Columns that do not start on 64 bytes cost: each four lanes' 64 bytes then
+// span two lines (3696, 105 pairs: 1.17 ms; 3710: 1.63).
+template <int R0, int TILES>
+__global__ __launch_bounds__(TILES == 1 || R0 <= 8 ? 1024 : 512, TILES == 1 || R0 <= 8 ? 4 : 3) void k_pair_cols_r(
+    const float2* __restrict__ spectra, size_t spec_stride, const int2* __restrict__ pairs,
+    int npairs, const float* __restrict__ wxy, int n, int box, float2* __restrict__ tbuf,
+    const float2* __restrict__ tw, int kxb, int nkx) {
+  extern __shared__ float4 cols_lds[];
+  constexpr int KP = R0 > 8 ? 16 : 8;   // columns of the exchange rows
+  constexpr int NH = 16 / KP;           // xi sets side by side
+  constexpr int NR = 16 / NH;           // rounds of 4 NH xi
+  constexpr int ZB = KP == 16 ? 8192 : 66 * 64;  // exchange bytes per wave
+  constexpr int S = R0 / 2;
+  const int A = n / R0, nw = (A + 63) / 64, H = n / 2 + 1, nt = nw * 64;
+  const int LC = ((A + nw - 1) / nw + 1) / 2 * 2;  // xi per wave, even, <= 64
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
+  // loads: lane (h, i) takes xi = x0, x0 + 1 in the rows r = s + S h; after the
+  // swap it holds xi = x0 + h in all rows.  An odd A's last pair starts one
+  // element early: its first element belongs to the pair before and gets
+  // weight zero.
+  const int h = l >> 5, i = l & 31;
+  auto pair_start = [&](int ii) {
+    const int x = w * LC + 2 * ii;
+    return 2 * ii >= LC || x >= A ? -1 : (x == A - 1 ? x - 1 : x);
+  };
+  const int x0 = pair_start(i);
+  const bool own = x0 >= 0, twice = own && x0 != w * LC + 2 * i;
+  const int voff = own ? 8 * (x0 + S * A * h) : n * 8;  // past the end: reads zero
+  const int xi = own ? x0 + h : 0;
+  const int ori = (n - box) / 2, c = ori % R0, base = ori - c, G = (box + R0 - 1) / R0;
+  float wy[R0];
+#pragma unroll
+  for (int s = 0; s < S; s++)
+#pragma unroll
+    for (int e = 0; e < 2; e++)
+      wy[s + S * e] = own && !(twice && e == 0) ? wxy[H + x0 + e + A * (s + S * h)] : 0.f;
+  float2 tk[R0];
+#pragma unroll
+  for (int k = 0; k < R0; k++) tk[k] = tw[(long long)xi * (k + (k < c ? R0 : 0)) % n];
+  // matrix rows m = l % 16: (re, im) of group 8 tile + m / 2 at the xi of
+  // exchange row 4 q + l / 16
+  float P[NR][TILES];
+#pragma unroll
+  for (int q = 0; q < NR; q++) {
+    const int row = 4 * q + (l >> 4), xs = pair_start(row & 31);
+    const int x = xs < 0 ? 0 : xs + (row >> 5);
+#pragma unroll
+    for (int t = 0; t < TILES; t++) {
+      const int g = 8 * t + ((l & 15) >> 1);
+      const float2 f = g < G ? tw[(long long)x * (base + R0 * g) % n] : make_float2(0.f, 0.f);
+      P[q][t] = (l & 1) ? f.y : f.x;
+    }
+  }
+  const int kl = l & (KP - 1), hf = (l >> 3) & (NH - 1), al = l >> 4;
+  // the second set's factor e^{2 pi i (base + R0 g)/n} for this lane's groups
+  float2 cf[TILES][2];
+#pragma unroll
+  for (int t = 0; t < TILES; t++)
+#pragma unroll
+    for (int e = 0; e < 2; e++)
+      cf[t][e] = hf ? tw[(base + R0 * (8 * t + 2 * al + e)) % n] : make_float2(1.f, 0.f);
+  // exchange row l (lane order), 16-byte slots permuted: by l mod 8 (KP = 16),
+  // by (l / 4) mod 4 with the second 32 rows two rows further (KP = 8)
+  const int zb = w * ZB + (KP == 16 ? l * 128 + (l & 7) * 16 : (l + 2 * h) * 64 + ((l >> 2) & 3) * 16);
+  const int rd = KP == 16 ? w * ZB + al * 128 + (((kl >> 1) ^ al) << 4) + (kl & 1) * 8
+                          : w * ZB + (al + 34 * hf) * 64 + ((kl >> 1) << 4) + (kl & 1) * 8;
+  float4* red = reinterpret_cast<float4*>(reinterpret_cast<char*>(cols_lds) + nw * ZB);
+  const int xcd = blockIdx.x % 8, lid = blockIdx.x / 8, nper = gridDim.x / 8;
+  const long long items = (long long)npairs * nkx;
+  const int i1 = (int)(items * (xcd + 1) / 8);
+  int it = (int)(items * xcd / 8) + lid;
+  if (it >= i1) return;
+  int kx = it / npairs, p = it - kx * npairs;
+  const int dkx = nper / npairs, dp = nper - dkx * npairs;
+  for (int par = 0;; par ^= nw * TILES * 64) {
+    const int2 pr = pairs[p];
+    const auto qa = buf_rsrc(spectra + (size_t)pr.x * spec_stride + (size_t)(kxb + kx) * n, n * 8);
+    const auto qb = buf_rsrc(spectra + (size_t)pr.y * spec_stride + (size_t)(kxb + kx) * n, n * 8);
+    float4 ra[S], rb[S];
+    float2 v[R0];
+    auto load = [&](int s) {
+      ra[s] = buf_ld4(qa, voff, 8 * A * s);
+      rb[s] = buf_ld4(qb, voff, 8 * A * s);
+    };
+    constexpr int D = S < 7 ? S : 7;  // as in k_pair_cols64
+#pragma unroll
+    for (int s = 0; s < D; s++) {
+      load(s);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+      v[s] = cscale(cmulc(make_float2(ra[s].x, ra[s].y), make_float2(rb[s].x, rb[s].y)), wy[s]);
+      v[s + S] = cscale(cmulc(make_float2(ra[s].z, ra[s].w), make_float2(rb[s].z, rb[s].w)), wy[s + S]);
+      swap32(v[s].x, v[s + S].x);
+      swap32(v[s].y, v[s + S].y);
+      if (s + D < S) load(s + D);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    dft<R0, 1>(v);
+#pragma unroll
+    for (int k = 0; k < R0; k++) v[k] = cmul(v[k], tk[k]);
+    int za = zb;
+    asm volatile("" : "+v"(za));
+#pragma unroll
+    for (int e = 0; e < R0 / 2; e++)
+      *reinterpret_cast<float4*>(reinterpret_cast<char*>(cols_lds) + (za ^ (16 * e))) =
+          make_float4(v[2 * e].x, v[2 * e].y, v[2 * e + 1].x, v[2 * e + 1].y);
+    wave_fence();
+    v4f D1[TILES], D2[TILES];
+#pragma unroll
+    for (int t = 0; t < TILES; t++) D1[t] = D2[t] = v4f{0.f, 0.f, 0.f, 0.f};
+    int ra0 = rd;
+    asm volatile("" : "+v"(ra0));
+#pragma unroll
+    for (int q = 0; q < NR; q++) {
+      // rounds whose rows hold no xi of any wave are skipped
+      if (2 * ((4 * q) & 31) >= LC) continue;
+      const int ad = KP == 16 ? (ra0 ^ ((q & 1) << 6)) + 512 * q : (ra0 ^ ((q & 3) << 4)) + 256 * q;
+      const float2 u = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(cols_lds) + ad);
+#pragma unroll
+      for (int t = 0; t < TILES; t++) {
+        D1[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(P[q][t], u.x, D1[t], 0, 0, 0);
+        D2[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(P[q][t], u.y, D2[t], 0, 0, 0);
+      }
+    }
+    wave_fence();
+    int lt;  // the lane, made again per item: one register less in the loop
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(lt));
+#pragma unroll
+    for (int t = 0; t < TILES; t++) {
+      float2 a = make_float2(D1[t][0] - D2[t][1], D1[t][1] + D2[t][0]);
+      float2 b = make_float2(D1[t][2] - D2[t][3], D1[t][3] + D2[t][2]);
+      if constexpr (NH == 2) {
+        a = cmul(a, cf[t][0]);
+        b = cmul(b, cf[t][1]);
+      }
+      red[par + (w * TILES + t) * 64 + lt] = make_float4(a.x, a.y, b.x, b.y);
+    }
+    if (nw > 1) lds_barrier();
+    else wave_fence();
+    const float wx = wxy[kxb + kx];
+    const float2* rp = reinterpret_cast<const float2*>(red + par);
+    const auto qt = buf_rsrc(tbuf + ((size_t)p * H + kxb + kx) * box, box * 8);
+    for (int r = w * 64 + lt; r < box; r += nt) {
+      const int g = r / R0, kk = r - g * R0 + c, k = kk < R0 ? kk : kk - R0;
+      const int o = ((g >> 3) * 64 + ((g & 7) >> 1) * 16 + k) * 2 + (g & 1);
+      float2 s = make_float2(0.f, 0.f);
+      for (int x = 0; x < nw; x++)
+#pragma unroll
+        for (int e = 0; e < NH; e++) s = cadd(s, rp[x * (TILES * 128) + o + 16 * e]);
+      buf_st2(qt, 8 * r, cscale(s, wx));
+    }
+    it += nper;
+    if (it >= i1) break;
+    kx += dkx;
+    p += dp;
+    if (p >= npairs) {
+      p -= npairs;
+      kx++;
+    }
+  }
+}
+
 // Resident workgroups of a persistent launch of nt threads with dynamic LDS,
 // asked once per kernel, device and workgroup size.
 template <class K> static int cols_grid(K kernel, int nw, size_t lds, std::atomic<int> (&cache)[16][17]) {
@@ -259,6 +441,34 @@ static hipError_t cols64(const float2* spectra, size_t spec_stride, const int2* 
                        });
 }
 
+template <int R0, int TILES>
+static hipError_t cols_r(const float2* spectra, size_t spec_stride, const int2* pairs, int npairs,
+                         const float* wxy, int n, int box, float2* tbuf, const float2* tw,
+                         hipStream_t st) {
+  static std::atomic<int> cache[16][17];
+  const int nw = (n / R0 + 63) / 64;
+  const size_t lds = (size_t)nw * ((R0 > 8 ? 8192 : 66 * 64) + TILES * 2048);
+  return cols_launches(k_pair_cols_r<R0, TILES>, nw, lds, cache, npairs, n / 2 + 1,
+                       [&](int grid, int kxb, int nkx) {
+                         hipLaunchKernelGGL((k_pair_cols_r<R0, TILES>), dim3(grid), dim3(nw * 64), lds,
+                                            st, spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf,
+                                            tw, kxb, nkx);
+                       });
+}
+
+// The radix of k_pair_cols_r at size n and the tiles of eight groups that the
+// box needs: the largest divisor whose tiles and waves the kernel holds (its
+// work per element falls with R0); 0: none, the chirp-z pass.
+static int cols_radix(int n, int box, int* tiles) {
+  for (int R0 : {16, 14, 12, 10, 8, 6}) {
+    const int t = (box + 8 * R0 - 1) / (8 * R0), waves = (n / R0 + 63) / 64;
+    if (n % R0 || t > (R0 > 8 ? 2 : 3) || waves > (t == 1 || R0 <= 8 ? 16 : 8)) continue;
+    *tiles = t;
+    return R0;
+  }
+  return 0;
+}
+
 hipError_t launch_pair_cols_fp32(const float2* spectra, size_t spec_stride, const int2* pairs,
                                  int npairs, const float* wxy, int n, int box, float2* tbuf,
                                  hipStream_t st) {
@@ -267,6 +477,16 @@ hipError_t launch_pair_cols_fp32(const float2* spectra, size_t spec_stride, cons
   if (n % 128 == 0 && box <= 128) {
     if (box <= 96) return cols64<6>(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, tw, st);
     return cols64<8>(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, tw, st);
+  }
+  int tiles = 0;
+  switch (cols_radix(n, box, &tiles) * 4 + tiles) {
+#define MC_COLS_R(R, T) \
+  case R * 4 + T: return cols_r<R, T>(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, tw, st);
+    MC_COLS_R(16, 1) MC_COLS_R(16, 2) MC_COLS_R(14, 1) MC_COLS_R(14, 2) MC_COLS_R(12, 1)
+    MC_COLS_R(12, 2) MC_COLS_R(10, 1) MC_COLS_R(10, 2) MC_COLS_R(8, 1) MC_COLS_R(8, 2)
+    MC_COLS_R(8, 3) MC_COLS_R(6, 1) MC_COLS_R(6, 2) MC_COLS_R(6, 3)
+#undef MC_COLS_R
+    default: break;
   }
   return launch_pair_cols_czt(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, st);
 }

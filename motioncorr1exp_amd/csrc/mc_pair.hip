@@ -9,8 +9,7 @@
 // and the inverse restricted to the box are fused:
 //
 //  column pass : T[r], the column inverse at the box rows R_r = (n-box)/2 + r
-//    of the product formed on the fly from the two spectra columns (mc_cols.hip;
-//    k_pair_cols here at some sizes and boxes).
+//    of the product formed on the fly from the two spectra columns (mc_cols.hip).
 //  k_pair_rows : one pair per workgroup: C[r][c] = sum_kx a_kx Re(T[kx][r]
 //    e^{2 pi i kx R_c/n}) with a_0 = a_{n/2} = 1, a_kx = 2 (the C2R row
 //    transform with the DC/Nyquist projection): a real GEMM with K =
@@ -37,171 +36,6 @@ namespace mc {
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-
-// Persistent: the grid is a multiple of 8 workgroups; workgroup b runs on
-// XCD b % 8 and walks a contiguous range of work items (kx major, pair
-// minor) owned by that XCD, so the frame columns of one kx are fetched from
-// HBM once into that XCD's L2 and reused by all pairs.  Per-workgroup
-// constants (M-point twiddles in LDS; ky weights, combine twiddles in
-// registers) are loaded once.
-//
-// ColGen: generic decimated pass, A = N/M inverse M-point FFTs in LDS
-// (fft_lds_t; M any Stockham length), combine by lane groups of SP lanes
-// whose lane h takes the terms a = h, h + SP, ... < A, summed through LDS.
-// F0 (for a small first radix R0, such as M = 70 = 2 5 7, or M = 128 under
-// stage plan PL = 1, 8 16): the first Stockham stage runs in registers on
-// the loaded products.  Its butterfly (a, j) takes the elements e + r N/R0
-// (e = a + A j < N/R0, r < R0), and writes row a at j R0 + r, so the
-// products skip one LDS round trip and two barriers.
-template <int N, int M, int NT, int SP, bool F0 = false, int PL = 0>
-struct ColGen {
-  static constexpr int NN = N;
-  static constexpr int A = N / M;
-  static constexpr int H = N / 2 + 1;
-  static constexpr int PB = 4;
-  static constexpr int TS = lds_len<PB>(M) | 1;
-  static constexpr int R0 = stage_radix(M, 0, PL);
-  static constexpr int E0 = N / R0;              // first-stage butterflies (all rows)
-  static constexpr int EP0 = (E0 + NT - 1) / NT;  // ... per thread
-  static constexpr int EPT = F0 ? EP0 * R0 : (N + NT - 1) / NT;  // elements per thread
-  static constexpr int AS = (A + SP - 1) / SP;   // combine terms per thread (at most)
-  static constexpr int LDS = A * TS + M + SP * 256;  // float2 elements
-  static_assert(A * M == N, "decimation");
-  static_assert(!F0 || (M % R0 == 0 && stage_count(M, PL) >= 2), "first stage");
-  static_assert(F0 || PL == 0, "plan");
-  float2* buf;
-  float2* twm;
-  float2* part;  // [SP][256]
-  float wy[EPT];
-  float2 ctw[AS];
-  int cr, ch, Rm, box, tid;
-  bool cact;
-
-  // Loads the workgroup constants; ends with a barrier.
-  MC_DEV void init(float2* lds, const float* __restrict__ wxy, const float2* __restrict__ tw,
-                   int box_, int tid_) {
-    tid = tid_;
-    box = box_;
-    buf = lds;
-    twm = lds + A * TS;
-    part = twm + M;
-    for (int i = tid; i < M; i += NT) twm[i] = tw[i * (N / M)];
-    // ky weights (-1)^{y'} exp(m y'^2) / sizec for this thread's elements
-#pragma unroll
-    for (int i = 0; i < EPT; i++) {
-      const int e = F0 ? tid + (i / R0) * NT + (i % R0) * E0 : tid + i * NT;
-      wy[i] = (F0 ? tid + (i / R0) * NT < E0 : e < N) ? wxy[H + e] : 0.f;
-    }
-    // combine: thread -> (output r, term block h)
-    const int ori = (N - box) / 2;
-    cr = tid % box;
-    ch = tid / box;
-    cact = tid < box * SP;
-    const int R = ori + cr;
-#pragma unroll
-    for (int i = 0; i < AS; i++) {
-      const int a = i * SP + ch;
-      ctw[i] = cact && a < A ? tw[(a * R) % N] : make_float2(0.f, 0.f);
-    }
-    Rm = R % M;
-    __syncthreads();
-  }
-  // Item (pair columns a, b at bin kx with column weight wx) -> tout[0, box).
-  // buf and part are rewritten only after the next item's first barrier.
-  MC_DEV void item(const float2* a, const float2* b, const float* __restrict__, float wx,
-                   float2* tout) {
-    const auto qa = buf_rsrc(a, N * 8), qb = buf_rsrc(b, N * 8);
-    float2 va[EPT], vb[EPT];
-    if constexpr (F0) {
-#pragma unroll
-      for (int p = 0; p < EP0; p++) {
-        if (E0 % NT == 0 || tid + p * NT < E0) {
-#pragma unroll
-          for (int r = 0; r < R0; r++) {
-            va[p * R0 + r] = buf_ld2(qa, 8 * tid, 8 * (p * NT + r * E0));
-            vb[p * R0 + r] = buf_ld2(qb, 8 * tid, 8 * (p * NT + r * E0));
-          }
-        }
-      }
-      // products (column weight wx applied to the combined outputs), then
-      // the first radix-R0 stage (Ns = 1: no twiddles) into the LDS rows
-#pragma unroll
-      for (int p = 0; p < EP0; p++) {
-        const int e = tid + p * NT;
-        if (E0 % NT == 0 || e < E0) {
-          float2 v[R0];
-#pragma unroll
-          for (int r = 0; r < R0; r++) v[r] = cscale(cmulc(va[p * R0 + r], vb[p * R0 + r]), wy[p * R0 + r]);
-          dft<R0, 1>(v);
-          float2* row = buf + (e % A) * TS;
-          const int j = e / A;
-#pragma unroll
-          for (int r = 0; r < R0; r++) row[lix<PB>(j * R0 + r)] = v[r];
-        }
-      }
-      __syncthreads();
-      const TwTable twt{twm, M};
-      fft_lds_stage<M, NT, 1, A, 1, TS, TwTable, PB, PL>(buf, twt, M);
-      if constexpr (stage_count(M, PL) > 2) fft_lds_stage<M, NT, 1, A, 2, TS, TwTable, PB, PL>(buf, twt, M);
-      if constexpr (stage_count(M, PL) > 3) fft_lds_stage<M, NT, 1, A, 3, TS, TwTable, PB, PL>(buf, twt, M);
-    } else {
-#pragma unroll
-      for (int i = 0; i < EPT; i++) {
-        const int e = tid + i * NT;
-        if (e < N) {
-          va[i] = buf_ld2(qa, 8 * tid, 8 * NT * i);
-          vb[i] = buf_ld2(qb, 8 * tid, 8 * NT * i);
-        }
-      }
-      // the column weight wx is applied to the combined outputs
-#pragma unroll
-      for (int i = 0; i < EPT; i++) {
-        const int e = tid + i * NT;
-        if (e < N) buf[(e % A) * TS + lix<PB>(e / A)] = cscale(cmulc(va[i], vb[i]), wy[i]);
-      }
-      __syncthreads();
-      fft_lds_t<M, NT, 1, A, TS, TwTable, PB>(buf, TwTable{twm, M}, M);
-    }
-    if (cact) {
-      float2 acc = make_float2(0.f, 0.f);
-#pragma unroll
-      for (int i = 0; i < AS; i++)
-        if (A % SP == 0 || i * SP + ch < A)
-          acc = cadd(acc, cmul(ctw[i], buf[(i * SP + ch) * TS + lix<PB>(Rm)]));
-      part[ch * 256 + cr] = acc;
-    }
-    __syncthreads();
-    if (tid < box) {
-      float2 acc = part[tid];
-#pragma unroll
-      for (int h = 1; h < SP; h++) acc = cadd(acc, part[h * 256 + tid]);
-      tout[tid] = cscale(acc, wx);
-    }
-  }
-};
-
-template <int N, int M, int NT, int SP, bool F0 = false, int PL = 0>
-__global__ __launch_bounds__(NT) void k_pair_cols(const float2* __restrict__ spectra,
-                                                  size_t spec_stride,
-                                                  const int2* __restrict__ pairs, int npairs,
-                                                  const float* __restrict__ wxy, int box,
-                                                  float2* __restrict__ tbuf,
-                                                  const float2* __restrict__ tw) {
-  typedef ColGen<N, M, NT, SP, F0, PL> B;
-  __shared__ float2 lds[B::LDS];
-  B b;
-  b.init(lds, wxy, tw, box, threadIdx.x);
-  const int xcd = blockIdx.x % 8, lid = blockIdx.x / 8, nper = gridDim.x / 8;
-  const long long items = (long long)npairs * B::H;
-  const long long i0 = items * xcd / 8, i1 = items * (xcd + 1) / 8;
-  for (long long it = i0 + lid; it < i1; it += nper) {
-    const int kx = (int)(it / npairs), p = (int)(it % npairs);
-    const int2 pr = pairs[p];
-    b.item(spectra + (size_t)pr.x * spec_stride + (size_t)kx * N,
-           spectra + (size_t)pr.y * spec_stride + (size_t)kx * N, wxy, wxy[kx],
-           tbuf + ((size_t)p * B::H + kx) * box);
-  }
-}
 
 // ----------------------------------------------- MFMA FP16 hi/lo form
 // The pruned inverse of a column (T of mc_cols.hip), decimated ky = a + A b
@@ -928,19 +762,6 @@ size_t pair_rows_part_elems(int npairs, int n, int box) {
 }
 
 
-template <int N, int M, int SP, bool F0 = false, int PL = 0>
-static hipError_t pair_cols_t(const float2* spectra, size_t spec_stride, const int2* pairs,
-                              int npairs, const float* wxy, int box, float2* tbuf,
-                              hipStream_t st) {
-  constexpr int NT = 256;
-  const float2* tw = twiddles(N);
-  if (!tw) return hipErrorOutOfMemory;
-  static const int grid = persistent_grid(k_pair_cols<N, M, NT, SP, F0, PL>, NT);
-  hipLaunchKernelGGL((k_pair_cols<N, M, NT, SP, F0, PL>), dim3(grid), dim3(NT), 0, st, spectra,
-                     spec_stride, pairs, npairs, wxy, box, tbuf, tw);
-  return hipGetLastError();
-}
-
 template <int N, int SP>
 static hipError_t pair_cols_mfma(const float2* spectra, size_t spec_stride, const int2* pairs,
                                  int npairs, const float* wxy, int box, float2* tbuf,
@@ -985,29 +806,8 @@ hipError_t launch_pair_cols(const float2* spectra, size_t spec_stride, const int
       default: return hipErrorInvalidValue;
     }
   }
-  if (n == 3710 && box <= 128)
-    // the default square crop of a 3838 x 3710 K2 frame: n = 70 * 53,
-    // decimated into 53 inverse 70-point FFTs (radix 2, 5, 7), the radix-2
-    // stage in registers on the loaded products
-    return pair_cols_t<3710, 70, 2, true>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st);
-  if (n == 4092 && box <= 128)
-    // the default square crop of a 5760 x 4092 K3 frame: n = 132 * 31,
-    // decimated into 31 inverse 132-point FFTs (radix 4, 3, 11)
-    return pair_cols_t<4092, 132, 2, true>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st);
-  if (box > 128) {
-    switch (n) {
-#define MC_COLS_256(NN) \
-  case NN: return pair_cols_t<NN, 256, 1>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st);
-      MC_COLS_256(256) MC_COLS_256(512) MC_COLS_256(768) MC_COLS_256(1024) MC_COLS_256(1280)
-      MC_COLS_256(1536) MC_COLS_256(2048) MC_COLS_256(2560) MC_COLS_256(3072) MC_COLS_256(3840)
-      MC_COLS_256(4096) MC_COLS_256(5120) MC_COLS_256(6144) MC_COLS_256(8192)
-#undef MC_COLS_256
-      default: break;
-    }
-    if (n % 128 == 0) return hipErrorInvalidValue;  // multiples of 128 take such boxes at 256 only
-  }
-  if (n == 64)
-    return pair_cols_t<64, 64, 1>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st);
+  // boxes above 128 on multiples of 128: at multiples of 256 only, as ever
+  if (box > 128 && n % 128 == 0 && n % 256) return hipErrorInvalidValue;
   return launch_pair_cols_fp32(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, st);
 }
 

@@ -1,7 +1,9 @@
 """The pair stage's column pass (mc_cols.hip) at the sizes where it can go
 wrong: transform sizes whose share per wave is full, ragged or a fraction of
-a wave, one to eight waves per item, boxes from 16 to the largest, odd ones
-and both sides of 96 among them.  Box maps of random spectra set directly,
+a wave, one to eight waves per item, every radix of the sizes that are not
+multiples of 128 (16, 14, 12, 10, 8, 6; even and odd shares, boxes of one to
+three tiles), boxes from 16 to the largest, odd ones and both sides of 96
+among them.  Box maps of random spectra set directly,
 against the FP64 cross power and inverse of the same spectra by numpy
 (cufunc.cu:343-370, DFAlign.cu:897, cufunc.cu:398-407).
 
@@ -44,7 +46,14 @@ def ctx():
     (128, 16), (128, 128), (256, 96), (256, 127), (512, 33), (512, 96), (512, 128), (768, 95),
     (1024, 64), (1024, 97), (1280, 96), (1280, 126), (1536, 17), (1920, 96), (2048, 96),
     (2560, 128), (3072, 70), (3840, 96), (3840, 128), (4096, 96), (5120, 96), (6144, 111),
-    (8192, 96), (8192, 128)])
+    (8192, 96), (8192, 128),
+    # radix 16, 14, 12, 10, 8, 6 (and 4096 with a box above 128)
+    (64, 33), (64, 64), (1808, 96), (1808, 129), (4096, 200), (512, 256),
+    (70, 64), (1022, 96), (3710, 96), (3710, 113), (3710, 224),
+    (132, 96), (4092, 96), (4092, 97), (4092, 192),
+    (110, 80), (2470, 96), (2470, 81), (2470, 160),
+    (72, 64), (1000, 65), (2472, 96), (2472, 192), (4024, 128),
+    (66, 48), (102, 49), (1854, 96), (1854, 97), (2046, 144), (4098, 96)])
 def test_box_maps_match_fp64(ctx, n, box):
     F = 3
     rng = np.random.default_rng(n + box)
