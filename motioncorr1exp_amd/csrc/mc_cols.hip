@@ -36,30 +36,35 @@ namespace mc {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-// n a multiple of 128, box <= 128.  ky = a + A (j + 4 r), A = n/64, j < 4,
+// n a multiple of 128, box <= 256.  ky = a + A (j + 4 r), A = n/64, j < 4,
 // r < 16.  Per (a, j) a 16-point DFT over r in registers; times
 // e^{2 pi i k (a + A j)/n}, which holds the twiddles of both later steps; per
 // (a, k) a 4-point DFT over j, giving Y_a[q] e^{2 pi i a k/n} with q the output
-// residue; then with the rows R = base + 16 g + k, base = n/2 - 64 (a multiple
-// of 64), g < 8, which contain every box up to 128,
+// residue; then with the rows R = base + 16 g + k, base = n/2 - 64 SETS (a
+// multiple of 64), g < 8 SETS, which contain every box up to 128 SETS,
 //   T[R] = sum_a e^{2 pi i a (base + 16 g)/n} (Y_a[g mod 4] e^{2 pi i a k/n}),
 // on v_mfma_f32_4x4x1 (16 blocks): block = (a mod 4, k / 4), columns k mod 4,
 // rows (re, im) of the factors of the groups q and q + 4.  The real and the
 // imaginary part of Y are multiplied by the same rows (D1, D2) and combined at
 // the end, which needs no second set of factors.  A wave takes up to 16 a of
 // all four j (64 lanes); the lanes' sums are added with lane swaps.
-// NG = 6 stores only the groups 1..6 (box <= 96), NG = 8 all.
+// NG = 6 stores only the groups 1..6 (box <= 96), NG = 8 all; NG = 16 takes a
+// second set of factors for the groups 8..15 (128 < box <= 256).
 // 128 VGPRs, 4 waves per SIMD (at 3 the pass takes 2.78 ms against 2.55).
 // 4096, 253 pairs: 2.5 ms; the two-stage 16 x 8 pass
 // with LDS combine that it replaces took 3.1.  2048, 153 pairs: 0.37 against
 // 0.47 and, untuned, 0.78.  Two pairs of one first operand per load of that
 // operand saved 6% of the issue and 25% of the loads and gave 2%: dropped.
+// Boxes above 128, 15 pairs: 4096, box 200: 0.24 ms against 0.25 for the
+// 256-point form of the former pass and 0.28 for k_pair_cols_r<16, 2>; 2048,
+// box 256: 67 us against 69 and 78.
 template <int NG>
-__global__ __launch_bounds__(512, 4) void k_pair_cols64(
+__global__ __launch_bounds__(512, NG > 8 ? 3 : 4) void k_pair_cols64(
     const float2* __restrict__ spectra, size_t spec_stride, const int2* __restrict__ pairs,
     int npairs, const float* __restrict__ wxy, int n, int box, float2* __restrict__ tbuf,
     const float2* __restrict__ tw, int kxb, int nkx) {
   extern __shared__ float4 cols_lds[];
+  constexpr int SETS = (NG + 7) / 8, NR = 128 * SETS;  // factor sets, rows R
   const int A = n / 64, nw = (A + 15) / 16, H = n / 2 + 1;
   const int AC = ((A + nw - 1) / nw + 1) / 2 * 2;  // a's per wave, even, <= 16
   const int tid = threadIdx.x, nt = nw * 64;
@@ -71,7 +76,7 @@ __global__ __launch_bounds__(512, 4) void k_pair_cols64(
   const bool act = 2 * ap < AC && a0 < A;
   const int voff = act ? 8 * (a0 + A * j + 32 * A * h) : n * 8;  // past the end: reads zero
   const int xi = act ? a0 + h + A * j : 0;
-  const int base = n / 2 - 64, ori = (n - box) / 2;
+  const int base = n / 2 - 64 * SETS, ori = (n - box) / 2;
   float wy[16];
 #pragma unroll
   for (int r = 0; r < 16; r++) wy[r] = wxy[H + xi + 4 * A * r];
@@ -79,13 +84,13 @@ __global__ __launch_bounds__(512, 4) void k_pair_cols64(
 #pragma unroll
   for (int k = 1; k < 16; k++) tk[k] = tw[k * xi];
   // matrix rows m = l % 4: (re, im) of the factor of group q + 4 (m / 2) at
-  // a = (l / 16) + 4 t of this wave
-  float P[4][4];
+  // a = (l / 16) + 4 t of this wave; q >= 4: the second set, groups 8 on
+  float P[4][4 * SETS];
 #pragma unroll
   for (int t = 0; t < 4; t++)
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int ac = (l >> 4) + 4 * t, a = w * AC + ac, g = q + 4 * ((l & 3) >> 1);
+    for (int q = 0; q < 4 * SETS; q++) {
+      const int ac = (l >> 4) + 4 * t, a = w * AC + ac, g = (q & 3) + 8 * (q >> 2) + 4 * ((l & 3) >> 1);
       const float2 f = ac < AC && a < A ? tw[a * (base + 16 * g) % n] : make_float2(0.f, 0.f);
       P[t][q] = (l & 1) ? f.y : f.x;
     }
@@ -94,7 +99,7 @@ __global__ __launch_bounds__(512, 4) void k_pair_cols64(
   const int zb = w * 8192 + (j * 16 + 2 * ap + h) * 128 + ap * 16;
   const int k = l & 15, al = l >> 4;
   const int rd = w * 8192 + al * 128 + (((k >> 1) ^ (al >> 1)) << 4) + (k & 1) * 8;
-  float* red = reinterpret_cast<float*>(cols_lds + nw * 512);  // [2][nw][128] complex
+  float* red = reinterpret_cast<float*>(cols_lds + nw * 512);  // [2][nw][NR] complex
   const int xcd = blockIdx.x % 8, lid = blockIdx.x / 8, nper = gridDim.x / 8;
   const long long items = (long long)npairs * nkx;
   const int i1 = (int)(items * (xcd + 1) / 8);
@@ -102,7 +107,7 @@ __global__ __launch_bounds__(512, 4) void k_pair_cols64(
   if (it >= i1) return;
   int kx = it / npairs, p = it - kx * npairs;
   const int dkx = nper / npairs, dp = nper - dkx * npairs;
-  for (int par = 0;; par ^= nw * 256) {
+  for (int par = 0;; par ^= nw * 2 * NR) {
     const int2 pr = pairs[p];
     const auto qa = buf_rsrc(spectra + (size_t)pr.x * spec_stride + (size_t)(kxb + kx) * n, n * 8);
     const auto qb = buf_rsrc(spectra + (size_t)pr.y * spec_stride + (size_t)(kxb + kx) * n, n * 8);
@@ -143,9 +148,9 @@ __global__ __launch_bounds__(512, 4) void k_pair_cols64(
       *reinterpret_cast<float4*>(reinterpret_cast<char*>(cols_lds) + (za ^ (16 * e))) =
           make_float4(v[2 * e].x, v[2 * e].y, v[2 * e + 1].x, v[2 * e + 1].y);
     wave_fence();
-    v4f D1[4], D2[4];
+    v4f D1[4 * SETS], D2[4 * SETS];
 #pragma unroll
-    for (int q = 0; q < 4; q++) D1[q] = D2[q] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int q = 0; q < 4 * SETS; q++) D1[q] = D2[q] = v4f{0.f, 0.f, 0.f, 0.f};
     int ra0 = rd;
     asm volatile("" : "+v"(ra0));
 #pragma unroll
@@ -157,28 +162,28 @@ __global__ __launch_bounds__(512, 4) void k_pair_cols64(
                                                  (ra0 ^ (t << 5)) + 512 * t + jj * 2048);
       dft4<1>(u);
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        D1[q] = __builtin_amdgcn_mfma_f32_4x4x1f32(P[t][q], u[q].x, D1[q], 0, 0, 0);
-        D2[q] = __builtin_amdgcn_mfma_f32_4x4x1f32(P[t][q], u[q].y, D2[q], 0, 0, 0);
+      for (int q = 0; q < 4 * SETS; q++) {
+        D1[q] = __builtin_amdgcn_mfma_f32_4x4x1f32(P[t][q], u[q & 3].x, D1[q], 0, 0, 0);
+        D2[q] = __builtin_amdgcn_mfma_f32_4x4x1f32(P[t][q], u[q & 3].y, D2[q], 0, 0, 0);
       }
     }
     wave_fence();
     // add the four a mod 4: lanes l < 32 end with the real parts, the others
     // with the imaginary ones; even rows of 16 lanes with group g, odd g + 1
-    constexpr int G0 = (8 - NG) / 2;
-    float S[8];
+    constexpr int G0 = (8 * SETS - NG) / 2;
+    float S[8 * SETS];
 #pragma unroll
-    for (int g = G0; g < 8 - G0; g++) {
-      const int q = g & 3, m = 2 * (g >> 2);
+    for (int g = G0; g < 8 * SETS - G0; g++) {
+      const int q = (g & 3) + 4 * (g >> 3), m = 2 * ((g >> 2) & 1);
       float re = D1[q][m] - D2[q][m + 1], im = D1[q][m + 1] + D2[q][m];
       swap32(re, im);
       S[g] = re + im;
     }
     int lt;  // the lane, made again per item: one register less in the loop
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(lt));
-    float* rw = red + par + w * 256 + (lt & 31) * 2 + (lt >> 5);
+    float* rw = red + par + w * 2 * NR + (lt & 31) * 2 + (lt >> 5);
 #pragma unroll
-    for (int g = G0; g < 8 - G0; g += 2) {
+    for (int g = G0; g < 8 * SETS - G0; g += 2) {
       swap16(S[g], S[g + 1]);
       rw[g * 32] = S[g] + S[g + 1];
     }
@@ -190,7 +195,7 @@ __global__ __launch_bounds__(512, 4) void k_pair_cols64(
     const auto qt = buf_rsrc(tbuf + ((size_t)p * H + kxb + kx) * box, box * 8);
     for (int r = w * 64 + lt; r < box; r += nt) {
       float2 s = rp[r + ori - base];
-      for (int x = 1; x < nw; x++) s = cadd(s, rp[x * 128 + r + ori - base]);
+      for (int x = 1; x < nw; x++) s = cadd(s, rp[x * NR + r + ori - base]);
       buf_st2(qt, 8 * r, cscale(s, wx));
     }
     it += nper;
@@ -260,18 +265,22 @@ __global__ __launch_bounds__(TILES == 1 || R0 <= 8 ? 1024 : 512, TILES == 1 || R
       wy[s + S * e] = own && !(twice && e == 0) ? wxy[H + x0 + e + A * (s + S * h)] : 0.f;
   float2 tk[R0];
 #pragma unroll
-  for (int k = 0; k < R0; k++) tk[k] = tw[(long long)xi * (k + (k < c ? R0 : 0)) % n];
+  for (int k = 0; k < R0; k++) {
+    const int e = xi * (k + (k < c ? R0 : 0));  // below 2 n
+    tk[k] = tw[e < n ? e : e - n];
+  }
   // matrix rows m = l % 16: (re, im) of group 8 tile + m / 2 at the xi of
   // exchange row 4 q + l / 16
   float P[NR][TILES];
 #pragma unroll
   for (int q = 0; q < NR; q++) {
     const int row = 4 * q + (l >> 4), xs = pair_start(row & 31);
-    const int x = xs < 0 ? 0 : xs + (row >> 5);
+    const unsigned x = xs < 0 ? 0 : xs + (row >> 5);
 #pragma unroll
     for (int t = 0; t < TILES; t++) {
       const int g = 8 * t + ((l & 15) >> 1);
-      const float2 f = g < G ? tw[(long long)x * (base + R0 * g) % n] : make_float2(0.f, 0.f);
+      // x < 1024 and n < 2^15: the product fits 32 bits
+      const float2 f = g < G ? tw[x * (unsigned)(base + R0 * g) % (unsigned)n] : make_float2(0.f, 0.f);
       P[q][t] = (l & 1) ? f.y : f.x;
     }
   }
@@ -432,7 +441,7 @@ static hipError_t cols64(const float2* spectra, size_t spec_stride, const int2* 
                          hipStream_t st) {
   static std::atomic<int> cache[16][17];
   const int nw = (n / 64 + 15) / 16;
-  const size_t lds = (size_t)nw * (8192 + 2048);
+  const size_t lds = (size_t)nw * (8192 + (NG > 8 ? 4096 : 2048));
   return cols_launches(k_pair_cols64<NG>, nw, lds, cache, npairs, n / 2 + 1,
                        [&](int grid, int kxb, int nkx) {
                          hipLaunchKernelGGL(k_pair_cols64<NG>, dim3(grid), dim3(nw * 64), lds, st,
@@ -474,8 +483,10 @@ hipError_t launch_pair_cols_fp32(const float2* spectra, size_t spec_stride, cons
                                  hipStream_t st) {
   const float2* tw = twiddles(n);
   if (!tw) return hipErrorOutOfMemory;
-  if (n % 128 == 0 && box <= 128) {
+  if (n % 128 == 0 && box <= 256) {
     if (box <= 96) return cols64<6>(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, tw, st);
+    if (box > 128)
+      return cols64<16>(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, tw, st);
     return cols64<8>(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, tw, st);
   }
   int tiles = 0;
