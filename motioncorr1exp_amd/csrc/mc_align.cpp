@@ -551,7 +551,7 @@ static int pair_reserve(mc_context_s* c, int np, int n, int box, int precision) 
   if (precision == MC_PREC_MFMA_HILO) HIP_TRY(c->tmax.ensure(sizeof(float) * (size_t)np * H));
   HIP_TRY(c->box.ensure(sizeof(float) * (size_t)np * box * box));
   HIP_TRY(c->boxpart.ensure(sizeof(float) * std::max<size_t>(1, mc::pair_rows_part_elems(np, n, box))));
-  HIP_TRY(c->peaks.ensure(sizeof(double) * mc::find_peaks_out_elems(np)));
+  HIP_TRY(c->peaks.ensure(sizeof(double) * 3 * (size_t)np));
   return MC_OK;
 }
 
@@ -813,7 +813,7 @@ extern "C" int mc_find_peaks(mc_context ctx, const float* boxmaps, int npairs, i
   if (!ctx || !boxmaps || npairs < 1 || box < 16) return set_err(MC_ERR_ARG, "bad arguments");
   HIP_TRY(hipSetDevice(ctx->device));
   HIP_TRY(ctx->box.ensure(sizeof(float) * (size_t)npairs * box * box));
-  HIP_TRY(ctx->peaks.ensure(sizeof(double) * mc::find_peaks_out_elems(npairs)));
+  HIP_TRY(ctx->peaks.ensure(sizeof(double) * 3 * (size_t)npairs));
   HIP_TRY(hipMemcpyAsync(ctx->box.p, boxmaps, sizeof(float) * (size_t)npairs * box * box,
                          hipMemcpyHostToDevice, ctx->st));
   HIP_TRY(mc::launch_find_peaks(ctx->box.as<float>(), npairs, box, n, wnoise,
@@ -1230,7 +1230,7 @@ struct PairPlan {
 // Reserves the pair buffers and uploads pairs (host slot pairs, span by span).
 static int pairs_prepare(mc_context_s* c, const std::vector<SizeGroup>& gs, PairPlan& L,
                          const std::vector<int>& slots) {
-  size_t np = 0, tel = 0, part = 0, pscr = 0;
+  size_t np = 0, tel = 0, part = 0;
   std::vector<size_t> gnp(gs.size(), 0);
   for (PairSpan& q : L.sp) {
     const int n = gs[q.gi].n;
@@ -1244,7 +1244,6 @@ static int pairs_prepare(mc_context_s* c, const std::vector<SizeGroup>& gs, Pair
   }
   for (size_t g = 0; g < gs.size(); g++) {
     part = std::max(part, mc::pair_rows_part_elems((int)gnp[g], gs[g].n, L.box));
-    pscr = std::max(pscr, mc::find_peaks_out_elems((int)gnp[g]) - 3 * gnp[g]);
   }
   if (slots.size() != 2 * np) return set_err(MC_ERR_ARG, "pair spans cover %zu of %zu pairs", np, slots.size() / 2);
   L.np = np;
@@ -1253,7 +1252,7 @@ static int pairs_prepare(mc_context_s* c, const std::vector<SizeGroup>& gs, Pair
   if (L.precision == MC_PREC_MFMA_HILO) HIP_TRY(c->tmax.ensure(sizeof(float) * std::max<size_t>(1, tel / L.box)));
   HIP_TRY(c->box.ensure(sizeof(float) * std::max<size_t>(1, np) * L.box * L.box));
   HIP_TRY(c->boxpart.ensure(sizeof(float) * std::max<size_t>(1, part)));
-  HIP_TRY(c->peaks.ensure(sizeof(double) * (3 * np + pscr + 1)));
+  HIP_TRY(c->peaks.ensure(sizeof(double) * 3 * std::max<size_t>(1, np)));
   HIP_TRY(hipMemcpyAsync(c->pairs_d.p, slots.data(), sizeof(int) * slots.size(), hipMemcpyHostToDevice,
                          c->st));
   return MC_OK;
@@ -1296,7 +1295,7 @@ static int pairs_launch(mc_context_s* c, const std::vector<SizeGroup>& gs, const
     {
       KScope ks(c, MC_KT_PEAKS);
       HIP_TRY(mc::launch_find_peaks(maps, np, box, n, L.wnoise, c->peaks.as<double>() + 3 * q.po,
-                                    c->st, c->peaks.as<double>() + 3 * L.np));
+                                    c->st));
     }
   }
   return MC_OK;

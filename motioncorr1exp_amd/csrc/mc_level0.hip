@@ -117,14 +117,14 @@ hipError_t launch_dc_gather(const float2* spectra, size_t stride, int nframes, d
 
 // ------------------------------------------------ FindShift without allocation
 // Device memory of mc_find_shift_noalloc: the box copied out of the caller's
-// map (MC_NOALLOC_MAX_BOX^2 floats), then the peak record of the search (the
-// result triple and the per-slice maxima, find_peaks_out_elems(1) doubles).
+// map (MC_NOALLOC_MAX_BOX^2 floats), then the result triple of the
+// search.
 // One copy per GPU, held until the process ends.  Every element a call reads
 // is written earlier in the same call, so nothing needs clearing between
 // calls; calls that overlap on one GPU race on it.
 namespace {
 constexpr size_t kNoallocBoxBytes = sizeof(float) * MC_NOALLOC_MAX_BOX * MC_NOALLOC_MAX_BOX;
-constexpr size_t kNoallocPeakDoubles = 32;
+constexpr size_t kNoallocPeakDoubles = 3;
 constexpr size_t kNoallocBytes = kNoallocBoxBytes + sizeof(double) * kNoallocPeakDoubles;
 }  // namespace
 
@@ -168,8 +168,6 @@ extern "C" int mc_find_shift_noalloc(const float* dsrc, int n, float* hboxmap, i
              box, MC_NOALLOC_MAX_BOX);
     return mc_internal_set_error(MC_ERR_ARG, buf);
   }
-  if (mc::find_peaks_out_elems(1) > kNoallocPeakDoubles)
-    return mc_internal_set_error(MC_ERR_ARG, "peak record exceeds the fixed scratch");
   unsigned char* base = nullptr;
   const int rc = noalloc_scratch(&base);
   if (rc != MC_OK) return rc;

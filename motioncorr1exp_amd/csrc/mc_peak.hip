@@ -17,8 +17,6 @@
 // a_0 = 1, a_kx = 2 (the C2R row weight), ky' = ky (ky < 8) or ky - 16.
 #include <hip/hip_runtime.h>
 
-#include <atomic>
-
 #include "mc_device.h"
 #include "mc_kernels.h"
 
@@ -52,232 +50,332 @@ MC_DEV void peak_result(int p, double v, int i, double u0, int offx, int offy, i
   out[3 * p + 2] = bv / n / n / 16 / 16;
 }
 
-// One workgroup per (pair, slice of 512/NS map rows), 512 threads.  NS = 1
-// writes the result; NS > 1 writes the slice's (max value, index, U[0],
-// window origin) to part[(p NS + slice) 5 ...] for k_find_peaks_final.
-template <int NT, int NS>
-__global__ __launch_bounds__(NT) void k_find_peaks(const float* __restrict__ boxmaps, int box,
-                                                   int n, int wnoise, double* __restrict__ out,
-                                                   double* __restrict__ part) {
-  static_assert(NT == 256 || NT == 512, "threads");
-  __shared__ double sv[NT];
-  __shared__ int si[NT];
-  __shared__ double sub[16][16];
+MC_DEV ValIdx wave_first_max(ValIdx b) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) b = better(b, ValIdx{__shfl_xor(b.v, o), __shfl_xor(b.i, o)});
+  return b;
+}
+
+// One workgroup per pair, 512 threads.
+//
+// What bounds it is FP64 issue: all 512 x 512 points cost 16 multiply-adds and
+// six instructions of comparison each, 107 us for 253 pairs (one workgroup per
+// CU), and for few pairs the serial chain of the steps before.  Only the first
+// maximum is wanted, so the points are searched in 64 x 64 cells of 8 x 8: with
+// T, Tx and Ty at the cell's centre, no point of the cell exceeds
+//   T + h (|Tx| + |Ty|) + h^2/2 sum |A| (|kx| + |ky|)^2,   h = 4 steps,
+// the Taylor bound of the trigonometric sum with coefficients A.  Cells whose
+// bound lies below the largest T found at an admitted centre hold no maximum;
+// the points of the others (10 to 40 of the 4096 cells for box maps with a
+// peak, up to 100 for noise) are evaluated as in the full search, so the
+// result is the same bit for bit.  1e-10 sum |A| covers the rounding of T and
+// of the points (about 1e-14).  A map without a bound (NaN, infinities) or
+// without structure (constant) keeps all cells (330 us).
+// 96 x 96 maps: 22 us up to 256 pairs, 37 to 46 for noise; the full search took
+// 51 (40 pairs, four workgroups each and a launch to combine them), 70 (105)
+// and 106 (253).  What is left is latency: one wave issues an instruction in
+// about 6 clocks and no step has work for more than two waves per SIMD.
+constexpr int PEAK_NT = 512, PEAK_CELL = 8, PEAK_NCELL = 512 / PEAK_CELL;
+constexpr int PEAK_ROWS = 14;  // cell rows whose row sums are held at a time
+
+__global__ __launch_bounds__(PEAK_NT) void k_find_peaks(const float* __restrict__ boxmaps, int box,
+                                                        int n, int wnoise, double* __restrict__ out) {
+  constexpr int NT = PEAK_NT, NW = NT / 64;
+  __shared__ double2 t512[512 + 64];  // entry e at e + e/8: no stride of 8 in one bank
+  __shared__ __align__(16) float sub[256];
+  __shared__ __align__(256) double tab[2][16];  // cos, -sin of 2 pi e/16
   __shared__ double2 G[16][9];
-  __shared__ double2 t512[512];
-  __shared__ int soff[2];
+  __shared__ double2 Hs[PEAK_ROWS * PEAK_CELL * 9];  // row sums; the centre rows' [64][9] before
+  __shared__ double2 Hy[PEAK_NCELL * 9];
+  __shared__ double rv[NW], rs[NW];
+  __shared__ int ri[NW];
+  __shared__ unsigned long long keep[PEAK_NCELL];
+  __shared__ double u0s;
+  static_assert(PEAK_ROWS * PEAK_CELL >= PEAK_NCELL, "the centre rows share Hs");
+  static_assert(NW == PEAK_CELL && PEAK_NCELL == 64, "waves are a cell's rows, a ballot a row of cells");
   const int p = blockIdx.x;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
   const float* bm = boxmaps + (size_t)p * box * box;
-  for (int i = tid; i < 512; i += NT) {
+  auto tw = [&](int e) {  // e^{2 pi i e/512}
+    e &= 511;
+    return t512[e + (e >> 3)];
+  };
+  {
     double s, c;
-    sincospi((double)i / 256.0, &s, &c);
-    t512[i] = make_double2(c, s);
-  }
-  // 1. integer peak (cufunc.cu:409-424)
-  ValIdx best = {-1e9, 0x7fffffff};
-  for (int i = tid; i < box * box; i += NT) {
-    const int r = i / box, c = i % box;
-    if (abs(c - box / 2) <= wnoise && abs(r - box / 2) <= wnoise) continue;
-    const double v = (double)bm[i];
-    if (v > best.v) best = ValIdx{v, i};
-  }
-  sv[tid] = best.v;
-  si[tid] = best.i;
-  __syncthreads();
-  for (int o = NT / 2; o > 0; o >>= 1) {
-    if (tid < o) {
-      ValIdx a{sv[tid], si[tid]}, b{sv[tid + o], si[tid + o]};
-      a = better(a, b);
-      sv[tid] = a.v;
-      si[tid] = a.i;
+    sincospi((double)tid / 256.0, &s, &c);
+    t512[tid + (tid >> 3)] = make_double2(c, s);
+    if (tid % 32 == 0) {
+      tab[0][tid / 32] = c;
+      tab[1][tid / 32] = -s;
     }
-    __syncthreads();
   }
-  if (tid == 0) {
-    int ix = 0, iy = 0;
-    if (si[0] != 0x7fffffff) {  // no candidate: the reference keeps (0, 0)
-      ix = si[0] % box;
-      iy = si[0] / box;
-    }
-    int offx = ix - 8, offy = iy - 8;  // cufunc.cu:430-435
-    if (offx + 16 > box) offx = box - 16;
-    else if (offx < 0) offx = 0;
-    if (offy + 16 > box) offy = box - 16;
-    else if (offy < 0) offy = 0;
-    soff[0] = offx;
-    soff[1] = offy;
-  }
-  __syncthreads();
-  const int offx = soff[0], offy = soff[1];
-  if (tid < 256) sub[tid / 16][tid % 16] = (double)bm[(size_t)(offy + tid / 16) * box + offx + tid % 16];
-  __syncthreads();
-  // 2. 16 x 16 R2C (forward) and cosine mask, times the C2R row weight
-  if (tid < 144) {
-    const int ky = tid / 9, kx = tid % 9;
-    double re = 0, im = 0;
-    for (int y = 0; y < 16; y++)
-      for (int x = 0; x < 16; x++) {
-        const int e = ((kx * x + ky * y) & 15) * 32;  // e^{-2 pi i e/512}
-        const double2 w = t512[e];
-        re += sub[y][x] * w.x;
-        im -= sub[y][x] * w.y;
+  // 1. integer peak (cufunc.cu:409-424); 18 loads in flight
+  {
+    float bv = -1e9f;
+    int bi = 0x7fffffff;
+    const int dr = NT / box, dc = NT - dr * box, nb = box * box;
+    int r = tid / box, c = tid - r * box;
+    for (int i0 = tid; i0 < nb; i0 += 18 * NT) {
+      float v[18];
+#pragma unroll
+      for (int e = 0; e < 18; e++) v[e] = bm[min(i0 + e * NT, nb - 1)];
+#pragma unroll
+      for (int e = 0; e < 18; e++) {
+        const int i = i0 + e * NT;
+        // selects, no branches: integer products of the conditions
+        const int ex = int(abs(c - box / 2) <= wnoise) & int(abs(r - box / 2) <= wnoise);
+        const int up = int(i < nb) & (ex ^ 1) & int(v[e] > bv);
+        bv = up ? v[e] : bv;
+        bi = up ? i : bi;
+        c += dc;
+        const int wrap = c >= box;
+        c -= wrap ? box : 0;
+        r += dr + wrap;
       }
-    const int yy = ky < 8 ? ky : ky - 16;
-    const int rr = (int)sqrt((double)(kx * kx + yy * yy));
-    double m = 0.0;
-    if (rr < 8) m = cospi((double)rr / 8.0) / 2 + 0.5;
-    if (kx > 0) m *= 2.0;
-    G[ky][kx] = make_double2(re * m, im * m);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const float v = __shfl_xor(bv, o);
+      const int i = __shfl_xor(bi, o);
+      if (v > bv || (v == bv && i < bi)) {
+        bv = v;
+        bi = i;
+      }
+    }
+    if (l == 0) {
+      rv[w] = bv;
+      ri[w] = bi;
+    }
   }
   __syncthreads();
-  // 3-4. exact evaluation of the 512 x 512 interpolated map, first maximum.
-  // Thread t owns the columns c0 + 128 j (c0 = t % 128, j < 4) in the rows
-  // q = t / 128 mod 4: the eight twiddles of each column stay in registers, and
-  // the row sums Hq[kx] of QC rows at a time are formed in LDS, where every
-  // lane reads the same address (a broadcast).  Each point keeps the
-  // arithmetic of a per-point evaluation, so the map does not depend on the
-  // thread layout; the first maximum in row-major order is the reduction's
-  // (value, smallest index).
-  static_assert(NT == 512, "four columns and one row class per thread");
-  constexpr int QC = 128;
-  __shared__ double2 Hs[QC][9];
+  ValIdx pk = {rv[0], ri[0]};
+#pragma unroll
+  for (int x = 1; x < NW; x++) pk = better(pk, ValIdx{rv[x], ri[x]});
+  int offx = -8, offy = -8;  // no candidate: the reference keeps (0, 0)
+  if (pk.i != 0x7fffffff) {
+    offx = pk.i % box - 8;
+    offy = pk.i / box - 8;
+  }
+  if (offx + 16 > box) offx = box - 16;  // cufunc.cu:430-435
+  else if (offx < 0) offx = 0;
+  if (offy + 16 > box) offy = box - 16;
+  else if (offy < 0) offy = 0;
+  offx = __builtin_amdgcn_readfirstlane(offx);
+  offy = __builtin_amdgcn_readfirstlane(offy);
+  if (tid < 256) sub[tid] = bm[(size_t)(offy + tid / 16) * box + offx + tid % 16];
+  __syncthreads();
+  // 2. 16 x 16 R2C (forward) and cosine mask, times the C2R row weight.  A
+  // thread sums the real or the imaginary part of ky and of ky + 8, whose
+  // factors differ by (-1)^y.
+  if (tid < 144) {
+    const int part = tid >= 72, o = tid - 72 * part, ky = o / 9, kx = o - 9 * ky;
+    int ex[16];
+#pragma unroll
+    for (int x = 0; x < 16; x++) ex[x] = 8 * kx * x;
+    double s0 = 0, s1 = 0;
+#pragma unroll 2
+    for (int y = 0; y < 16; y++) {
+      const int ey = 8 * ky * y;
+#pragma unroll
+      for (int x = 0; x < 16; x++) {
+        unsigned a = (ey + ex[x]) & 127 | part * 128;
+        asm("" : "+v"(a));  // keeps the table's address out of the sum
+        const double t = *reinterpret_cast<const double*>(reinterpret_cast<const char*>(tab) + a);
+        const double v = (double)sub[16 * y + x];
+        s0 = fma(v, t, s0);
+        s1 = fma(v, (y & 1) ? -t : t, s1);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      const int yy = e ? ky - 8 : ky;
+      // floor(sqrt(kx^2 + yy^2)), up to 8; cos(pi r/8) is the table's
+      int rr = 0;
+#pragma unroll
+      for (int i = 1; i <= 8; i++) rr += kx * kx + yy * yy >= i * i;
+      double m = rr < 8 ? tab[0][rr] / 2 + 0.5 : 0.0;
+      if (kx > 0) m *= 2.0;
+      double2& g = G[ky + 8 * e][kx];
+      (part ? g.y : g.x) = (e ? s1 : s0) * m;
+    }
+  }
+  __syncthreads();
+  // 3. the bound's constant term, and T, Tx, Ty at the cell centres (8 R, 8 C):
+  // row sums of the centre rows, then a thread takes the columns C = l % 16 + 16 k,
+  // k < 4, whose factors differ by i^(kx k), in the rows R = 4 w + 32 j + l / 16
+  {
+    double s = 0.0;
+    constexpr double h = PEAK_CELL / 2 * 2 * 3.14159265358979323846 / 512;
+    if (tid < 144) {
+      const int ky = tid / 9, kx = tid - 9 * ky, yy = ky < 8 ? ky : 16 - ky;
+      const double k = (kx + yy) * h;
+      s = (fabs(G[ky][kx].x) + fabs(G[ky][kx].y)) * (0.5 * k * k + 1e-10);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (l == 0) rs[w] = s;
+  }
+  // (rows R and R + 32, whose factors differ by (-1)^yy, per thread)
+  if (tid < PEAK_NCELL / 2 * 9) {
+    const int q = PEAK_CELL * (tid / 9), kx = tid % 9;
+    double2 h[2] = {}, d[2] = {};
+#pragma unroll
+    for (int ky = 0; ky < 16; ky++) {
+      const int yy = ky < 8 ? ky : ky - 16;
+      const double2 t = tw(yy * q), g = G[ky][kx];
+      const double2 v = make_double2(g.x * t.x - g.y * t.y, g.x * t.y + g.y * t.x);
+      double2& a = h[ky & 1];
+      double2& b = d[ky & 1];
+      a.x += v.x;
+      a.y += v.y;
+      b.x -= yy * v.y;
+      b.y += yy * v.x;
+    }
+    constexpr int up = PEAK_NCELL / 2 * 9;
+    Hs[tid] = make_double2(h[0].x + h[1].x, h[0].y + h[1].y);
+    Hs[tid + up] = make_double2(h[0].x - h[1].x, h[0].y - h[1].y);
+    Hy[tid] = make_double2(d[0].x + d[1].x, d[0].y + d[1].y);
+    Hy[tid + up] = make_double2(d[0].x - d[1].x, d[0].y - d[1].y);
+  }
+  __syncthreads();
   const int scale = 32;
   const int wns = scale * wnoise;
   const int ox = (box / 2 - offx) * scale, oy = (box / 2 - offy) * scale;
-  constexpr int NC = 4;
-  const int c0 = tid % (512 / NC), par = tid / (512 / NC);
-  double2 wc[NC][8];
+  double bound[2][4], m0 = -1e300;
+  {
+    constexpr double h = PEAK_CELL / 2 * 2 * 3.14159265358979323846 / 512;
+    const double b2 = rs[0] + rs[1] + rs[2];
+    const int c0 = PEAK_CELL * (l & 15);
 #pragma unroll
-  for (int j = 0; j < NC; j++)
+    for (int j = 0; j < 2; j++) {
+      const int R = 4 * w + 32 * j + (l >> 4), q = PEAK_CELL * R;
+      // sums of the terms kx = m mod 4 (complex: T and Tx take both parts)
+      double2 S[4] = {}, X[4] = {}, Y[4] = {};
+      S[0].x = Hs[R * 9].x;
+      Y[0].x = Hy[R * 9].x;
 #pragma unroll
-    for (int kx = 1; kx < 9; kx++) wc[j][kx - 1] = t512[(kx * (c0 + (512 / NC) * j)) & 511];
+      for (int kx = 1; kx < 9; kx++) {
+        const double2 t = tw(kx * c0), a = Hs[R * 9 + kx], d = Hy[R * 9 + kx];
+        const double2 v = make_double2(a.x * t.x - a.y * t.y, a.x * t.y + a.y * t.x);
+        const int m = kx & 3;
+        S[m].x += v.x;
+        S[m].y += v.y;
+        X[m].x -= kx * v.y;
+        X[m].y += kx * v.x;
+        Y[m].x += d.x * t.x - d.y * t.y;
+        Y[m].y += d.x * t.y + d.y * t.x;
+      }
+      // Re sum_m i^(m k) z[m]
+      auto at = [](const double2* z, int k) {
+        const double e = (k & 1) ? z[0].x - z[2].x : z[0].x + z[2].x;
+        return k == 0 ? e + (z[1].x + z[3].x) : k == 1 ? e - (z[1].y - z[3].y)
+             : k == 2 ? e - (z[1].x + z[3].x) : e + (z[1].y - z[3].y);
+      };
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const double T = at(S, k);
+        bound[j][k] = T + h * (fabs(at(X, k)) + fabs(at(Y, k))) + b2;
+        if (!(abs(q - oy) <= wns && abs(c0 + 128 * k - ox) <= wns) && T > m0) m0 = T;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m0 = fmax(m0, __shfl_xor(m0, o));
+    if (l == 0) rv[w] = m0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int x = 0; x < NW; x++) m0 = fmax(m0, rv[x]);
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    unsigned long long b[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) b[k] = __ballot(!(bound[j][k] < m0));
+    if (l < 4) {
+      const int R = 4 * w + 32 * j + l;
+      unsigned long long k = 0;
+#pragma unroll
+      for (int x = 0; x < 4; x++) k |= (b[x] >> (16 * l) & 0xffff) << (16 * x);
+      // cell (0, 0) is always kept: the search starts from U[0]
+      keep[R] = R == 0 ? k | 1 : k;
+    }
+  }
+  __syncthreads();
+  // 4. exact evaluation of the kept cells, first maximum
   ValIdx bb = {-1e300, 0x7fffffff};
-  double u0 = 0.0;
-  static_assert((512 / NS) % QC == 0, "whole row chunks per slice");
-  const int qb = blockIdx.y * (512 / NS);
-  for (int q0 = qb; q0 < qb + 512 / NS; q0 += QC) {
-    __syncthreads();  // the previous chunk's rows are read
-    for (int i = tid; i < QC * 9; i += NT) {
-      const int q = q0 + i / 9, kx = i % 9;
+  unsigned long long rows = __ballot(keep[l] != 0);
+  while (rows) {
+    // the next (up to PEAK_ROWS) cell rows: row sums, then wave w takes row w of
+    // each cell and 64 lanes the points of eight cells
+    unsigned long long todo = rows;
+    int nr = 0;
+    for (; nr < PEAK_ROWS && rows; nr++) rows &= rows - 1;
+    for (int i = tid; i < nr * PEAK_CELL * 9; i += NT) {
+      const int s = i / (PEAK_CELL * 9), e = i - s * (PEAK_CELL * 9), dq = e / 9, kx = e - 9 * dq;
+      unsigned long long t = todo;
+      for (int x = 0; x < s; x++) t &= t - 1;
+      const int q = PEAK_CELL * (__ffsll((long long)t) - 1) - PEAK_CELL / 2 + dq;
       double2 h = make_double2(0.0, 0.0);
+#pragma unroll
       for (int ky = 0; ky < 16; ky++) {
         const int yy = ky < 8 ? ky : ky - 16;
-        const double2 w = t512[(yy * q) & 511];
+        const double2 t = tw(yy * q);
         const double2 g = G[ky][kx];
-        h.x += g.x * w.x - g.y * w.y;
-        h.y += g.x * w.y + g.y * w.x;
+        h.x += g.x * t.x - g.y * t.y;
+        h.y += g.x * t.y + g.y * t.x;
       }
-      Hs[i / 9][kx] = h;
+      Hs[i] = h;
     }
     __syncthreads();
-    for (int qi = par; qi < QC; qi += NC) {
-      const int q = q0 + qi;
-      const bool rowex = abs(q - oy) <= wns;
+    for (int s = 0; s < nr; s++, todo &= todo - 1) {
+      const int R = __ffsll((long long)todo) - 1;
+      const int q = (PEAK_CELL * R - PEAK_CELL / 2 + w) & 511;
       double2 hq[9];
 #pragma unroll
-      for (int kx = 0; kx < 9; kx++) hq[kx] = Hs[qi][kx];
+      for (int kx = 0; kx < 9; kx++) hq[kx] = Hs[(s * PEAK_CELL + w) * 9 + kx];
+      for (unsigned long long k = keep[R]; k;) {
+        unsigned long long mine = k;
 #pragma unroll
-      for (int j = 0; j < NC; j++) {
-        const int pp = c0 + (512 / NC) * j;
+        for (int x = 0; x < 8; x++) {
+          if (x < l / PEAK_CELL) mine &= mine - 1;
+          k &= k - 1;
+        }
+        if (!mine) continue;
+        const int C = __ffsll((long long)mine) - 1;
+        const int pp = (PEAK_CELL * C - PEAK_CELL / 2 + l % PEAK_CELL) & 511;
         double u = hq[0].x;
 #pragma unroll
-        for (int kx = 1; kx < 9; kx++) u += hq[kx].x * wc[j][kx - 1].x - hq[kx].y * wc[j][kx - 1].y;
-        if (q == 0 && pp == 0) u0 = u;
-        if (rowex && abs(pp - ox) <= wns) continue;
-        if (u > bb.v) bb = ValIdx{u, q * 512 + pp};
+        for (int kx = 1; kx < 9; kx++) {
+          const double2 t = tw(kx * pp);
+          u += hq[kx].x * t.x - hq[kx].y * t.y;
+        }
+        if (q == 0 && pp == 0) u0s = u;
+        if (abs(q - oy) <= wns && abs(pp - ox) <= wns) continue;
+        // rows and cells wrap round: the points come in no particular order
+        if (u > bb.v || (u == bb.v && q * 512 + pp < bb.i)) bb = ValIdx{u, q * 512 + pp};
       }
-    }
-  }
-  __syncthreads();
-  sv[tid] = bb.v;
-  si[tid] = bb.i;
-  __syncthreads();
-  for (int o = NT / 2; o > 0; o >>= 1) {
-    if (tid < o) {
-      ValIdx a{sv[tid], si[tid]}, b{sv[tid + o], si[tid + o]};
-      a = better(a, b);
-      sv[tid] = a.v;
-      si[tid] = a.i;
     }
     __syncthreads();
   }
+  bb = wave_first_max(bb);
+  if (l == 0) {
+    rs[w] = bb.v;
+    ri[w] = bb.i;
+  }
+  __syncthreads();
   if (tid == 0) {
-    if (NS == 1) {
-      peak_result(p, sv[0], si[0], u0, offx, offy, box, n, out);
-    } else {
-      // U[0] is evaluated by thread 0 of slice 0 (row 0, column 0)
-      double* q = part + ((size_t)p * NS + blockIdx.y) * 5;
-      q[0] = sv[0];
-      q[1] = (double)si[0];
-      q[2] = u0;
-      q[3] = offx;
-      q[4] = offy;
-    }
-  }
-}
-
-// Combines the NS slices of each pair (one thread per pair): first maximum
-// in row-major order over the slices, then the result as for one slice.
-template <int NS>
-__global__ __launch_bounds__(64) void k_find_peaks_final(const double* __restrict__ part,
-                                                         int npairs, int box, int n,
-                                                         double* __restrict__ out) {
-  const int p = blockIdx.x * 64 + threadIdx.x;
-  if (p >= npairs) return;
-  const double* q = part + (size_t)p * NS * 5;
-  ValIdx b = {q[0], (int)q[1]};
+    bb = ValIdx{rs[0], ri[0]};
 #pragma unroll
-  for (int s = 1; s < NS; s++) b = better(b, ValIdx{q[5 * s], (int)q[5 * s + 1]});
-  peak_result(p, b.v, b.i, q[2], (int)q[3], (int)q[4], box, n, out);
-}
-
-// Row slices per pair: one workgroup per pair fills the device from half as
-// many pairs as CUs; fewer pairs split their maps over 2 or 4 workgroups.
-static int peak_slices(int npairs) {
-  static std::atomic<int> cache[64];
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  if (dev < 0 || dev >= 64) dev = 0;
-  int cus = cache[dev].load(std::memory_order_relaxed);
-  if (cus <= 0) {
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus <= 0)
-      cus = 256;
-    cache[dev].store(cus, std::memory_order_relaxed);
+    for (int x = 1; x < NW; x++) bb = better(bb, ValIdx{rs[x], ri[x]});
+    peak_result(p, bb.v, bb.i, u0s, offx, offy, box, n, out);
   }
-  return npairs >= cus / 2 ? 1 : (npairs >= cus / 4 ? 2 : 4);
-}
-
-size_t find_peaks_out_elems(int npairs) {
-  const int ns = peak_slices(npairs);
-  return (size_t)npairs * 3 + (ns > 1 ? (size_t)npairs * ns * 5 : 0);
 }
 
 hipError_t launch_find_peaks(const float* boxmaps, int npairs, int box, int n, int wnoise,
-                             double* out, hipStream_t st, double* part) {
+                             double* out, hipStream_t st) {
   if (npairs <= 0) return hipSuccess;
   if (box < 16) return hipErrorInvalidValue;
-  if (!part) part = out + (size_t)npairs * 3;
-  const unsigned fg = (unsigned)((npairs + 63) / 64);
-  switch (peak_slices(npairs)) {
-    case 1:
-      hipLaunchKernelGGL((k_find_peaks<512, 1>), dim3(npairs), dim3(512), 0, st, boxmaps, box, n,
-                         wnoise, out, part);
-      break;
-    case 2:
-      hipLaunchKernelGGL((k_find_peaks<512, 2>), dim3(npairs, 2), dim3(512), 0, st, boxmaps, box,
-                         n, wnoise, out, part);
-      hipLaunchKernelGGL(k_find_peaks_final<2>, dim3(fg), dim3(64), 0, st, part, npairs, box, n,
-                         out);
-      break;
-    default:
-      hipLaunchKernelGGL((k_find_peaks<512, 4>), dim3(npairs, 4), dim3(512), 0, st, boxmaps, box,
-                         n, wnoise, out, part);
-      hipLaunchKernelGGL(k_find_peaks_final<4>, dim3(fg), dim3(64), 0, st, part, npairs, box, n,
-                         out);
-      break;
-  }
+  hipLaunchKernelGGL(k_find_peaks, dim3(npairs), dim3(PEAK_NT), 0, st, boxmaps, box, n, wnoise, out);
   return hipGetLastError();
 }
 
