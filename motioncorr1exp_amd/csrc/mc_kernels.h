@@ -174,16 +174,14 @@ hipError_t launch_small_c2r(const float2* X, int ld, int d, float div, float2* t
                             hipStream_t st);
 hipError_t launch_disp_short(const float* buf, int size, short* out, hipStream_t st);
 
-// Sharpness J of the shifted sum S (already formed by launch_shift_sum with
-// the same shifts) and dJ/ds_f: out[f] = (dJ/dsx_f, dJ/dsy_f), out[F] = (J, 0).
-// wk: [n/2+1] column weights (incl. the half-plane factor) then [n] row
-// weights, w(kx, ky) = wk[kx] * wk[n/2+1+ky].  part: nchunks*(F+1) double2.
-// jonly = 1 computes only J (out[F]; out[0..F) are then not meaningful), with
-// the same blocks and summation order as the full pass.
+// Shifted sum S of the frames (as launch_shift_sum forms it), its sharpness J
+// and dJ/ds_f: out[f] = (dJ/dsx_f, dJ/dsy_f), out[F] = (J, 0).  wk: [n/2+1]
+// column weights (incl. the half-plane factor) then [n] row weights, w(kx, ky)
+// = wk[kx] * wk[n/2+1+ky].  part: sharp_part_elems(F, n) double2.
+size_t sharp_part_elems(int nframes, int n);
 hipError_t launch_sharpness(const float2* spectra, size_t spec_stride, int nframes, int n,
-                            const double2* shifts, const float2* S, const float* wk,
-                            double2* part, int nchunks, double2* out, int jonly,
-                            hipStream_t st);
+                            const double2* shifts, float2* S, const float* wk, double2* part,
+                            double2* out, hipStream_t st);
 
 // Layout conversion between the resident [kx][ky] spectrum and the padded
 // row-major [ky][kx] layout (n rows of n/2+1 complex).

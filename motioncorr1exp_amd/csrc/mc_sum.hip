@@ -16,10 +16,65 @@
 
 namespace mc {
 
-// Frames are consumed in groups of U whose loads are issued together (the
-// loop over frames is otherwise a chain of dependent load-use latencies);
-// the accumulation order is the frame order either way.
+// Element e (kx, yy) of the frames f0 .. f0 + U - 1 times its phase factor.
+// All loads are issued together, whatever the shifts are: a test before each
+// would make the load wait for the shift (2048, 24 frames: 84 us with the tests,
+// 78 without).  NaN: frame not summed, value zero.  y2 is the imaginary part
+// with the other of its two products rounded.
 template <int U>
+MC_DEV void rotate_frames(const float2* __restrict__ spectra, size_t spec_stride,
+                          const double2* __restrict__ shifts, int f0, size_t e, int kx, int yy,
+                          double inv_n, float2 (&g)[U], float (&y2)[U]) {
+  double2 s[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    g[u] = spectra[(size_t)(f0 + u) * spec_stride + e];
+    s[u] = shifts[f0 + u];
+  }
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    // contractions written out: sum and gradient keep their rounding wherever
+    // this is compiled into
+    double w = fma(s[u].x, (double)kx, s[u].y * yy);
+    w = fma(inv_n, w, -floor(inv_n * w));
+    float sn, cs;
+    sincospif(2.0f * (float)w, &sn, &cs);
+    const float2 v = g[u];
+    const bool in = s[u].x == s[u].x;
+    g[u].x = in ? fmaf(v.x, cs, -(v.y * sn)) : 0.f;
+    g[u].y = in ? fmaf(v.y, cs, v.x * sn) : 0.f;
+    y2[u] = in ? fmaf(v.x, sn, v.y * cs) : 0.f;
+  }
+}
+// use(f, value, y2) for all frames in order: groups of eight, of four, single ones
+template <class F>
+MC_DEV void rotate_all(const float2* __restrict__ spectra, size_t spec_stride,
+                       const double2* __restrict__ shifts, int nframes, size_t e, int kx, int yy,
+                       double inv_n, F&& use) {
+  int f = 0;
+  for (; f + 8 <= nframes; f += 8) {
+    float2 g[8];
+    float y2[8];
+    rotate_frames<8>(spectra, spec_stride, shifts, f, e, kx, yy, inv_n, g, y2);
+#pragma unroll
+    for (int u = 0; u < 8; u++) use(f + u, g[u], y2[u]);
+  }
+  if (f + 4 <= nframes) {
+    float2 g[4];
+    float y2[4];
+    rotate_frames<4>(spectra, spec_stride, shifts, f, e, kx, yy, inv_n, g, y2);
+#pragma unroll
+    for (int u = 0; u < 4; u++) use(f + u, g[u], y2[u]);
+    f += 4;
+  }
+  for (; f < nframes; f++) {
+    float2 g[1];
+    float y2[1];
+    rotate_frames<1>(spectra, spec_stride, shifts, f, e, kx, yy, inv_n, g, y2);
+    use(f, g[0], y2[0]);
+  }
+}
+
 __global__ __launch_bounds__(256) void k_shift_sum(const float2* __restrict__ spectra,
                                                    size_t spec_stride, int nframes, int n,
                                                    const double2* __restrict__ shifts,
@@ -30,30 +85,11 @@ __global__ __launch_bounds__(256) void k_shift_sum(const float2* __restrict__ sp
   if (e >= total) return;
   const int kx = (int)(e / n), ky = (int)(e % n);
   const int yy = ky < n / 2 ? ky : ky - n;
-  const double inv_n = 1.0 / n;
   float2 acc = make_float2(0.f, 0.f), acc2 = make_float2(0.f, 0.f);
-  for (int f0 = 0; f0 < nframes; f0 += U) {
-    float2 v[U];
-    double2 sh[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      sh[u] = f0 + u < nframes ? shifts[f0 + u] : make_double2(NAN, NAN);
-      v[u] = sh[u].x == sh[u].x ? spectra[(size_t)(f0 + u) * spec_stride + e] : make_float2(0.f, 0.f);
-    }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int f = f0 + u;
-      const double2 s = sh[u];
-      if (s.x != s.x) continue;  // NaN: frame not summed (or past the end)
-      double w = (s.x * kx + s.y * yy) * inv_n;
-      w -= floor(w);
-      float sn, cs;
-      sincospif(2.0f * (float)w, &sn, &cs);
-      const float2 t = cmul(v[u], make_float2(cs, sn));
-      acc = cadd(acc, t);
-      if (sum2 && f <= f2_last) acc2 = cadd(acc2, t);
-    }
-  }
+  rotate_all(spectra, spec_stride, shifts, nframes, e, kx, yy, 1.0 / n, [&](int f, float2 t, float) {
+    acc = cadd(acc, t);
+    if (sum2 && f <= f2_last) acc2 = cadd(acc2, t);
+  });
   sum[e] = acc;
   if (sum2) sum2[e] = acc2;
 }
@@ -62,7 +98,7 @@ hipError_t launch_shift_sum(const float2* spectra, size_t spec_stride, int nfram
                             const double2* shifts, float2* sum, float2* sum2, int f2_last,
                             hipStream_t st) {
   const size_t total = (size_t)(n / 2 + 1) * n;
-  hipLaunchKernelGGL(k_shift_sum<8>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
+  hipLaunchKernelGGL(k_shift_sum, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
                      spectra, spec_stride, nframes, n, shifts, sum, sum2, f2_last);
   return hipGetLastError();
 }
@@ -80,29 +116,9 @@ __global__ __launch_bounds__(256) void k_shift_sum_multi(float2* spectra, size_t
   const int4 jb = jobs[blockIdx.y];
   const int kx = (int)(e / n), ky = (int)(e % n);
   const int yy = ky < n / 2 ? ky : ky - n;
-  const double inv_n = 1.0 / n;
   float2 acc = make_float2(0.f, 0.f);
-  constexpr int U = 8;
-  for (int f0 = 0; f0 < jb.y; f0 += U) {
-    float2 v[U];
-    double2 sh[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      sh[u] = f0 + u < jb.y ? shifts[jb.z + f0 + u] : make_double2(NAN, NAN);
-      v[u] = sh[u].x == sh[u].x ? spectra[(size_t)(jb.x + f0 + u) * spec_stride + e]
-                                : make_float2(0.f, 0.f);
-    }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const double2 s = sh[u];
-      if (s.x != s.x) continue;
-      double w = (s.x * kx + s.y * yy) * inv_n;
-      w -= floor(w);
-      float sn, cs;
-      sincospif(2.0f * (float)w, &sn, &cs);
-      acc = cadd(acc, cmul(v[u], make_float2(cs, sn)));
-    }
-  }
+  rotate_all(spectra + (size_t)jb.x * spec_stride, spec_stride, shifts + jb.z, jb.y, e, kx, yy,
+             1.0 / n, [&](int, float2 t, float) { acc = cadd(acc, t); });
   spectra[(size_t)jb.w * spec_stride + e] = acc;
 }
 
@@ -307,110 +323,187 @@ hipError_t launch_fsc_sums(const float2* a, const float2* b, int n, int padded, 
 // 2 pi (s_fx kx + s_fy ky')/n, w = exp(-B|k|^2/(2n^2)) * a_kx (a = 1 at DC and
 // Nyquist columns, 2 otherwise: the half-plane counts both halves).
 // dJ/ds_fx = -2 sum_k w (2 pi kx/n) Im(conj(S) F_f e^{i phi_f}); same for y.
-// Work item (chunk c, frame f): frame f < F accumulates its two gradient
-// components over the chunk's elements, f == F accumulates J.  Items of one
-// chunk are consecutive on one XCD, so the chunk of S is reused from L2.
-__global__ __launch_bounds__(256) void k_sharp_partial(const float2* __restrict__ spectra,
-                                                       size_t spec_stride, int nframes, int n,
-                                                       const double2* __restrict__ shifts,
-                                                       const float2* __restrict__ S,
-                                                       const float* __restrict__ wk,
-                                                       int nchunks, int jonly,
-                                                       double2* __restrict__ part) {
-  __shared__ double rx[256], ry[256];
-  const int L = xcd_remap(blockIdx.x, gridDim.x);
-  const int c = jonly ? L : L / (nframes + 1), f = jonly ? nframes : L % (nframes + 1);
-  const int H = n / 2 + 1;
-  const size_t total = (size_t)H * n;
-  const size_t e0 = total * c / nchunks, e1 = total * (c + 1) / nchunks;
-  double gx = 0, gy = 0;
-  const double2 s = f < nframes ? shifts[f] : make_double2(0.0, 0.0);
-  const bool skip = f < nframes && s.x != s.x;
-  const float2* F = spectra + (size_t)(f < nframes ? f : 0) * spec_stride;
+//
+// The phase factors bound it: sincospif and the FP64 phase are 40 of about 60
+// instructions per element and frame, so each is formed once.  Per tile of NT
+// elements a thread rotates its element of every frame, in frame order as
+// k_shift_sum, keeps the rotated values in LDS and has S at the end; then a
+// thread takes the frames (f, f + FH) over part of the tile's elements, so
+// that an element's S, weight and indexes are read once for two frames and the
+// per-frame sums need no reduction until the end.  Frames are read once.
+// LDS entry (f, e) lies at f NT + (e + f) mod NT: both phases without bank
+// conflicts.
+// 2048, 24 frames: 132 us for sum, J and gradient with the closing sum; the
+// sum (84 us), a second pass over frames and sum (125) and a closing sum in
+// one wave (77) before.
+// SUM = false: S was formed before and is read; the frames are split over
+// blockIdx.y (more frames than the LDS holds for a useful number of waves).
+template <int NT, bool SUM>
+__global__ __launch_bounds__(NT) void k_sharp(const float2* __restrict__ spectra, size_t spec_stride,
+                                              int nframes, int FB, int n,
+                                              const double2* __restrict__ shifts,
+                                              float2* __restrict__ S, const float* __restrict__ wk,
+                                              double2* __restrict__ part) {
+  extern __shared__ float4 sharp_lds[];
+  float4* rec = sharp_lds;  // [NT] S, weight, kx | ky' << 16
+  float2* G = reinterpret_cast<float2*>(sharp_lds + NT);  // [FB][NT]
+  const int H = n / 2 + 1, t = threadIdx.x;
+  const long long total = (long long)H * n;
+  const int c = blockIdx.x, nchunks = gridDim.x;
+  const int e0 = (int)(total * c / nchunks), e1 = (int)(total * (c + 1) / nchunks);
+  const int fb = blockIdx.y * FB, nf = min(FB, nframes - fb);
   const double inv_n = 1.0 / n;
-  if (!skip) {
-    // U elements per round, all loads issued first (at valid addresses; the
-    // elements past the chunk get weight 0); (kx, ky) advance by the stride
-    // instead of being divided out of the element index.
-    constexpr int U = 4;
-    const int ie1 = (int)e1;
-    int e = (int)e0 + threadIdx.x;
-    int kx = e / n, ky = e - kx * n;
-    const int kadv = 256 / n, yadv = 256 % n;  // (kx, ky) step of e += 256
-    for (; e < ie1; e += 256 * U) {
-      float2 sv[U], fv[U];
-      float w[U];
-      int kxs[U], yys[U];
-      int ee = e;
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int ec = ee < ie1 ? ee : ie1 - 1;
-        sv[u] = S[ec];
-        fv[u] = F[ec];
-        w[u] = wk[kx] * wk[H + ky] * (ee < ie1 ? 1.f : 0.f);
-        kxs[u] = kx;
-        yys[u] = ky < n / 2 ? ky : ky - n;
-        ee += 256;
-        ky += yadv;
-        kx += kadv;
-        const bool wrap = ky >= n;
-        ky = wrap ? ky - n : ky;
-        kx = wrap ? kx + 1 : kx;
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        if (f == nframes) {
-          gx += (double)w[u] * ((double)sv[u].x * sv[u].x + (double)sv[u].y * sv[u].y);
-        } else {
-          double uu = (s.x * kxs[u] + s.y * yys[u]) * inv_n;
-          uu -= floor(uu);
-          float sn, cs;
-          sincospif(2.0f * (float)uu, &sn, &cs);
-          const float2 g = cmul(fv[u], make_float2(cs, sn));
-          const double im = (double)sv[u].x * g.y - (double)sv[u].y * g.x;  // Im(conj(S) G)
-          const double t = -2.0 * w[u] * im * (2.0 * M_PI * inv_n);
-          gx += t * kxs[u];
-          gy += t * yys[u];
-        }
-      }
+  const int FH = (nf + 1) / 2, P = NT / FH;
+  const int fa = t % FH, fz = fa + FH < nf ? fa + FH : fa, ep = t / FH;
+  double J = 0, ax = 0, ay = 0, zx = 0, zy = 0;
+  for (int et = e0; et < e1; et += NT) {
+    const int e = min(et + t, e1 - 1);
+    const int kx = e / n, ky = e - kx * n;
+    const int yy = ky < n / 2 ? ky : ky - n;
+    const float w = wk[kx] * wk[H + ky] * (et + t < e1 ? 1.f : 0.f);
+    float2 acc = make_float2(0.f, 0.f);
+    rotate_all(spectra + (size_t)fb * spec_stride, spec_stride, shifts + fb, nf, e, kx, yy, inv_n,
+               [&](int f, float2 g, float y2) {
+                 // sum and gradient round the product as their former passes did
+                 acc = cadd(acc, g);
+                 G[f * NT + (t + f < NT ? t + f : t + f - NT)] = make_float2(g.x, y2);
+               });
+    if (SUM) {
+      if (et + t < e1) S[e] = acc;
+    } else {
+      acc = S[e];
     }
-  }
-  rx[threadIdx.x] = gx;
-  ry[threadIdx.x] = gy;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) {
-      rx[threadIdx.x] += rx[threadIdx.x + o];
-      ry[threadIdx.x] += ry[threadIdx.x + o];
+    rec[t] = make_float4(acc.x, acc.y, w, __int_as_float(kx | yy * 65536));
+    J += (double)w * ((double)acc.x * acc.x + (double)acc.y * acc.y);
+    __syncthreads();
+    if (ep < P) {
+#pragma unroll 4
+      for (int x = ep; x < NT; x += P) {
+        const float4 r = rec[x];
+        const int k = __float_as_int(r.w);
+        const double dkx = k & 0xffff, dyy = k >> 16, sx = r.x, sy = r.y, dw = r.z;
+        const int ra = x + fa < NT ? x + fa : x + fa - NT, rz = x + fz < NT ? x + fz : x + fz - NT;
+        const float2 ga = G[fa * NT + ra], gz = G[fz * NT + rz];
+        const double ta = dw * (sx * ga.y - sy * ga.x);  // w Im(conj(S) G)
+        const double tz = dw * (sx * gz.y - sy * gz.x);
+        ax += ta * dkx;
+        ay += ta * dyy;
+        zx += tz * dkx;
+        zy += tz * dyy;
+      }
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) part[(size_t)c * (nframes + 1) + f] = make_double2(rx[0], ry[0]);
+  double2* red = reinterpret_cast<double2*>(G);  // [P][nf], at most 2 NT
+  double* rj = reinterpret_cast<double*>(rec);
+  if (ep < P) {
+    if (fa + FH < nf) red[ep * nf + fa + FH] = make_double2(zx, zy);
+    red[ep * nf + fa] = make_double2(ax, ay);
+  }
+  rj[t] = J;
+  __syncthreads();
+  const double m = -2.0 * (2.0 * M_PI * inv_n);
+  double2* out = part + (size_t)c * (nframes + 1);
+  for (int f = t; f < nf; f += NT) {
+    double x = 0, y = 0;
+    for (int q = 0; q < P; q++) {
+      const double2 v = red[q * nf + f];
+      x += v.x;
+      y += v.y;
+    }
+    const double sx = shifts[fb + f].x;
+    out[fb + f] = sx == sx ? make_double2(m * x, m * y) : make_double2(0.0, 0.0);
+  }
+  if (blockIdx.y == 0 && t < 64) {
+    double x = 0;
+    for (int q = t; q < NT; q += 64) x += rj[q];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+    if (t == 0) out[nframes] = make_double2(x, 0.0);
+  }
 }
 
-// Sums the chunk partials in a fixed order: out[f] = (gx, gy), out[F] = (J, 0).
-__global__ void k_sharp_final(const double2* __restrict__ part, int nchunks, int nframes,
-                              double2* __restrict__ out) {
-  const int f = blockIdx.x * blockDim.x + threadIdx.x;
-  if (f > nframes) return;
+// Sums the chunk partials in a fixed order, one workgroup per output:
+// out[f] = (gx, gy), out[F] = (J, 0).
+__global__ __launch_bounds__(256) void k_sharp_final(const double2* __restrict__ part, int nchunks,
+                                                     int nframes, double2* __restrict__ out) {
+  __shared__ double2 red[4];
+  const int f = blockIdx.x, t = threadIdx.x;
   double x = 0, y = 0;
-  for (int c = 0; c < nchunks; c++) {
+  for (int c = t; c < nchunks; c += 256) {
     const double2 v = part[(size_t)c * (nframes + 1) + f];
     x += v.x;
     y += v.y;
   }
-  out[f] = make_double2(x, y);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    x += __shfl_xor(x, o);
+    y += __shfl_xor(y, o);
+  }
+  if ((t & 63) == 0) red[t >> 6] = make_double2(x, y);
+  __syncthreads();
+  if (t == 0)
+    out[f] = make_double2(red[0].x + red[1].x + red[2].x + red[3].x,
+                          red[0].y + red[1].y + red[2].y + red[3].y);
+}
+
+// Tiles: as many threads as leave the LDS room for two workgroups per CU, the
+// grid as many workgroups as the CUs then hold (at most four each) and no
+// shorter chunks than a tile.  The rotated values of all frames of a tile limit
+// the waves per CU (12 at 24 frames, 4 at 64), so up to 64 frames the sum is
+// formed in the same pass (2048: 40 frames 285 us, 64 frames 599) and above by
+// a pass of its own, then 24 frames at a time (64: 630, 80: 755).  The two
+// passes that this replaces took 448, 668 and 859.
+struct SharpPlan {
+  bool fused;
+  int nb, FB, NT, lds, nchunks;
+};
+static SharpPlan sharp_plan(int nframes, int n) {
+  SharpPlan p;
+  p.fused = nframes <= 64;
+  p.nb = p.fused ? 1 : (nframes + 23) / 24;
+  p.FB = (nframes + p.nb - 1) / p.nb;
+  p.NT = p.FB <= 38 ? 256 : p.FB <= 51 ? 192 : 128;
+  p.lds = p.NT * (std::max(p.FB, 4) * 8 + 16);  // the closing sums take 32 bytes per thread
+  const long long tiles = ((long long)(n / 2 + 1) * n + p.NT - 1) / p.NT;
+  p.nchunks = (int)std::min<long long>(tiles, 256 * std::min(4, 160 * 1024 / p.lds));
+  return p;
+}
+size_t sharp_part_elems(int nframes, int n) {
+  return (size_t)sharp_plan(nframes, n).nchunks * (nframes + 1);
+}
+
+template <int NT, bool SUM>
+static hipError_t sharp_launch(const SharpPlan& p, const float2* spectra, size_t spec_stride,
+                               int nframes, int n, const double2* shifts, float2* S,
+                               const float* wk, double2* part, hipStream_t st) {
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_sharp<NT, SUM>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, p.lds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((k_sharp<NT, SUM>), dim3(p.nchunks, p.nb), dim3(NT), p.lds, st, spectra,
+                     spec_stride, nframes, p.FB, n, shifts, S, wk, part);
+  return hipGetLastError();
 }
 
 hipError_t launch_sharpness(const float2* spectra, size_t spec_stride, int nframes, int n,
-                            const double2* shifts, const float2* S, const float* wk,
-                            double2* part, int nchunks, double2* out, int jonly,
-                            hipStream_t st) {
-  const int nb = nchunks * (jonly ? 1 : nframes + 1);
-  hipLaunchKernelGGL(k_sharp_partial, dim3(nb), dim3(256), 0, st, spectra, spec_stride, nframes,
-                     n, shifts, S, wk, nchunks, jonly, part);
-  hipLaunchKernelGGL(k_sharp_final, dim3((nframes + 1 + 63) / 64), dim3(64), 0, st, part,
-                     nchunks, nframes, out);
+                            const double2* shifts, float2* S, const float* wk, double2* part,
+                            double2* out, hipStream_t st) {
+  const SharpPlan p = sharp_plan(nframes, n);
+  hipError_t e = hipSuccess;
+  if (!p.fused) {
+    e = launch_shift_sum(spectra, spec_stride, nframes, n, shifts, S, nullptr, -1, st);
+    if (e != hipSuccess) return e;
+    e = sharp_launch<256, false>(p, spectra, spec_stride, nframes, n, shifts, S, wk, part, st);
+  } else if (p.NT == 256) {
+    e = sharp_launch<256, true>(p, spectra, spec_stride, nframes, n, shifts, S, wk, part, st);
+  } else if (p.NT == 192) {
+    e = sharp_launch<192, true>(p, spectra, spec_stride, nframes, n, shifts, S, wk, part, st);
+  } else {
+    e = sharp_launch<128, true>(p, spectra, spec_stride, nframes, n, shifts, S, wk, part, st);
+  }
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_sharp_final, dim3(nframes + 1), dim3(256), 0, st, part, p.nchunks, nframes,
+                     out);
   return hipGetLastError();
 }
 
