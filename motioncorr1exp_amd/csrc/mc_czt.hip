@@ -1,7 +1,7 @@
-// mc_czt.hip -- transforms of any even length (the reference's default
-// square crop, e.g. 3710 = 2*5*7*53 for a 3838 x 3710 K2 frame, or a
-// non-integer -bin): Bluestein's chirp-z algorithm on the power-of-two LDS
-// Stockham engine of mc_device.h.  The reference plans cuFFT at any size
+// mc_czt.hip -- transforms of the lengths that mc_mixed.hip has no factors for
+// (a prime above 127): Bluestein's chirp-z algorithm on the power-of-two LDS
+// Stockham engine of mc_device.h.  Stage 1 and the sum image at any even size
+// are dispatched here.  The reference plans cuFFT at any size
 // (cufunc.cu:202-215, called for nsamUnbin and nsam, DFAlign.cu:596,838).
 //
 // A length-L DFT with sign S, X_k = sum_m x_m e^{S 2 pi i m k/L}, is
@@ -67,7 +67,7 @@ int czt_len(int need) {
   return M;
 }
 
-static float2* upload(const std::vector<float2>& h) {
+float2* upload_table(const std::vector<float2>& h) {
   float2* d = nullptr;
   if (hipMalloc(&d, sizeof(float2) * h.size()) != hipSuccess) return nullptr;
   if (hipMemcpy(d, h.data(), sizeof(float2) * h.size(), hipMemcpyHostToDevice) != hipSuccess) {
@@ -109,8 +109,8 @@ static const BsTab* bs_tables(int L, int S) {
   std::vector<float2> F(M);
   for (int k = 0; k < M; k++) F[k] = f2(h[k] / (double)M);
   BsTab t;
-  t.chirp = upload(c);
-  t.filt = upload(F);
+  t.chirp = upload_table(c);
+  t.filt = upload_table(F);
   t.M = M;
   if (!t.chirp || !t.filt) return nullptr;
   return &(cache[key] = t);
@@ -146,9 +146,9 @@ static const CztTab* czt_tables(int n, int box) {
   std::vector<float2> F(M);
   for (int k = 0; k < M; k++) F[k] = f2(g[k] / (double)M);
   CztTab t;
-  t.pre = upload(pre);
-  t.filt = upload(F);
-  t.post = upload(post);
+  t.pre = upload_table(pre);
+  t.filt = upload_table(F);
+  t.post = upload_table(post);
   t.M = M;
   if (!t.pre || !t.filt || !t.post) return nullptr;
   return &(cache[key] = t);
@@ -156,7 +156,7 @@ static const CztTab* czt_tables(int n, int box) {
 
 // Twiddles of the two-level column transform n = Q P:
 // tw[k2 Q + a] = e^{-2 pi i ((a k2) mod n)/n}, k2 < P, a < Q.
-static const float2* qp_twiddles(int Q, int P) {
+const float2* qp_twiddles(int Q, int P) {
   static std::mutex mu;
   static std::map<std::tuple<int, int, int>, const float2*> cache;
   int dev = 0;
@@ -172,7 +172,7 @@ static const float2* qp_twiddles(int Q, int P) {
       const double t = -2.0 * M_PI * (double)((a * k2) % n) / (double)n;
       h[(size_t)k2 * Q + a] = make_float2((float)std::cos(t), (float)std::sin(t));
     }
-  const float2* d = upload(h);
+  const float2* d = upload_table(h);
   if (d) cache[key] = d;
   return d;
 }
@@ -233,19 +233,6 @@ MC_DEV void bluestein_rw(float2* buf, const FftTw<M, NT, -1, 1>& ftw,
   }
   __syncthreads();
   fft_lds_rw<M, NT, 1, 1, M, PB>(buf, ftw);
-}
-
-// Pixel x of canvas row y of a frame: decoded, corrected, zero outside the
-// data region.
-template <int DT>
-MC_DEV float row_px(const R2CGeom& g, const char* fbase, bool corr, int x, int y) {
-  typedef typename Elem<DT>::T T;
-  if (x >= g.w) return 0.f;
-  const int2 sp = stretch_src(g, g.offx + x, g.offy + y);
-  const float v = (float)reinterpret_cast<const T*>(fbase + (size_t)sp.y * g.row_pitch)[sp.x];
-  if (!corr) return v;
-  const size_t idx = (size_t)sp.y * g.nx + sp.x;
-  return correct(g, v, g.dark ? g.dark[idx] : 0.f, g.gain ? g.gain[idx] : 1.f);
 }
 
 // Stage-1 row pass of one canvas row y < h of frame f (any even nu): the
@@ -435,173 +422,6 @@ __global__ __launch_bounds__(NT, czt_waves<NT>()) void k_c2c_cols_czt_p(
   }
 }
 
-// Stage-1 row pass at nu = 2 Q P (packed length N = Q P, Q with a Stockham
-// plan, P odd), for the rows of the 3710 and 4092 crops (N = 1855 = 35 x 53,
-// 2046 = 66 x 31): the
-// packing, N-point DFT and unpack of row_czt, with the DFT in two levels as
-// in k_c2c_cols_qp below.  Lane a < Q reads the packed values z[a + Q b]
-// (pixels 2 (a + Q b) and 2 (a + Q b) + 1) straight from the frame and runs
-// the P-point direct DFT into LDS row k2, element a; after the twiddles and
-// the P Q-point FFTs, Z[k] is row k % P, element k / P (and the unpack puts
-// X[N] in the spare element Q of row 0).  The LDS rows are unpadded (odd
-// stride; at 3710, 16 KB per row fits 10 workgroups per CU against 9 with
-// the padded layout, 0.5 ms less per 40-frame movie for the two passes).
-// One row per workgroup of Q lanes rounded up to whole waves;
-// the rows are numbered XCD-major, so the four rows that share a line of
-// the row-pass scratch are written through one L2.
-template <int Q, int P, int R, int NT, int DT>
-__global__ __launch_bounds__(NT) void k_r2c_rows_qp(R2CGeom g, int f0, int nframes, int nkx,
-                                                    float2* __restrict__ rt, size_t rt_fstride,
-                                                    float* __restrict__ rowsum,
-                                                    const float2* __restrict__ gtw,
-                                                    const float2* __restrict__ twqp,
-                                                    const float2* __restrict__ twnu) {
-  constexpr int N = Q * P;
-  constexpr int NH = N / 2 + 1;
-  constexpr int PB = 0;  // unpadded rows (odd stride): more workgroups per CU
-  constexpr int TS = lds_len<PB>(Q + 1) | 1;
-  constexpr int RS = P * TS;  // one row's LDS block
-  static_assert(NT >= R * Q && NT % 64 == 0, "one lane per P-point DFT");
-  __shared__ float2 buf[R * RS];
-  __shared__ float2 twm[Q];
-  const int nitems = g.h * nframes;
-  const int L0 = R * ((int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8));
-  if (L0 >= nitems) return;
-  const int nr = nitems - L0 < R ? nitems - L0 : R;  // rows of this workgroup
-  for (int i = threadIdx.x; i < Q; i += NT) twm[i] = gtw[i * P];  // e^{+2 pi i i/Q}
-  const bool corr = g.dark || g.gain || g.xs < 1.f || g.ys < 1.f;
-  {
-    const int r = threadIdx.x / Q, a = threadIdx.x - r * Q;
-    if (r < nr) {
-      const int L = L0 + r, y = L % g.h, f = L / g.h;
-      const char* fbase = g.src + (size_t)(f0 + f) * g.frame_pitch;
-      float2 x[P];
-      if (!corr && g.vec) {
-        // the pixel pairs as single aligned loads (the row is all data)
-        typedef typename Elem<DT>::T T;
-        struct alignas(2 * sizeof(T)) Pair {
-          T a, b;
-        };
-        const Pair* row = reinterpret_cast<const Pair*>(
-            reinterpret_cast<const T*>(fbase + (size_t)(y + g.offy) * g.row_pitch) + g.offx);
-#pragma unroll
-        for (int b = 0; b < P; b++) {
-          const Pair v = row[a + Q * b];
-          x[b] = make_float2((float)v.a, (float)v.b);
-        }
-      } else {
-#pragma unroll
-        for (int b = 0; b < P; b++) {
-          const int m = a + Q * b;
-          x[b] = make_float2(row_px<DT>(g, fbase, corr, 2 * m, y),
-                             row_px<DT>(g, fbase, corr, 2 * m + 1, y));
-        }
-      }
-      float2* rb = buf + r * RS;
-      odd_dft<P, -1>(x, [&](int k, float2 v) { rb[k * TS + lix<PB>(a)] = v; });
-    }
-  }
-  __syncthreads();
-  // twiddles e^{-2 pi i a k2/N} (row k2 = 0 has none)
-  for (int e = threadIdx.x; e < R * (N - Q); e += NT) {
-    const int r = e / (N - Q), j = e - r * (N - Q) + Q;
-    const int k2 = j / Q, i = j - k2 * Q;
-    float2* p = buf + r * RS + k2 * TS + lix<PB>(i);
-    *p = cmul(*p, twqp[j]);
-  }
-  __syncthreads();
-  fft_lds_t<Q, NT, -1, R * P, TS, TwTable, PB>(buf, TwTable{twm, Q}, Q);
-  auto at = [&](int k) -> int { return (k % P) * TS + lix<PB>(k / P); };
-  // unpack, one thread per bin pair (k, N-k): X[k] = E[k] + e^{-2 pi i k/2N} O[k]
-  for (int t = threadIdx.x; t < R * NH; t += NT) {
-    const int r = t / NH, k = t - r * NH;
-    float2* rb = buf + r * RS;
-    const int lk = at(k), lm = at(k ? N - k : 0);
-    const float2 zk = rb[lk], zm = rb[lm];
-    {
-      const float2 zc = cconj(zm);
-      const float2 E = cscale(cadd(zk, zc), 0.5f);
-      const float2 D = csub(zk, zc);
-      const float2 O = make_float2(0.5f * D.y, -0.5f * D.x);
-      if (k == 0) rb[at(N)] = csub(E, O);
-      rb[lk] = cadd(E, cmul(cconj(twnu[k]), O));
-    }
-    if (k > 0 && k < N - k) {
-      const float2 zc = cconj(zk);
-      const float2 E = cscale(cadd(zm, zc), 0.5f);
-      const float2 D = csub(zm, zc);
-      const float2 O = make_float2(0.5f * D.y, -0.5f * D.x);
-      rb[lm] = cadd(E, cmul(cconj(twnu[N - k]), O));
-    }
-  }
-  __syncthreads();
-  for (int t = threadIdx.x; t < nr * nkx; t += NT) {
-    const int r = t / nkx, k = t - r * nkx;
-    const int L = L0 + r, y = L % g.h, f = L / g.h;
-    const float2 X = buf[r * RS + at(k)];
-    rt[(size_t)f * rt_fstride + ((size_t)(k >> 2) * (2 * N) + y) * 4 + (k & 3)] = X;
-    if (k == 0 && rowsum) rowsum[(size_t)f * (2 * N) + y] = X.x;
-  }
-}
-
-// Stage-1 column pass at N = Q P without fill rows (Q with a Stockham plan,
-// P odd), for the 3710 = 70 x 53 crop of a 3838 x 3710 frame and the 4092 =
-// 132 x 31 crop of a K3 frame:
-//   X[k2 + P k1] = sum_a e^{-2 pi i a k1/Q} (e^{-2 pi i a k2/N}
-//                  sum_b x[a + Q b] e^{-2 pi i b k2/P}).
-// Lane a < Q loads x[a + Q b] (b < P) and runs the direct P-point DFT
-// (odd_dft) in registers into LDS row k2, element a; a second pass applies
-// the twiddles; then P Q-point FFTs run in LDS, and row k2 element k1 is
-// X[k2 + P k1]; the rows of the Fourier crop to n are stored.  At 3710
-// about 0.4x the arithmetic of the 8192-point chirp-z convolution, in a 31
-// KB LDS buffer (unpadded rows of odd stride 71, 5 workgroups per CU).  One
-// column per workgroup (a
-// persistent loop would hoist the LDS addresses of every FFT stage out of
-// the loop and hold them in registers); the columns are numbered XCD-major,
-// so the four columns of one row-pass line group share an L2.
-template <int Q, int P, int NT, int W>
-__global__ __launch_bounds__(NT, W) void k_c2c_cols_qp(const float2* __restrict__ rt,
-                                                       size_t rt_fstride, int nkx, int nitems,
-                                                       int n, float2* __restrict__ spec,
-                                                       size_t spec_stride,
-                                                       const float2* __restrict__ gtw,
-                                                       const float2* __restrict__ twqp) {
-  constexpr int N = Q * P;
-  constexpr int PB = 0;  // as in k_r2c_rows_qp
-  constexpr int TS = lds_len<PB>(Q) | 1;
-  static_assert(NT >= Q && NT % 64 == 0, "one lane per P-point DFT");
-  __shared__ float2 buf[P * TS];
-  __shared__ float2 twm[Q];
-  const int L = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);
-  if (L >= nitems) return;
-  for (int i = threadIdx.x; i < Q; i += NT) twm[i] = gtw[i * P];  // e^{+2 pi i i/Q}
-  const int a = threadIdx.x;
-  const int kx = L % nkx, f = L / nkx;
-  const float2* src = rt + (size_t)f * rt_fstride + (size_t)(kx >> 2) * N * 4 + (kx & 3);
-  if (a < Q) {
-    const auto q = buf_rsrc(src, N * 32);
-    float2 x[P];
-#pragma unroll
-    for (int b = 0; b < P; b++) x[b] = buf_ld2(q, 32 * a, 32 * Q * b);
-    odd_dft<P, -1>(x, [&](int k, float2 v) { buf[k * TS + lix<PB>(a)] = v; });
-  }
-  __syncthreads();
-  // twiddles e^{-2 pi i a k2/N} (row k2 = 0 has none)
-  for (int e = Q + threadIdx.x; e < N; e += NT) {
-    const int k2 = e / Q, i = e - k2 * Q;
-    float2* p = buf + k2 * TS + lix<PB>(i);
-    *p = cmul(*p, twqp[e]);
-  }
-  __syncthreads();
-  fft_lds_t<Q, NT, -1, P, TS, TwTable, PB>(buf, TwTable{twm, Q}, Q);
-  // the rows of the Fourier crop to n (n = N unbinned)
-  float2* dst = spec + (size_t)f * spec_stride + (size_t)kx * n;
-  for (int o = threadIdx.x; o < n; o += NT) {
-    const int si = o < n / 2 ? o : N - n + o;
-    dst[o] = buf[(si % P) * TS + lix<PB>(si / P)];
-  }
-}
-
 // Pair-stage column pass (any even n): per (pair, kx) item, the weighted
 // cross power X[ky] = F_a[kx][ky] conj(F_b[kx][ky]) wx[kx] wy[ky], then the
 // pruned chirp-z inverse to the box rows, T[p][kx][u].  Persistent: each
@@ -673,45 +493,6 @@ __global__ __launch_bounds__(NT, czt_waves<NT>()) void k_cols_inv_czt(const floa
   bluestein<M, NT, 1>(buf, TwSplit{tlo, thi, LB, M}, chirpv, filt, n);
   float2* dst = tmp + (size_t)(kx >> 2) * n * 4 + (kx & 3);
   for (int i = threadIdx.x; i < n; i += NT) dst[(size_t)i * 4] = buf[lix<PB>(i)];
-}
-
-// Sum-image C2R, column pass at N = Q P (the 3710 and 4092 sizes): the
-// inverse of k_c2c_cols_qp, X[k2 + P k1] = sum_a e^{2 pi i a k1/Q}
-// (e^{2 pi i a k2/N} sum_b x[a + Q b] e^{2 pi i b k2/P}), on column kx of the
-// spectrum, stored like k_cols_inv_czt (tmp[kx/4][y][kx%4]).
-template <int Q, int P, int NT>
-__global__ __launch_bounds__(NT, 2) void k_cols_inv_qp(const float2* __restrict__ spec, int nkx,
-                                                       float2* __restrict__ tmp,
-                                                       const float2* __restrict__ gtw,
-                                                       const float2* __restrict__ twqp) {
-  constexpr int N = Q * P;
-  constexpr int PB = 0;
-  constexpr int TS = lds_len<PB>(Q) | 1;
-  static_assert(NT >= Q && NT % 64 == 0, "one lane per P-point DFT");
-  __shared__ float2 buf[P * TS];
-  __shared__ float2 twm[Q];
-  const int kx = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);
-  if (kx >= nkx) return;
-  for (int i = threadIdx.x; i < Q; i += NT) twm[i] = gtw[i * P];  // e^{+2 pi i i/Q}
-  const int a = threadIdx.x;
-  if (a < Q) {
-    const auto q = buf_rsrc(spec + (size_t)kx * N, N * 8);
-    float2 x[P];
-#pragma unroll
-    for (int b = 0; b < P; b++) x[b] = buf_ld2(q, 8 * a, 8 * Q * b);
-    odd_dft<P, 1>(x, [&](int k, float2 v) { buf[k * TS + lix<PB>(a)] = v; });
-  }
-  __syncthreads();
-  // twiddles e^{+2 pi i a k2/N} (the table holds e^{-2 pi i a k2/N})
-  for (int e = Q + threadIdx.x; e < N; e += NT) {
-    const int k2 = e / Q, i = e - k2 * Q;
-    float2* p = buf + k2 * TS + lix<PB>(i);
-    *p = cmulc(*p, twqp[e]);
-  }
-  __syncthreads();
-  fft_lds_t<Q, NT, 1, P, TS, TwTable, PB>(buf, TwTable{twm, Q}, Q);
-  float2* dst = tmp + (size_t)(kx >> 2) * N * 4 + (kx & 3);
-  for (int o = threadIdx.x; o < N; o += NT) dst[(size_t)o * 4] = buf[(o % P) * TS + lix<PB>(o / P)];
 }
 
 // Sum-image C2R, row pass (any even n): the n/2+1 bins of row y with the
@@ -817,41 +598,6 @@ static hipError_t cols_czt_t(const R2CGeom& g, int nframes, int nkx, const float
   return hipGetLastError();
 }
 
-template <int Q, int P>
-static hipError_t rows_qp_t(const R2CGeom& g, int f0, int nframes, int nkx, float2* rt,
-                            size_t rt_fstride, float* rs, const float2* twnu, hipStream_t st) {
-  constexpr int R = 1, NT = (Q + 63) / 64 * 64;
-  const float2* gtw = twiddles(Q * P);
-  const float2* twqp = qp_twiddles(Q, P);
-  if (!gtw || !twqp) return hipErrorOutOfMemory;
-  // pixel pairs load as one element when the pairs are aligned
-  const size_t es = g.dtype == DT_FLOAT32 ? 4 : (g.dtype == DT_INT16 || g.dtype == DT_UINT16) ? 2 : 1;
-  R2CGeom gq = g;
-  gq.vec = ((uintptr_t)g.src % (2 * es) == 0 && g.row_pitch % (2 * es) == 0 &&
-            g.frame_pitch % (2 * es) == 0 && (g.offx & 1) == 0) ? 1 : 0;
-  const int grid = ((g.h * nframes + R - 1) / R + 7) / 8 * 8;
-  switch (g.dtype) {
-#define MC_RQ(D) case D: hipLaunchKernelGGL((k_r2c_rows_qp<Q, P, R, NT, D>), dim3(grid), dim3(NT), 0, st, gq, f0, nframes, nkx, rt, rt_fstride, rs, gtw, twqp, twnu); break;
-    MC_RQ(DT_INT8) MC_RQ(DT_UINT8) MC_RQ(DT_INT16) MC_RQ(DT_UINT16) MC_RQ(DT_FLOAT32)
-#undef MC_RQ
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-
-template <int Q, int P>
-static hipError_t cols_qp_t(int nframes, int nkx, const float2* rt, size_t rt_fstride, int n,
-                            float2* spectra, size_t spec_stride, hipStream_t st) {
-  constexpr int NT = (Q + 63) / 64 * 64, W = 2;
-  const float2* gtw = twiddles(Q * P);
-  const float2* twqp = qp_twiddles(Q, P);
-  if (!gtw || !twqp) return hipErrorOutOfMemory;
-  const int grid = (nkx * nframes + 7) / 8 * 8;
-  hipLaunchKernelGGL((k_c2c_cols_qp<Q, P, NT, W>), dim3(grid), dim3(NT), 0, st, rt, rt_fstride, nkx,
-                     nkx * nframes, n, spectra, spec_stride, gtw, twqp);
-  return hipGetLastError();
-}
-
 hipError_t launch_frames_to_spectra_czt(const R2CGeom& g, int f0, int nframes, float2* spectra,
                                         size_t spec_stride, float2* rt, float* rowsum,
                                         float* fill, const float2* padP, hipStream_t st) {
@@ -859,25 +605,15 @@ hipError_t launch_frames_to_spectra_czt(const R2CGeom& g, int f0, int nframes, f
   const int nkx = g.n / 2 + 1;
   const size_t rt_fstride = rt_frame_elems(g.n, g.nu);
   float* rs = g.pad_mode ? rowsum : nullptr;
-  R2CGeom gv = g;
-  gv.vec = 0;
-  const BsTab* tr = bs_tables(g.nu / 2, -1);
-  const BsTab* tc = bs_tables(g.nu, -1);
-  const float2* twnu = twiddles(g.nu);
-  if (!tr || !tc || !twnu) return hipErrorOutOfMemory;
   hipError_t e = hipErrorInvalidValue;
-  // square canvases of 3710 (K2 crop) and 4092 (K3 crop) without fill:
-  // two-level transforms, 35 x 53 (66 x 31) for the packed rows and 70 x 53
-  // (132 x 31) for the columns, any binning
-  const int qp = (!g.pad_mode && g.h == g.nu && g.w == g.nu && (g.nu == 3710 || g.nu == 4092))
-                     ? g.nu : 0;
-  if (qp == 3710) {
-    e = rows_qp_t<35, 53>(gv, f0, nframes, nkx, rt, rt_fstride, rs, twnu, st);
-  } else if (qp == 4092) {
-    e = rows_qp_t<66, 31>(gv, f0, nframes, nkx, rt, rt_fstride, rs, twnu, st);
+  if (mix_size_ok(g.nu / 2)) {
+    e = launch_rows_mix(g, f0, nframes, nkx, rt, rt_fstride, rs, st);
   } else {
+    const BsTab* tr = bs_tables(g.nu / 2, -1);
+    const float2* twnu = twiddles(g.nu);
+    if (!tr || !twnu) return hipErrorOutOfMemory;
     switch (tr->M) {
-#define MC_R(MM) case MM: e = rows_czt_t<MM>(gv, f0, nframes, nkx, rt, rt_fstride, rs, *tr, twnu, st); break;
+#define MC_R(MM) case MM: e = rows_czt_t<MM>(g, f0, nframes, nkx, rt, rt_fstride, rs, *tr, twnu, st); break;
       MC_CZT_SIZES(MC_R)
 #undef MC_R
     }
@@ -889,11 +625,11 @@ hipError_t launch_frames_to_spectra_czt(const R2CGeom& g, int f0, int nframes, f
   }
   e = hipErrorInvalidValue;
   const float* fl = g.pad_mode ? fill : nullptr;
-  if (qp == 3710) {
-    e = cols_qp_t<70, 53>(nframes, nkx, rt, rt_fstride, g.n, spectra, spec_stride, st);
-  } else if (qp == 4092) {
-    e = cols_qp_t<132, 31>(nframes, nkx, rt, rt_fstride, g.n, spectra, spec_stride, st);
+  if (mix_size_ok(g.nu)) {
+    e = launch_cols_mix(g, nframes, nkx, rt, rt_fstride, fl, padP, spectra, spec_stride, st);
   } else {
+    const BsTab* tc = bs_tables(g.nu, -1);
+    if (!tc) return hipErrorOutOfMemory;
     switch (tc->M) {
 #define MC_C(MM) case MM: e = cols_czt_t<MM>(g, nframes, nkx, rt, rt_fstride, fl, padP, spectra, spec_stride, *tc, st); break;
       MC_CZT_SIZES(MC_C)
@@ -954,31 +690,15 @@ static hipError_t c2r_rows_czt_t(const float2* tmp, int n, float scale, float* i
   return hipGetLastError();
 }
 
-template <int Q, int P>
-static hipError_t cols_inv_qp_t(const float2* spec, float2* tmp, hipStream_t st) {
-  constexpr int NT = (Q + 63) / 64 * 64;
-  const float2* gtw = twiddles(Q * P);
-  const float2* twqp = qp_twiddles(Q, P);
-  if (!gtw || !twqp) return hipErrorOutOfMemory;
-  const int nkx = Q * P / 2 + 1;
-  hipLaunchKernelGGL((k_cols_inv_qp<Q, P, NT>), dim3((nkx + 7) / 8 * 8), dim3(NT), 0, st, spec,
-                     nkx, tmp, gtw, twqp);
-  return hipGetLastError();
-}
-
 hipError_t launch_spectrum_to_image_czt(const float2* spec, int n, float scale, float* img,
                                         size_t img_pitch, float2* tmp, hipStream_t st) {
   if (n < 64 || n > 8192 || n % 2) return hipErrorInvalidValue;
-  const BsTab* tc = bs_tables(n, 1);
-  const BsTab* tr = bs_tables(n / 2, 1);
-  const float2* twn = twiddles(n);
-  if (!tc || !tr || !twn) return hipErrorOutOfMemory;
   hipError_t e = hipErrorInvalidValue;
-  if (n == 3710) {
-    e = cols_inv_qp_t<70, 53>(spec, tmp, st);
-  } else if (n == 4092) {
-    e = cols_inv_qp_t<132, 31>(spec, tmp, st);
+  if (mix_size_ok(n)) {
+    e = launch_cols_inv_mix(spec, n, tmp, st);
   } else {
+    const BsTab* tc = bs_tables(n, 1);
+    if (!tc) return hipErrorOutOfMemory;
     switch (tc->M) {
 #define MC_CI(MM) case MM: e = cols_inv_czt_t<MM>(spec, n, tmp, *tc, st); break;
       MC_CZT_SIZES(MC_CI)
@@ -986,6 +706,10 @@ hipError_t launch_spectrum_to_image_czt(const float2* spec, int n, float scale, 
     }
   }
   if (e != hipSuccess) return e;
+  if (mix_size_ok(n / 2)) return launch_c2r_rows_mix(tmp, n, scale, img, img_pitch, st);
+  const BsTab* tr = bs_tables(n / 2, 1);
+  const float2* twn = twiddles(n);
+  if (!tr || !twn) return hipErrorOutOfMemory;
   e = hipErrorInvalidValue;
   switch (tr->M) {
 #define MC_CR(MM) case MM: e = c2r_rows_czt_t<MM>(tmp, n, scale, img, img_pitch, *tr, twn, st); break;

@@ -38,4 +38,17 @@ MC_DEV float correct(const R2CGeom& g, float v, float d, float gn) {
   return v;
 }
 
+// Pixel x of canvas row y of a frame: decoded, corrected, zero outside the
+// data region.
+template <int DT>
+MC_DEV float row_px(const R2CGeom& g, const char* fbase, bool corr, int x, int y) {
+  typedef typename Elem<DT>::T T;
+  if (x >= g.w) return 0.f;
+  const int2 sp = stretch_src(g, g.offx + x, g.offy + y);
+  const float v = (float)reinterpret_cast<const T*>(fbase + (size_t)sp.y * g.row_pitch)[sp.x];
+  if (!corr) return v;
+  const size_t idx = (size_t)sp.y * g.nx + sp.x;
+  return correct(g, v, g.dark ? g.dark[idx] : 0.f, g.gain ? g.gain[idx] : 1.f);
+}
+
 }  // namespace mc

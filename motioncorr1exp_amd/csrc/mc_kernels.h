@@ -1,6 +1,7 @@
 // mc_kernels.h -- host-side launch wrappers of the HIP kernels (internal).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <vector>
 #include <stddef.h>
 #include <stdint.h>
 
@@ -86,6 +87,18 @@ hipError_t launch_frames_to_spectra_czt(const R2CGeom& g, int f0, int nframes, f
                                         float* fill, const float2* padP, hipStream_t st);
 hipError_t launch_spectrum_to_image_czt(const float2* spec, int n, float scale, float* img,
                                         size_t img_pitch, float2* tmp, hipStream_t st);
+// Transforms of N = P Q with both factors in 7..127 (mc_mixed.hip).
+float2* upload_table(const std::vector<float2>& h);  // device copy, nullptr on failure
+const float2* qp_twiddles(int Q, int P);  // e^{-2 pi i a k2/(Q P)} at k2 Q + a, a < Q, k2 < P
+bool mix_size_ok(int N);
+hipError_t launch_rows_mix(const R2CGeom& g, int f0, int nframes, int nkx, float2* rt,
+                             size_t rt_fstride, float* rowsum, hipStream_t st);
+hipError_t launch_cols_mix(const R2CGeom& g, int nframes, int nkx, const float2* rt,
+                             size_t rt_fstride, const float* fill, const float2* padP,
+                             float2* spectra, size_t spec_stride, hipStream_t st);
+hipError_t launch_cols_inv_mix(const float2* spec, int n, float2* tmp, hipStream_t st);
+hipError_t launch_c2r_rows_mix(const float2* tmp, int n, float scale, float* img, size_t pitch,
+                                 hipStream_t st);
 hipError_t launch_pair_cols_czt(const float2* spectra, size_t spec_stride, const int2* pairs,
                                 int npairs, const float* wxy, int n, int box, float2* tbuf,
                                 hipStream_t st);
