@@ -292,9 +292,8 @@ int mc_align_batch(mc_context ctx, const mc_batch_item *items, int count,
  *            1024 to 8192, the radix plan of its FFT (balanced, reversed
  *            order, radix-8 chain) x its LDS index padding (one float2 per
  *            16, or none);
- *   pair stage (FP32 form): row kernel (FP32 MFMA with 4 or 8 waves per
- *            pair, vector ALU); the column pass has one kernel per size,
- *            whose time is reported.
+ *   pair stage (FP32 form): the column and the row pass have one kernel per
+ *            size, whose times are reported.
  * Each candidate runs once untimed and 3 times timed (minimum kept); the
  * context's resident spectra are overwritten, so the stage entry points need
  * mc_load_frames again afterwards.  With
@@ -302,21 +301,18 @@ int mc_align_batch(mc_context ctx, const mc_batch_item *items, int count,
  * ({"arch", "cus", "nu", "n", "dtype", "box", "precision", "r2c", "chunk",
  * "cols", "rows"}); mc_tune_load reads the lines of the same device type
  * back (later lines win).  Without tuning, the defaults are 4x512 (4x256
- * below 4096), 192 MB of row-pass scratch per launch and the streaming FP32
- * MFMA row kernel. */
+ * below 4096) and 192 MB of row-pass scratch per launch. */
 typedef struct {
   int r2c_variant;        /* 1: 4x256, 2: 2x256, 3: 4x512; +8: persistent
                              column pass with register twiddles           */
   int chunk_frames;       /* frames per stage-1 launch                      */
   int pair_cols_variant;  /* 0 (cache files may hold 0 to 3: the codes of former
                              column kernels; all run the same one)        */
-  int pair_rows_variant;  /* 0: FP32 MFMA streaming (box <= 96), 1: vector
-                             ALU, 2: FP32 MFMA through LDS (8 waves),
-                             3: FP32 MFMA through LDS (4 waves)             */
+  int pair_rows_variant;  /* 0, as for the columns                          */
   float ms_stage1[2][4][4]; /* [column pass: per column, persistent]
                                [row shape][chunk 1, 2, 4, 8]; 0 = not run  */
   float ms_pair_cols[4];  /* [0]: the column pass; the others 0             */
-  float ms_pair_rows[4];
+  float ms_pair_rows[4];  /* [0]: the row pass; the others 0                */
   int cols_plan;          /* per-column pass of stage 1: radix plan cols_plan/2
                              (0 balanced, 1 reversed order, 2 radix-8 chain)
                              and LDS padding cols_plan%2 (0 one float2 per 16,

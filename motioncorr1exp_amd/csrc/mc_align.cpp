@@ -92,7 +92,7 @@ struct mc_context_s {
   int device = 0;
   hipStream_t st = nullptr;
   DevBuf spec, rt, rowsum, fill, padP, pairs_d, tbuf, box, boxpart, peaks, shifts, image, tmp, means,
-      sum2img, wk, gpart, gout, jobs, tmax, fsc, disp;
+      sum2img, wk, gpart, gout, jobs, fsc, disp;
   int graph_captures = 0, graph_replays = 0;
   // autotuned launch shapes (mc_autotune / mc_tune_load)
   struct Tune {
@@ -170,7 +170,7 @@ extern "C" int mc_context_destroy(mc_context ctx) {
   DevBuf* bufs[] = {&ctx->spec, &ctx->rt, &ctx->rowsum, &ctx->fill, &ctx->padP,
                     &ctx->pairs_d, &ctx->tbuf, &ctx->box, &ctx->boxpart, &ctx->peaks,
                     &ctx->shifts, &ctx->image, &ctx->tmp, &ctx->means, &ctx->sum2img,
-                    &ctx->wk, &ctx->gpart, &ctx->gout, &ctx->jobs, &ctx->tmax, &ctx->fsc,
+                    &ctx->wk, &ctx->gpart, &ctx->gout, &ctx->jobs, &ctx->fsc,
                     &ctx->disp};
   for (DevBuf* b : bufs) b->release();
   for (hipEvent_t e : ctx->pool) (void)hipEventDestroy(e);
@@ -548,7 +548,6 @@ static int pair_reserve(mc_context_s* c, int np, int n, int box, int precision) 
   const int H = n / 2 + 1;
   HIP_TRY(c->pairs_d.ensure(sizeof(int) * 2 * (size_t)np));
   HIP_TRY(c->tbuf.ensure(sizeof(float2) * (size_t)np * H * box));
-  if (precision == MC_PREC_MFMA_HILO) HIP_TRY(c->tmax.ensure(sizeof(float) * (size_t)np * H));
   HIP_TRY(c->box.ensure(sizeof(float) * (size_t)np * box * box));
   HIP_TRY(c->boxpart.ensure(sizeof(float) * std::max<size_t>(1, mc::pair_rows_part_elems(np, n, box))));
   HIP_TRY(c->peaks.ensure(sizeof(double) * 3 * (size_t)np));
@@ -559,21 +558,19 @@ static int pair_reserve(mc_context_s* c, int np, int n, int box, int precision) 
 // (one movie's region); results stay on the device (peaks, box maps).
 // Capturable.
 static int pair_launch(mc_context_s* c, int np, int n, float bfactor, int box, int wnoise,
-                       int precision, int cols = -1, int rows = -1) {
+                       int precision) {
   const mc_context_s::Tune* tn = pair_tune(c, n, box, precision);
-  if (cols < 0) cols = tn ? tn->cols : mc::PAIR_COLS_AUTO;
-  if (rows < 0) rows = tn ? tn->rows : mc::PAIR_ROWS_AUTO;
+  const int cols = tn ? tn->cols : mc::PAIR_COLS_AUTO;
   {
     KScope ks(c, MC_KT_PAIR_COLS);
     HIP_TRY(mc::launch_pair_cols(slot(c, 0), c->spec_stride, c->pairs_d.as<int2>(), np, n, bfactor,
-                                 box, c->tbuf.as<float2>(), c->tmax.as<float>(), precision, cols,
+                                 box, c->tbuf.as<float2>(), precision, cols,
                                  c->st));
   }
   {
     KScope ks(c, MC_KT_PAIR_ROWS);
-    HIP_TRY(mc::launch_pair_rows(c->tbuf.as<float2>(), c->tmax.as<float>(), np, n, box,
-                                 c->box.as<float>(), c->boxpart.as<float>(), precision, rows,
-                                 c->st));
+    HIP_TRY(mc::launch_pair_rows(c->tbuf.as<float2>(), np, n, box, c->box.as<float>(),
+                                 c->boxpart.as<float>(), c->st));
   }
   {
     KScope ks(c, MC_KT_PEAKS);
@@ -1243,7 +1240,6 @@ static int pairs_prepare(mc_context_s* c, const std::vector<SizeGroup>& gs, Pair
   L.np = np;
   HIP_TRY(c->pairs_d.ensure(sizeof(int) * 2 * std::max<size_t>(1, np)));
   HIP_TRY(c->tbuf.ensure(sizeof(float2) * std::max<size_t>(1, tel)));
-  if (L.precision == MC_PREC_MFMA_HILO) HIP_TRY(c->tmax.ensure(sizeof(float) * std::max<size_t>(1, tel / L.box)));
   HIP_TRY(c->box.ensure(sizeof(float) * std::max<size_t>(1, np) * L.box * L.box));
   HIP_TRY(c->boxpart.ensure(sizeof(float) * std::max<size_t>(1, part)));
   HIP_TRY(c->peaks.ensure(sizeof(double) * 3 * std::max<size_t>(1, np)));
@@ -1261,10 +1257,9 @@ static int pairs_launch(mc_context_s* c, const std::vector<SizeGroup>& gs, const
     for (const PairSpan& q : L.sp) {
       if (q.np == 0) continue;
       const SizeGroup& g = gs[q.gi];
-      float* tmax = L.precision == MC_PREC_MFMA_HILO ? c->tmax.as<float>() + q.to / box : nullptr;
       HIP_TRY(mc::launch_pair_cols(c->spec.as<float2>() + g.off, g.stride,
                                    c->pairs_d.as<int2>() + q.po, q.np, g.n, L.bfactor, box,
-                                   c->tbuf.as<float2>() + q.to, tmax, L.precision, q.cols, c->st));
+                                   c->tbuf.as<float2>() + q.to, L.precision, q.cols, c->st));
     }
   }
   // consecutive spans of one size group share a row-pass and a peak launch
@@ -1277,14 +1272,11 @@ static int pairs_launch(mc_context_s* c, const std::vector<SizeGroup>& gs, const
     const int n = gs[q.gi].n;
     i = j;
     if (np == 0) continue;
-    const mc_context_s::Tune* tn = pair_tune(c, n, box, L.precision);
-    const int rows = tn ? tn->rows : mc::PAIR_ROWS_AUTO;
     float* maps = c->box.as<float>() + q.po * box * box;
     {
       KScope ks(c, MC_KT_PAIR_ROWS);
-      float* tmax = L.precision == MC_PREC_MFMA_HILO ? c->tmax.as<float>() + q.to / box : nullptr;
-      HIP_TRY(mc::launch_pair_rows(c->tbuf.as<float2>() + q.to, tmax, np, n, box, maps,
-                                   c->boxpart.as<float>(), L.precision, rows, c->st));
+      HIP_TRY(mc::launch_pair_rows(c->tbuf.as<float2>() + q.to, np, n, box, maps,
+                                   c->boxpart.as<float>(), c->st));
     }
     {
       KScope ks(c, MC_KT_PEAKS);
@@ -1892,34 +1884,26 @@ extern "C" int mc_autotune(mc_context ctx, const mc_movie_desc* m, const mc_para
   MC_TRY(pair_reserve(c, r.P, n, box, p->precision));
   HIP_TRY(hipMemcpyAsync(c->pairs_d.p, slots.data(), sizeof(int) * slots.size(),
                          hipMemcpyHostToDevice, c->st));
-  int bcol = mc::PAIR_COLS_AUTO, brow = mc::PAIR_ROWS_AUTO;
+  const int bcol = mc::PAIR_COLS_AUTO, brow = mc::PAIR_ROWS_AUTO;
   if (p->precision == MC_PREC_FP32) {
-    {  // one column kernel per size: its time is reported
+    {  // one column and one row kernel per size: their times are reported
       float ms = 0;
       MC_TRY(time_min(c, reps, &ms, [&] {
         const hipError_t e = mc::launch_pair_cols(slot(c, 0), c->spec_stride,
                                                   c->pairs_d.as<int2>(), r.P, n, p->bfactor, box,
-                                                  c->tbuf.as<float2>(), c->tmax.as<float>(),
-                                                  p->precision, bcol, c->st);
+                                                  c->tbuf.as<float2>(), p->precision, bcol, c->st);
         return e == hipSuccess ? MC_OK : set_err(MC_ERR_DEVICE, "pair columns: %s", hipGetErrorString(e));
       }));
       tr.ms_pair_cols[bcol] = ms;
     }
-    best = 1e30f;
-    for (int v = 0; v < mc::PAIR_ROWS_VARIANTS; v++) {
-      if (v != mc::PAIR_ROWS_VALU && box > 96) continue;
+    {
       float ms = 0;
       MC_TRY(time_min(c, reps, &ms, [&] {
-        const hipError_t e = mc::launch_pair_rows(
-            c->tbuf.as<float2>(), c->tmax.as<float>(), r.P, n, box, c->box.as<float>(),
-            c->boxpart.as<float>(), p->precision, v, c->st);
+        const hipError_t e = mc::launch_pair_rows(c->tbuf.as<float2>(), r.P, n, box,
+                                                  c->box.as<float>(), c->boxpart.as<float>(), c->st);
         return e == hipSuccess ? MC_OK : set_err(MC_ERR_DEVICE, "pair rows: %s", hipGetErrorString(e));
       }));
-      tr.ms_pair_rows[v] = ms;
-      if (ms < best) {
-        best = ms;
-        brow = v;
-      }
+      tr.ms_pair_rows[brow] = ms;
     }
   }
   HIP_TRY(hipStreamSynchronize(c->st));

@@ -112,25 +112,17 @@ hipError_t launch_spectrum_to_image(const float2* spec, int n, float scale, floa
 // Pair stage: for each pair p, T[p][kx][r] (column pass) then the box map
 // C[p][r][c] (row pass).  pairs: device int2 (a, b) indices into `spectra`
 // (frame slots of stride spec_stride); operand a is kept, b conjugated.
-// precision 0: FP32 (vector ALUs; row pass on FP32 MFMA); 1: the first DFT
-// stage of the column pass and the row pass as FP16 hi/lo MFMA products
-// (tmax: npairs*(n/2+1) floats of column maxima, written by the column pass
-// and read by the row pass).
-// The column pass has one kernel per size and form (`variant` is one of the
-// codes that tuning files may hold; all run it).  Row-pass variants of the plain
-// form: AUTO = FP32 MFMA
-//   streaming each wave's kx range from memory (box <= 96; from n = 2048
-//   the kx range is also split over workgroups, a count set by n alone, whose
-//   partial maps go to `part`, pair_rows_part_elems(npairs, n, box) floats,
-//   and are added in order), VALU = register-tiled vector ALU kernel, MFMA8 / MFMA4 = FP32
-//   MFMA staged through LDS with 8 / 4 waves per (pair, 32-row block).
+// precision 0: FP32; 1: the first DFT stage of the column pass as FP16 hi/lo MFMA
+// products.  Each pass has one kernel per size (`variant` is one of the codes
+// that tuning files may hold; all run it).  The row pass splits the kx range over
+// workgroups, a count set by n alone, whose partial maps go to `part`
+// (pair_rows_part_elems(npairs, n, box) floats) and are added in order.
 enum { PAIR_COLS_AUTO = 0, PAIR_COLS_VARIANTS = 4 };
-enum { PAIR_ROWS_AUTO = 0, PAIR_ROWS_VALU = 1, PAIR_ROWS_MFMA8 = 2, PAIR_ROWS_MFMA4 = 3,
-       PAIR_ROWS_VARIANTS = 4 };
+enum { PAIR_ROWS_AUTO = 0, PAIR_ROWS_VARIANTS = 4 };
 bool pair_form_supported(int precision, int n, int box);
 hipError_t launch_pair_cols(const float2* spectra, size_t spec_stride, const int2* pairs,
                             int npairs, int n, float bfactor, int box, float2* tbuf,
-                            float* tmax, int precision, int variant, hipStream_t st);
+                            int precision, int variant, hipStream_t st);
 // The FP32 column pass (mc_cols.hip; wxy: the weight table of mc_pair.hip), and
 // the kx segments of a persistent column-pass launch sequence.
 hipError_t launch_pair_cols_fp32(const float2* spectra, size_t spec_stride, const int2* pairs,
@@ -138,9 +130,8 @@ hipError_t launch_pair_cols_fp32(const float2* spectra, size_t spec_stride, cons
                                  hipStream_t st);
 int col_segments(int npairs, int H, int grid);
 size_t pair_rows_part_elems(int npairs, int n, int box);
-hipError_t launch_pair_rows(const float2* tbuf, const float* tmax, int npairs, int n, int box,
-                            float* boxmaps, float* part, int precision, int variant,
-                            hipStream_t st);
+hipError_t launch_pair_rows(const float2* tbuf, int npairs, int n, int box, float* boxmaps,
+                            float* part, hipStream_t st);
 
 // Peaks: integer peak + FP64 16x16 -> 512x512 sub-pixel search per box map.
 // out: 3 doubles per pair (sx, sy, cc).

@@ -10,11 +10,9 @@
 //
 //  column pass : T[r], the column inverse at the box rows R_r = (n-box)/2 + r
 //    of the product formed on the fly from the two spectra columns (mc_cols.hip).
-//  k_pair_rows : one pair per workgroup: C[r][c] = sum_kx a_kx Re(T[kx][r]
-//    e^{2 pi i kx R_c/n}) with a_0 = a_{n/2} = 1, a_kx = 2 (the C2R row
-//    transform with the DC/Nyquist projection): a real GEMM with K =
-//    2(n/2+1), on the matrix cores (k_pair_rows_mfma, box <= 96) or
-//    register-tiled on the vector ALUs.
+//  row pass    : C[r][c] = sum_kx a_kx Re(T[kx][r] e^{2 pi i kx R_c/n}) with
+//    a_0 = a_{n/2} = 1, a_kx = 2 (the C2R row transform with the DC/Nyquist
+//    projection): a real GEMM with K = 2(n/2+1) on the matrix cores.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -31,6 +29,8 @@
 #include "mc_kernels.h"
 
 namespace mc {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 // MFMA operand and accumulator vectors
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -66,7 +66,6 @@ __global__ __launch_bounds__(256) void k_pair_cols_mfma(const float2* __restrict
                                                         int npairs,
                                                         const float* __restrict__ wxy, int box,
                                                         float2* __restrict__ tbuf,
-                                                        float* __restrict__ tmax,
                                                         const float2* __restrict__ tw,
                                                         int kxb, int nkx) {
   constexpr int NT = 256;
@@ -82,7 +81,6 @@ __global__ __launch_bounds__(256) void k_pair_cols_mfma(const float2* __restrict
   constexpr int AS = A / SP;
   static_assert(CB >= 1 && (8 * A) % 32 == 0 && A % SP == 0, "shape");
   __shared__ float2 buf[A * TS];
-  __shared__ float red[NT / 64];
   const int tid = threadIdx.x;
   const int wv = tid / 64, l = tid % 64, li = l % 32, lh = l / 32;
   // DFT-16 matrix fragments (rows (k1, re|im), columns (b1, re|im)), hi/lo
@@ -216,258 +214,88 @@ __global__ __launch_bounds__(256) void k_pair_cols_mfma(const float2* __restrict
       acc.x += __shfl_xor(acc.x, o);
       acc.y += __shfl_xor(acc.y, o);
     }
-    float mx = (cact && ch == 0) ? fmaxf(fabsf(acc.x), fabsf(acc.y)) : 0.f;
     if (cact && ch == 0) tbuf[((size_t)p * H + kx) * box + cr] = acc;
-    // column maximum of T for the scale of the row pass
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    if (l == 0) red[wv] = mx;
-    __syncthreads();  // also: buf is rewritten by the next item's stage 0
-    if (tid == 0) tmax[(size_t)p * H + kx] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    __syncthreads();  // buf is rewritten by the next item's stage 0
   }
 }
 
-template <int BT>
-__global__ __launch_bounds__(256) void k_pair_rows(const float2* __restrict__ tbuf, int n,
-                                                   int box, float* __restrict__ boxmaps,
-                                                   const float2* __restrict__ tw) {
-  constexpr int KC = 16;
-  constexpr int W = 16 * BT;
-  __shared__ float2 Ts[KC][W];
-  __shared__ float2 Es[KC][W];
-  const int p = blockIdx.x;
+// Row pass: per pair the box map is the real product C = A B with
+// A[r][(kx, 0|1)] = a_kx (Re, Im) T[kx][r] and B[(kx, 0|1)][c] = (cos, -sin)(2 pi
+// kx R_c/n), K = 2(n/2+1) (the row half of the C2R at DFAlign.cu:897 restricted to
+// FindShift's box, cufunc.cu:398-407), on FP32 matrix instructions, whose rate
+// bounds it.  So it is computed as the even and odd parts about the box's
+// centre: with T' = T e^{2 pi i kx c/n}, c = ori + (box - 1)/2, the columns c +- x
+// (x = i + 1/2, of an odd box x = i) are
+//   E_x -+ O_x,  E_x = sum a_kx Re T' cos(2 pi kx x/n),  O_x = sum a_kx Im T' sin(..),
+// half the multiply-adds.  v_mfma_f32_16x16x4: rows r, columns i, four bins per
+// instruction; lane l holds T[kx + l / 16][16 i + l % 16] and the factors of its
+// bin, D steps ahead in registers, and keeps all 2 MR NC blocks.  No LDS in the
+// main loop.  Rows of A past the box repeat the last box row; their outputs are
+// never stored.  A workgroup takes 16 MR rows (blockIdx.z).
+// The bins of a pair are split over ks workgroups and over the NW waves of each.
+// The NW partial maps are summed in LDS, 16 bytes per lane; workgroup s writes
+// partial map s of its pair and k_sum_parts adds them.  Bin 0 is added last and
+// the partial maps from the highest bins down: the terms grow that way (B-factor
+// weight, and the mean of the image in bin 0 is the largest of all), so the
+// rounding of the partial sums is that of the correlation itself and not that of
+// its constant offset.
+// Box 96: 512, 21 pairs 18 us; 1854, 66 pairs 29; 2048, 15 pairs 23, 55 pairs 27;
+// 4096, 91 pairs 67.  The product over all columns (32x32x2, 128 bins per wave)
+// took 58, 111, 79, 82 and 140; forms staged through LDS or in FP16 pieces more.
+template <int MR, int NC, int NW, int D>
+__global__ __launch_bounds__(NW * 64, (8 / NW > 1 ? 8 / NW : 1)) void k_pair_rows_stream(
+    const float2* __restrict__ tbuf, int n, int box, int ks, float* __restrict__ out,
+    const float2* __restrict__ ef, const float2* __restrict__ ph) {
+  constexpr int W = 16 * NC;
+  const int p = blockIdx.x, s = blockIdx.y, r0 = 16 * MR * blockIdx.z;
   const int H = n / 2 + 1;
-  const int ori = (n - box) / 2;
-  const float2* T = tbuf + (size_t)p * H * box;
-  const int tr = threadIdx.x / 16, tc = threadIdx.x % 16;
-  float acc[BT][BT];
-#pragma unroll
-  for (int i = 0; i < BT; i++)
-#pragma unroll
-    for (int j = 0; j < BT; j++) acc[i][j] = 0.f;
-  // bins from high to low (see k_pair_rows_stream)
-  for (int k0 = (H - 1) / KC * KC; k0 >= 0; k0 -= KC) {
-    for (int i = threadIdx.x; i < KC * W; i += 256) {
-      const int kk = i / W, c = i % W;
-      const int kx = k0 + kk;
-      float2 t = make_float2(0.f, 0.f), e = make_float2(0.f, 0.f);
-      if (kx < H && c < box) {
-        const float al = (kx == 0 || 2 * kx == n) ? 1.f : 2.f;
-        t = cscale(T[(size_t)kx * box + c], al);
-        e = tw[(int)(((long long)kx * (ori + c)) % n)];
-      }
-      Ts[kk][c] = t;
-      Es[kk][c] = e;
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int kk = KC - 1; kk >= 0; kk--) {
-      float2 tv[BT], ev[BT];
-#pragma unroll
-      for (int i = 0; i < BT; i++) {
-        tv[i] = Ts[kk][tr + 16 * i];
-        ev[i] = Es[kk][tc + 16 * i];
-      }
-#pragma unroll
-      for (int i = 0; i < BT; i++)
-#pragma unroll
-        for (int j = 0; j < BT; j++) acc[i][j] += tv[i].x * ev[j].x - tv[i].y * ev[j].y;
-    }
-    __syncthreads();
-  }
-  float* out = boxmaps + (size_t)p * box * box;
-#pragma unroll
-  for (int i = 0; i < BT; i++)
-#pragma unroll
-    for (int j = 0; j < BT; j++) {
-      const int r = tr + 16 * i, c = tc + 16 * j;
-      if (r < box && c < box) out[(size_t)r * box + c] = acc[i][j];
-    }
-}
-
-// The same row pass on the matrix cores: per pair the box map is the real
-// product C = A B with A[r][(kx, 0|1)] = a_kx (Re, Im) T[kx][r] and
-// B[(kx, 0|1)][c] = (cos, -sin)(2 pi kx R_c/n), K = 2(n/2+1).  One
-// v_mfma_f32_32x32x2f32 consumes one kx for a 32 x 32 block (FP32 operands
-// and accumulation).  Chunks of KC bins of T and of the twiddles are staged
-// in LDS (double-buffered: the next chunk is fetched into registers while
-// the current one is multiplied); each of the four waves takes a quarter of
-// every chunk for all NB x NB blocks, and the four partial maps are summed
-// in LDS in wave order.  Lane layout (32x32x2 f32): lane l feeds
-// A[l % 32][l / 32] and B[l / 32][l % 32]; accumulator v of lane l is
-// C[8 (v / 4) + 4 (l / 32) + v % 4][l % 32].
-template <int NB, int NT>
-__global__ __launch_bounds__(NT) void k_pair_rows_mfma(const float2* __restrict__ tbuf, int n,
-                                                        int box, float* __restrict__ boxmaps,
-                                                        const float2* __restrict__ etab) {
-  constexpr int W = 32 * NB;
-  constexpr int KC = 32;
-  constexpr int NW = NT / 64;  // waves; each takes KC/NW bins of every chunk
-  static_assert(KC % NW == 0, "chunk split");
-  constexpr int PT = (KC * 32 + NT - 1) / NT;  // T elements (this row block) per thread
-  constexpr int PE = (KC * W + NT - 1) / NT;   // twiddles per thread
-  __shared__ float2 Ts[2][KC][32];
-  __shared__ float2 Es[2][KC][W];
-  const int p = blockIdx.x;
-  const int rb = blockIdx.y;  // 32-row block of the box map
-  const int H = n / 2 + 1;
-  const float2* T = tbuf + (size_t)p * H * box;
-  const int wv = threadIdx.x / 64, l = threadIdx.x % 64;
-  const int li = l % 32, lh = l / 32;
-  v16f acc[NB];
-#pragma unroll
-  for (int j = 0; j < NB; j++)
-#pragma unroll
-    for (int v = 0; v < 16; v++) acc[j][v] = 0.f;
-  float2 pt[PT], pe[PE];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int q = 0; q < PT; q++) {
-      const int i = threadIdx.x + NT * q;
-      const int kk = i / 32, r = 32 * rb + i % 32, kx = k0 + kk;
-      float2 t = make_float2(0.f, 0.f);
-      if (i < KC * 32 && kx < H && r < box) {
-        const float al = (kx == 0 || 2 * kx == n) ? 1.f : 2.f;
-        t = cscale(T[(size_t)kx * box + r], al);
-      }
-      pt[q] = t;
-    }
-#pragma unroll
-    for (int q = 0; q < PE; q++) {
-      const int i = threadIdx.x + NT * q;
-      const int kk = i / W, c = i % W, kx = k0 + kk;
-      float2 e = make_float2(0.f, 0.f);
-      if (i < KC * W && kx < H && c < box) e = etab[(size_t)kx * box + c];
-      pe[q] = e;
-    }
-  };
-  auto stash = [&](int b) {
-#pragma unroll
-    for (int q = 0; q < PT; q++) {
-      const int i = threadIdx.x + NT * q;
-      if (i < KC * 32) Ts[b][i / 32][i % 32] = pt[q];
-    }
-#pragma unroll
-    for (int q = 0; q < PE; q++) {
-      const int i = threadIdx.x + NT * q;
-      if (i < KC * W) Es[b][i / W][i % W] = pe[q];
-    }
-  };
-  // bins from high to low (see k_pair_rows_stream)
-  const int nch = (H + KC - 1) / KC;
-  fetch((nch - 1) * KC);
-  stash((nch - 1) & 1);
-  __syncthreads();
-  for (int ch = nch - 1; ch >= 0; ch--) {
-    const int b = ch & 1;
-    if (ch > 0) fetch((ch - 1) * KC);
-#pragma unroll 2
-    for (int kk = (wv + 1) * (KC / NW) - 1; kk >= wv * (KC / NW); kk--) {
-      const float2 tv = Ts[b][kk][li];
-      const float a = lh ? tv.y : tv.x;
-      float bb[NB];
-#pragma unroll
-      for (int j = 0; j < NB; j++) {
-        const float2 ev = Es[b][kk][32 * j + li];
-        bb[j] = lh ? -ev.y : ev.x;
-      }
-#pragma unroll
-      for (int j = 0; j < NB; j++)
-        acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, bb[j], acc[j], 0, 0, 0);
-    }
-    if (ch > 0) stash(b ^ 1);
-    __syncthreads();
-  }
-  // ordered sum of the NW partial row blocks in LDS (reuses the buffers)
-  float* red = reinterpret_cast<float*>(&Es[0][0][0]);
-  static_assert(sizeof(Es) >= sizeof(float) * 32 * W, "reduction buffer");
-  for (int w = NW - 1; w >= 0; w--) {
-    if (wv == w) {
-#pragma unroll
-      for (int j = 0; j < NB; j++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-          const int r = 8 * (v / 4) + 4 * lh + (v % 4), c = 32 * j + li;
-          if (w == NW - 1) red[r * W + c] = acc[j][v];
-          else red[r * W + c] += acc[j][v];
-        }
-    }
-    __syncthreads();
-  }
-  float* out = boxmaps + (size_t)p * box * box;
-  const int rows = min(32, box - 32 * rb);
-  for (int e = threadIdx.x; e < rows * box; e += NT)
-    out[(size_t)(32 * rb + e / box) * box + e % box] = red[(e / box) * W + e % box];
-}
-
-// Streaming form of the same GEMM (box <= 96), with no LDS staging in the
-// main loop.  The K range of a pair (bins kx in [0, n/2]) is split over ks
-// workgroups and over the NW waves of each; a wave walks its contiguous kx
-// range, each lane loading just the float it feeds (A[l % 32][l / 32] =
-// (Re | Im) T[kx][r]; B[l / 32][l % 32] from a table that holds
-// a_kx (cos, -sin)(2 pi kx R_c/n), zero past the box), D bins ahead in
-// registers, and keeps all NB x NB accumulator blocks.  Rows of A past the
-// box repeat the last box row; their outputs are never stored.  The NW
-// partial maps are summed in LDS; with ks > 1 workgroup s writes partial map s
-// of its pair and k_sum_parts adds them.  Bin 0 is added last and the partial
-// maps from the highest bins down: the terms grow that way (B-factor weight,
-// and the mean of the image in bin 0 is the largest of all), so the rounding of
-// the partial sums is that of the correlation itself and not that of its
-// constant offset (box maps at n = 1536, 20 frames: 1.1e-7 of the maximum
-// against 6e-7 with bin 0 first).
-template <int NB, int NW, int D>
-__global__ __launch_bounds__(NW * 64, (8 / NW > 1 ? 8 / NW : 1)) void k_pair_rows_stream(const float* __restrict__ tf, int n,
-                                                              int box, int ks,
-                                                              float* __restrict__ out,
-                                                              const float* __restrict__ ef) {
-  constexpr int W = 32 * NB;
-  const int p = blockIdx.x, s = blockIdx.y;
-  const int H = n / 2 + 1;
-  const int wv = threadIdx.x / 64, l = threadIdx.x % 64, li = l % 32, lh = l / 32;
+  const int wv = threadIdx.x / 64, l = threadIdx.x % 64, li = l % 16, lk = l / 16;
   const int nsub = ks * NW, sub = s * NW + wv;
   const int k0 = (int)((long long)H * sub / nsub), k1 = (int)((long long)H * (sub + 1) / nsub);
   const int kb = k0 > 0 ? k0 : 1;  // bin 0 comes last
-  const float* T = tf + (size_t)p * H * box * 2;
-  int roff[NB];
+  const float2* T = tbuf + (size_t)p * H * box;
+  int roff[MR];
 #pragma unroll
-  for (int i = 0; i < NB; i++) roff[i] = 2 * min(32 * i + li, box - 1) + lh;
-  const int eoff = 2 * li + lh;
-  v16f acc[NB][NB];
+  for (int i = 0; i < MR; i++) roff[i] = min(r0 + 16 * i + li, box - 1);
+  v4f e[MR][NC], o[MR][NC];
 #pragma unroll
-  for (int i = 0; i < NB; i++)
+  for (int i = 0; i < MR; i++)
 #pragma unroll
-    for (int j = 0; j < NB; j++)
+    for (int j = 0; j < NC; j++) e[i][j] = o[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+  float2 a[D][MR], b[D][NC], f[D];
+  // operands of the bins kx + lk (at most n/2) into slot d; bins at or past
+  // `end` get the factor zero
+  auto load = [&](int d, int kx, int end) {
+    const int kc = min(kx + lk, H - 1);
+    const float2* tr = T + (size_t)kc * box;
+    const float2* er = ef + (size_t)kc * W + li;
 #pragma unroll
-      for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-  float a[D][NB], b[D][NB];
-  // operands of bin min(kx, n/2) into slot d (bins past the wave's range
-  // are loaded but never multiplied)
-  auto load = [&](int d, int kx) {
-    const int kc = min(kx, H - 1);
-    const float* tr = T + (size_t)kc * box * 2;
-    const float* er = ef + (size_t)kc * W * 2;
+    for (int i = 0; i < MR; i++) a[d][i] = tr[roff[i]];
 #pragma unroll
-    for (int i = 0; i < NB; i++) a[d][i] = tr[roff[i]];
-#pragma unroll
-    for (int j = 0; j < NB; j++) b[d][j] = er[eoff + 64 * j];
+    for (int j = 0; j < NC; j++) b[d][j] = er[16 * j];
+    f[d] = ph[kx + lk < end ? kc : H];
   };
   auto mul = [&](int d) {
 #pragma unroll
-    for (int i = 0; i < NB; i++)
+    for (int i = 0; i < MR; i++) {
+      const float2 t = cmul(a[d][i], f[d]);
 #pragma unroll
-      for (int j = 0; j < NB; j++)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d][i], b[d][j], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < NC; j++) {
+        e[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(t.x, b[d][j].x, e[i][j], 0, 0, 0);
+        o[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(t.y, b[d][j].y, o[i][j], 0, 0, 0);
+      }
+    }
   };
 #pragma unroll
-  for (int d = 0; d < D; d++) load(d, kb + d);
-  const int nfull = (k1 - kb) / D, rem = (k1 - kb) % D;
+  for (int d = 0; d < D; d++) load(d, kb + 4 * d, k1);
+  const int steps = (k1 - kb + 3) / 4, nfull = steps / D, rem = steps % D;
   for (int it = 0; it < nfull; it++) {
-    const int kn = kb + (it + 1) * D;
+    const int kn = kb + (it + 1) * 4 * D;
 #pragma unroll
     for (int d = 0; d < D; d++) {
       mul(d);
-      load(d, kn + d);
-      // keeps each step's loads in that step, D bins ahead of their use: the
+      load(d, kn + 4 * d, k1);
+      // keeps each step's loads in that step, D steps ahead of their use: the
       // memory clobber stops them sinking into the next iteration, the
       // scheduling barrier stops the MFMAs of later steps moving above them
       asm volatile("" ::: "memory");
@@ -478,28 +306,48 @@ __global__ __launch_bounds__(NW * 64, (8 / NW > 1 ? 8 / NW : 1)) void k_pair_row
   for (int d = 0; d < D; d++)
     if (d < rem) mul(d);
   if (k0 == 0) {
-    load(0, 0);
+    load(0, 0, 1);
     mul(0);
   }
-  // ordered sum of the NW wave maps, high bins first
-  __shared__ float red[W * W];
+  // ordered sum of the NW wave maps, high bins first: blocks [E | O][i][j] of
+  // 64 lanes x 4
+  __shared__ float4 red[2 * MR * NC][64];
   for (int w = NW - 1; w >= 0; w--) {
     if (wv == w) {
 #pragma unroll
-      for (int i = 0; i < NB; i++)
+      for (int i = 0; i < MR; i++)
 #pragma unroll
-        for (int j = 0; j < NB; j++)
+        for (int j = 0; j < NC; j++)
 #pragma unroll
-          for (int v = 0; v < 16; v++) {
-            const int r = 32 * i + 8 * (v / 4) + 4 * lh + (v % 4), c = 32 * j + li;
-            if (w == NW - 1) red[r * W + c] = acc[i][j][v];
-            else red[r * W + c] += acc[i][j][v];
+          for (int q = 0; q < 2; q++) {
+            const v4f v = q ? o[i][j] : e[i][j];
+            float4& r = red[(q * MR + i) * NC + j][l];
+            float4 x = make_float4(v[0], v[1], v[2], v[3]);
+            if (w < NW - 1) {
+              const float4 y = r;
+              x = make_float4(y.x + x.x, y.y + x.y, y.z + x.z, y.w + x.w);
+            }
+            r = x;
           }
     }
     __syncthreads();
   }
-  float* o = out + ((size_t)p * ks + s) * box * box;
-  for (int e = threadIdx.x; e < box * box; e += NW * 64) o[e] = red[(e / box) * W + e % box];
+  // columns c + x: E - O, c - x: E + O
+  float* om = out + ((size_t)p * ks + s) * box * box;
+  const int half = (box + 1) / 2;
+  for (int t = wv; t < MR * NC; t += NW) {
+    const float4 x = red[t][l], y = red[MR * NC + t][l];
+    const int i = t / NC, c = 16 * (t - i * NC) + li;
+    const float E[4] = {x.x, x.y, x.z, x.w}, O[4] = {y.x, y.y, y.z, y.w};
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int r = r0 + 16 * i + 4 * lk + v;
+      if (r < box && c < half) {
+        om[(size_t)r * box + box - half + c] = E[v] - O[v];
+        om[(size_t)r * box + half - 1 - c] = E[v] + O[v];
+      }
+    }
+  }
 }
 
 // out[p][e] = sum_{s < ks} part[p][s][e] (e < m), added from the last s to 0.
@@ -512,141 +360,6 @@ __global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ par
   float v = q[(size_t)(ks - 1) * m];
   for (int s = ks - 2; s >= 0; s--) v += q[(size_t)s * m];
   out[i] = v;
-}
-
-// Row pass of the MFMA FP16 hi/lo form: the GEMM of k_pair_rows_mfma with
-// v_mfma_f32_32x32x8f16 (four kx per instruction: K index 2 kk + (Re|Im)).
-// T of a pair is scaled by the power of two that puts max|T| (the column
-// maxima tmax written by k_pair_cols_mfma) in [2^13, 2^14); T and the
-// twiddles are split into FP16 hi/lo pairs when staged in LDS and
-// multiplied as hi*hi + hi*lo + lo*hi.
-template <int NB>
-__global__ __launch_bounds__(256) void k_pair_rows_mfma16(const float2* __restrict__ tbuf,
-                                                          const float* __restrict__ tmax, int n,
-                                                          int box, float* __restrict__ boxmaps,
-                                                          const float2* __restrict__ etab) {
-  constexpr int W = 32 * NB;
-  constexpr int KC = 32;
-  constexpr int PER = (KC * W + 255) / 256;
-  __shared__ h2 S4[4][2][KC][W];  // T hi, T lo, E hi, E lo; double-buffered
-  __shared__ float red[4];
-  auto Th = S4[0];
-  auto Tl = S4[1];
-  auto Eh = S4[2];
-  auto El = S4[3];
-  const int p = blockIdx.x;
-  const int H = n / 2 + 1;
-  const float2* T = tbuf + (size_t)p * H * box;
-  const int wv = threadIdx.x / 64, l = threadIdx.x % 64;
-  const int li = l % 32, lh = l / 32;
-  // pair scale
-  float m = 0.f;
-  for (int k = threadIdx.x; k < H; k += 256) m = fmaxf(m, tmax[(size_t)p * H + k]);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-  if (l == 0) red[wv] = m;
-  __syncthreads();
-  m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  int ex = 0;
-  (void)frexpf(m, &ex);
-  const int sh = m > 0.f ? 14 - ex : 0;
-  v16f acc[NB][NB];
-#pragma unroll
-  for (int i = 0; i < NB; i++)
-#pragma unroll
-    for (int j = 0; j < NB; j++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-  float2 pt[PER], pe[PER];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int q = 0; q < PER; q++) {
-      const int i = threadIdx.x + 256 * q;
-      const int kk = i / W, c = i % W, kx = k0 + kk;
-      float2 t = make_float2(0.f, 0.f), e = make_float2(0.f, 0.f);
-      if (i < KC * W && kx < H && c < box) {
-        const float al = (kx == 0 || 2 * kx == n) ? 1.f : 2.f;
-        t = T[(size_t)kx * box + c];
-        t = make_float2(ldexpf(al * t.x, sh), ldexpf(al * t.y, sh));
-        e = etab[(size_t)kx * box + c];
-        e.y = -e.y;
-      }
-      pt[q] = t;
-      pe[q] = e;
-    }
-  };
-  auto stash = [&](int b) {
-#pragma unroll
-    for (int q = 0; q < PER; q++) {
-      const int i = threadIdx.x + 256 * q;
-      if (i < KC * W) {
-        _Float16 a0, a1, b0, b1;
-        split_hilo(pt[q].x, a0, a1);
-        split_hilo(pt[q].y, b0, b1);
-        Th[b][i / W][i % W] = h2{a0, b0};
-        Tl[b][i / W][i % W] = h2{a1, b1};
-        split_hilo(pe[q].x, a0, a1);
-        split_hilo(pe[q].y, b0, b1);
-        Eh[b][i / W][i % W] = h2{a0, b0};
-        El[b][i / W][i % W] = h2{a1, b1};
-      }
-    }
-  };
-  const int nch = (H + KC - 1) / KC;
-  // bins from high to low (see k_pair_rows_stream)
-  fetch((nch - 1) * KC);
-  stash((nch - 1) & 1);
-  __syncthreads();
-  for (int ch = nch - 1; ch >= 0; ch--) {
-    const int b = ch & 1;
-    if (ch > 0) fetch((ch - 1) * KC);
-#pragma unroll
-    for (int ks = KC / 16 - 1; ks >= 0; ks--) {
-      const int kk = wv * (KC / 4) + 4 * ks + 2 * lh;  // this lane's two bins
-      v4h ah[NB], al_[NB], bh[NB], bl[NB];
-#pragma unroll
-      for (int i = 0; i < NB; i++) {
-        const h2 x0 = Th[b][kk][32 * i + li], x1 = Th[b][kk + 1][32 * i + li];
-        const h2 y0 = Tl[b][kk][32 * i + li], y1 = Tl[b][kk + 1][32 * i + li];
-        ah[i] = v4h{x0[0], x0[1], x1[0], x1[1]};
-        al_[i] = v4h{y0[0], y0[1], y1[0], y1[1]};
-        const h2 e0 = Eh[b][kk][32 * i + li], e1 = Eh[b][kk + 1][32 * i + li];
-        const h2 f0 = El[b][kk][32 * i + li], f1 = El[b][kk + 1][32 * i + li];
-        bh[i] = v4h{e0[0], e0[1], e1[0], e1[1]};
-        bl[i] = v4h{f0[0], f0[1], f1[0], f1[1]};
-      }
-#pragma unroll
-      for (int i = 0; i < NB; i++)
-#pragma unroll
-        for (int j = 0; j < NB; j++) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x8f16(ah[i], bl[j], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x8f16(al_[i], bh[j], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x8f16(ah[i], bh[j], acc[i][j], 0, 0, 0);
-        }
-    }
-    if (ch > 0) stash(b ^ 1);
-    __syncthreads();
-  }
-  float* redm = reinterpret_cast<float*>(&S4[0][0][0][0]);
-  static_assert(sizeof(S4) >= sizeof(float) * W * W, "reduction buffer");
-  for (int w = 3; w >= 0; w--) {
-    if (wv == w) {
-#pragma unroll
-      for (int i = 0; i < NB; i++)
-#pragma unroll
-        for (int j = 0; j < NB; j++)
-#pragma unroll
-          for (int v = 0; v < 16; v++) {
-            const int r = 32 * i + 8 * (v / 4) + 4 * lh + (v % 4), c = 32 * j + li;
-            if (w == 3) redm[r * W + c] = acc[i][j][v];
-            else redm[r * W + c] += acc[i][j][v];
-          }
-    }
-    __syncthreads();
-  }
-  float* out = boxmaps + (size_t)p * box * box;
-  for (int e = threadIdx.x; e < box * box; e += 256)
-    out[e] = ldexpf(redm[(e / box) * W + e % box], -sh);
 }
 
 // Weight table: wxy[kx] = (-1)^kx exp(m kx^2), kx in [0, n/2]; wxy[n/2+1+ky]
@@ -680,10 +393,11 @@ static const float* weights(int n, float bfactor) {
   return d;
 }
 
-// Row-pass twiddles of a box: etab[kx * box + c] = e^{2 pi i kx R_c/n},
-// R_c = (n - box)/2 + c, kx in [0, n/2] (double on the host, the same values
-// as the n-point table), so the MFMA row kernels stream them like T.
-static const float2* row_twiddles(int n, int box) {
+// Tables of k_pair_rows_stream: per bin kx W columns of a_kx
+// (cos, sin)(2 pi kx x_i/n), x_i = i + 1/2 (of an odd box i), a_0 = a_{n/2} = 1,
+// a_kx = 2 otherwise, zeros past the half box; then e^{2 pi i kx c/n}, c = ori +
+// (box - 1)/2, and a zero.
+static const float2* row_twiddles_stream(int n, int box, int W) {
   static std::mutex mu;
   static std::map<std::tuple<int, int, int>, float2*> cache;
   int dev = 0;
@@ -692,14 +406,18 @@ static const float2* row_twiddles(int n, int box) {
   auto key = std::make_tuple(dev, n, box);
   auto it = cache.find(key);
   if (it != cache.end()) return it->second;
-  const int H = n / 2 + 1, ori = (n - box) / 2;
-  std::vector<float2> h((size_t)H * box);
-  for (int kx = 0; kx < H; kx++)
-    for (int c = 0; c < box; c++) {
-      const long long e = ((long long)kx * (ori + c)) % n;
-      const double a = 2.0 * M_PI * (double)e / (double)n;
-      h[(size_t)kx * box + c] = make_float2((float)cos(a), (float)sin(a));
+  const int H = n / 2 + 1, ori = (n - box) / 2, half = (box + 1) / 2;
+  std::vector<float2> h((size_t)H * W + H + 1, make_float2(0.f, 0.f));
+  const double u = M_PI / n;  // angles in units of pi/n, reduced mod 2 n
+  for (int kx = 0; kx < H; kx++) {
+    const float al = (kx == 0 || 2 * kx == n) ? 1.f : 2.f;
+    for (int i = 0; i < half; i++) {
+      const double a = u * (double)(((long long)kx * (2 * i + (box % 2 ? 0 : 1))) % (2 * n));
+      h[(size_t)kx * W + i] = make_float2(al * (float)cos(a), al * (float)sin(a));
     }
+    const double c = u * (double)(((long long)kx * (2 * ori + box - 1)) % (2 * n));
+    h[(size_t)H * W + kx] = make_float2((float)cos(c), (float)sin(c));
+  }
   float2* d = nullptr;
   if (hipMalloc(&d, sizeof(float2) * h.size()) != hipSuccess) return nullptr;
   if (hipMemcpy(d, h.data(), sizeof(float2) * h.size(), hipMemcpyHostToDevice) != hipSuccess) {
@@ -710,62 +428,25 @@ static const float2* row_twiddles(int n, int box) {
   return d;
 }
 
-// B operand table of k_pair_rows_stream: per bin kx, 32 ceil(box/32)
-// columns of (a_kx cos t, -a_kx sin t), t = 2 pi (kx R_c mod n)/n, with
-// a_0 = a_{n/2} = 1, a_kx = 2 otherwise, and zeros past the box.
-static const float* row_twiddles_stream(int n, int box) {
-  static std::mutex mu;
-  static std::map<std::tuple<int, int, int>, float*> cache;
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  std::lock_guard<std::mutex> lk(mu);
-  auto key = std::make_tuple(dev, n, box);
-  auto it = cache.find(key);
-  if (it != cache.end()) return it->second;
-  const int H = n / 2 + 1, ori = (n - box) / 2, W = 32 * ((box + 31) / 32);
-  std::vector<float> h((size_t)H * W * 2, 0.f);
-  for (int kx = 0; kx < H; kx++) {
-    const float al = (kx == 0 || 2 * kx == n) ? 1.f : 2.f;
-    for (int c = 0; c < box; c++) {
-      const long long e = ((long long)kx * (ori + c)) % n;
-      const double a = 2.0 * M_PI * (double)e / (double)n;
-      h[((size_t)kx * W + c) * 2] = al * (float)cos(a);
-      h[((size_t)kx * W + c) * 2 + 1] = -al * (float)sin(a);
-    }
-  }
-  float* d = nullptr;
-  if (hipMalloc(&d, sizeof(float) * h.size()) != hipSuccess) return nullptr;
-  if (hipMemcpy(d, h.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice) != hipSuccess) {
-    (void)hipFree(d);
-    return nullptr;
-  }
-  cache[key] = d;
-  return d;
-}
-
-// Waves per workgroup of the streaming row pass; two workgroups share a CU.
+// Waves per workgroup of the row pass; two workgroups share a CU.
 constexpr int ROWS_NW = 4;
 
-// K splits of the streaming row pass: ks = clamp((n/2+1)/512, 1, 8), so that
-// a wave walks about 128 bins.  The split fixes the order in which the FP32
-// partial products of a box map are added, so it depends on the transform
-// size alone: a pair gives the same map whatever the number of pairs in the
-// launch (one movie or a batch, a full pair set or an align-to-sum round)
-// and whatever the device's CU count.
-static int pair_rows_splits(int n) {
-  return std::max(1, std::min(8, (n / 2 + 1) / 512));
-}
+// K splits of the row pass: ks = clamp((n/2+1)/256, 2, 8), so that a wave walks
+// about 64 bins (128: 2048, 15 pairs 33 us against 23; 32: 4096, 91 pairs the
+// same).  The split fixes the order in which the FP32 partial products of a box
+// map are added, so it depends on the transform size alone: a pair gives the
+// same map whatever the number of pairs in the launch (one movie or a batch, a
+// full pair set or an align-to-sum round) and whatever the device's CU count.
+static int pair_rows_splits(int n) { return std::max(2, std::min(8, (n / 2 + 1) / 256)); }
 
 size_t pair_rows_part_elems(int npairs, int n, int box) {
-  const int ks = pair_rows_splits(n);
-  return ks > 1 ? (size_t)npairs * ks * box * box : 0;
+  return (size_t)npairs * pair_rows_splits(n) * box * box;
 }
-
 
 template <int N, int SP>
 static hipError_t pair_cols_mfma(const float2* spectra, size_t spec_stride, const int2* pairs,
                                  int npairs, const float* wxy, int box, float2* tbuf,
-                                 float* tmax, hipStream_t st) {
+                                 hipStream_t st) {
   const float2* tw = twiddles(N);
   if (!tw) return hipErrorOutOfMemory;
   static const int g = persistent_grid(k_pair_cols_mfma<N, SP>, 256);
@@ -774,7 +455,7 @@ static hipError_t pair_cols_mfma(const float2* spectra, size_t spec_stride, cons
   for (int sgi = 0; sgi < S; sgi++) {
     const int kxb = H * sgi / S, nkx = H * (sgi + 1) / S - kxb;
     hipLaunchKernelGGL((k_pair_cols_mfma<N, SP>), dim3(g), dim3(256), 0, st, spectra, spec_stride,
-                       pairs, npairs, wxy, box, tbuf, tmax, tw, kxb, nkx);
+                       pairs, npairs, wxy, box, tbuf, tw, kxb, nkx);
   }
   return hipGetLastError();
 }
@@ -788,17 +469,16 @@ bool pair_form_supported(int precision, int n, int box) {
 
 hipError_t launch_pair_cols(const float2* spectra, size_t spec_stride, const int2* pairs,
                             int npairs, int n, float bfactor, int box, float2* tbuf,
-                            float* tmax, int precision, int variant, hipStream_t st) {
+                            int precision, int variant, hipStream_t st) {
   if (npairs <= 0) return hipSuccess;
   if (!pair_form_supported(precision, n, box)) return hipErrorInvalidValue;
   const float* wxy = weights(n, bfactor);
   if (!wxy) return hipErrorOutOfMemory;
   if (precision == 1) {
-    if (!tmax) return hipErrorInvalidValue;
     switch (n) {
 #define MC_COLS_MFMA(NN) \
-  case NN: return box <= 64 ? pair_cols_mfma<NN, 4>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, tmax, st) \
-                            : pair_cols_mfma<NN, 2>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, tmax, st);
+  case NN: return box <= 64 ? pair_cols_mfma<NN, 4>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st) \
+                            : pair_cols_mfma<NN, 2>(spectra, spec_stride, pairs, npairs, wxy, box, tbuf, st);
       MC_COLS_MFMA(512) MC_COLS_MFMA(1024) MC_COLS_MFMA(2048) MC_COLS_MFMA(4096) MC_COLS_MFMA(8192)
       MC_COLS_MFMA(1536) MC_COLS_MFMA(3072) MC_COLS_MFMA(6144) MC_COLS_MFMA(2560)
       MC_COLS_MFMA(5120)
@@ -811,73 +491,37 @@ hipError_t launch_pair_cols(const float2* spectra, size_t spec_stride, const int
   return launch_pair_cols_fp32(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, st);
 }
 
-hipError_t launch_pair_rows(const float2* tbuf, const float* tmax, int npairs, int n, int box,
-                            float* boxmaps, float* part, int precision, int variant,
+template <int MR, int NC, int D>
+static hipError_t pair_rows(const float2* tbuf, int npairs, int n, int box, float* part,
                             hipStream_t st) {
+  constexpr int W = 16 * NC;
+  const float2* ef = row_twiddles_stream(n, box, W);
+  if (!ef) return hipErrorOutOfMemory;
+  const int ks = pair_rows_splits(n);
+  hipLaunchKernelGGL((k_pair_rows_stream<MR, NC, ROWS_NW, D>),
+                     dim3(npairs, ks, (box + 16 * MR - 1) / (16 * MR)), dim3(ROWS_NW * 64), 0, st, tbuf,
+                     n, box, ks, part, ef, ef + (size_t)(n / 2 + 1) * W);
+  return hipGetLastError();
+}
+
+// Tiles by the box: all rows up to 96; above, as many rows per workgroup as leave
+// the accumulators of its columns in registers (box 200, 4096, 15 pairs: 65 us
+// against 2.9 ms on the vector ALU).
+hipError_t launch_pair_rows(const float2* tbuf, int npairs, int n, int box, float* boxmaps,
+                            float* part, hipStream_t st) {
   if (npairs <= 0) return hipSuccess;
-  if (!pair_form_supported(precision, n, box)) return hipErrorInvalidValue;
-  const float2* tw = twiddles(n);
-  if (!tw) return hipErrorOutOfMemory;
-  if (precision == 0 && variant == PAIR_ROWS_AUTO && box <= 96) {
-    const float* ef = row_twiddles_stream(n, box);
-    if (!ef) return hipErrorOutOfMemory;
-    const int ks = pair_rows_splits(n);
-    if (ks > 1 && !part) return hipErrorInvalidValue;
-    float* dst = ks > 1 ? part : boxmaps;
-    const float* tf = reinterpret_cast<const float*>(tbuf);
-    constexpr int NT = ROWS_NW * 64;
-    switch ((box + 31) / 32) {
-      case 1: hipLaunchKernelGGL((k_pair_rows_stream<1, ROWS_NW, 16>), dim3(npairs, ks), dim3(NT), 0, st, tf, n, box, ks, dst, ef); break;
-      case 2: hipLaunchKernelGGL((k_pair_rows_stream<2, ROWS_NW, 12>), dim3(npairs, ks), dim3(NT), 0, st, tf, n, box, ks, dst, ef); break;
-      default: hipLaunchKernelGGL((k_pair_rows_stream<3, ROWS_NW, 8>), dim3(npairs, ks), dim3(NT), 0, st, tf, n, box, ks, dst, ef); break;
-    }
-    if (ks > 1) {
-      const long long total = (long long)npairs * box * box;
-      hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, part,
-                         ks, box * box, total, boxmaps);
-    }
-    return hipGetLastError();
-  }
-  const float2* etab = (precision == 1 || variant != PAIR_ROWS_VALU) ? row_twiddles(n, box) : nullptr;
-  if ((precision == 1 || variant != PAIR_ROWS_VALU) && !etab) return hipErrorOutOfMemory;
-  if (precision == 1) {
-    if (!tmax) return hipErrorInvalidValue;
-    switch ((box + 31) / 32) {
-#define MC_ROWS_MFMA16(B) \
-  case B: hipLaunchKernelGGL(k_pair_rows_mfma16<B>, dim3(npairs), dim3(256), 0, st, tbuf, tmax, n, box, boxmaps, etab); return hipGetLastError();
-      MC_ROWS_MFMA16(1) MC_ROWS_MFMA16(2) MC_ROWS_MFMA16(3)
-#undef MC_ROWS_MFMA16
-      default: return hipErrorInvalidValue;
-    }
-  }
-  if (variant != PAIR_ROWS_VALU && box <= 96) {
-    // one workgroup per (pair, 32-row block of the box)
-    const int nrb = (box + 31) / 32;
-    switch (nrb) {
-#define MC_ROWS_MFMA(B) \
-  case B: \
-    if (variant == PAIR_ROWS_MFMA8) \
-      hipLaunchKernelGGL((k_pair_rows_mfma<B, 512>), dim3(npairs, nrb), dim3(512), 0, st, tbuf, n, box, boxmaps, etab); \
-    else \
-      hipLaunchKernelGGL((k_pair_rows_mfma<B, 256>), dim3(npairs, nrb), dim3(256), 0, st, tbuf, n, box, boxmaps, etab); \
-    break;
-      MC_ROWS_MFMA(1) MC_ROWS_MFMA(2) MC_ROWS_MFMA(3)
-#undef MC_ROWS_MFMA
-      default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-  }
-  const int bt = (box + 15) / 16;
-  switch (bt) {
-#define MC_ROWS_CASE(B) \
-  case B: hipLaunchKernelGGL(k_pair_rows<B>, dim3(npairs), dim3(256), 0, st, tbuf, n, box, boxmaps, tw); break;
-    MC_ROWS_CASE(1) MC_ROWS_CASE(2) MC_ROWS_CASE(3) MC_ROWS_CASE(4) MC_ROWS_CASE(5)
-    MC_ROWS_CASE(6) MC_ROWS_CASE(7) MC_ROWS_CASE(8) MC_ROWS_CASE(9) MC_ROWS_CASE(10)
-    MC_ROWS_CASE(11) MC_ROWS_CASE(12) MC_ROWS_CASE(13) MC_ROWS_CASE(14) MC_ROWS_CASE(15)
-    MC_ROWS_CASE(16)
-#undef MC_ROWS_CASE
-    default: return hipErrorInvalidValue;
-  }
+  if (!pair_form_supported(0, n, box) || !part) return hipErrorInvalidValue;
+  hipError_t e;
+  if (box <= 32) e = pair_rows<2, 1, 6>(tbuf, npairs, n, box, part, st);
+  else if (box <= 64) e = pair_rows<4, 2, 4>(tbuf, npairs, n, box, part, st);
+  else if (box <= 96) e = pair_rows<6, 3, 3>(tbuf, npairs, n, box, part, st);
+  else if (box <= 128) e = pair_rows<4, 4, 3>(tbuf, npairs, n, box, part, st);
+  else if (box <= 192) e = pair_rows<3, 6, 3>(tbuf, npairs, n, box, part, st);
+  else e = pair_rows<2, 8, 3>(tbuf, npairs, n, box, part, st);
+  if (e != hipSuccess) return e;
+  const long long total = (long long)npairs * box * box;
+  hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, part,
+                     pair_rows_splits(n), box * box, total, boxmaps);
   return hipGetLastError();
 }
 
