@@ -84,6 +84,29 @@ struct DevBuf {
   template <class T> T* as() const { return reinterpret_cast<T*>(p); }
 };
 
+// Small results in pinned host memory that kernels write through the same
+// address: read after the stream's synchronisation, with no copy between. (The
+// copy and its staging left the GPU idle for 10 to 20 us each: 512x10 191 us per
+// call with copies.)
+struct PinBuf {
+  void* p = nullptr;
+  size_t cap = 0;
+  hipError_t ensure(size_t bytes) {
+    if (bytes <= cap) return hipSuccess;
+    release();
+    hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocDefault);
+    if (e == hipSuccess) cap = bytes;
+    else p = nullptr;
+    return e;
+  }
+  void release() {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    cap = 0;
+  }
+  template <class T> T* as() const { return reinterpret_cast<T*>(p); }
+};
+
 struct KTimer {
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
 };
@@ -91,8 +114,9 @@ struct KTimer {
 struct mc_context_s {
   int device = 0;
   hipStream_t st = nullptr;
-  DevBuf spec, rt, rowsum, fill, padP, pairs_d, tbuf, box, boxpart, peaks, shifts, image, tmp, means,
-      sum2img, wk, gpart, gout, jobs, fsc, disp;
+  DevBuf spec, rt, rowsum, fill, padP, pairs_d, tbuf, box, boxpart, shifts, image, tmp, sum2img,
+      wk, gpart, jobs, fsc, disp;
+  PinBuf peaks, means, gout;
   int graph_captures = 0, graph_replays = 0;
   // autotuned launch shapes (mc_autotune / mc_tune_load)
   struct Tune {
@@ -168,11 +192,12 @@ extern "C" int mc_context_destroy(mc_context ctx) {
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->st);
   DevBuf* bufs[] = {&ctx->spec, &ctx->rt, &ctx->rowsum, &ctx->fill, &ctx->padP,
-                    &ctx->pairs_d, &ctx->tbuf, &ctx->box, &ctx->boxpart, &ctx->peaks,
-                    &ctx->shifts, &ctx->image, &ctx->tmp, &ctx->means, &ctx->sum2img,
-                    &ctx->wk, &ctx->gpart, &ctx->gout, &ctx->jobs, &ctx->fsc,
+                    &ctx->pairs_d, &ctx->tbuf, &ctx->box, &ctx->boxpart,
+                    &ctx->shifts, &ctx->image, &ctx->tmp, &ctx->sum2img,
+                    &ctx->wk, &ctx->gpart, &ctx->jobs, &ctx->fsc,
                     &ctx->disp};
   for (DevBuf* b : bufs) b->release();
+  for (PinBuf* b : {&ctx->peaks, &ctx->means, &ctx->gout}) b->release();
   for (hipEvent_t e : ctx->pool) (void)hipEventDestroy(e);
   for (hipEvent_t e : ctx->gev)
     if (e) (void)hipEventDestroy(e);
@@ -589,13 +614,11 @@ static int pair_stage(mc_context_s* c, const std::vector<int>& slots, float bfac
   HIP_TRY(hipMemcpyAsync(c->pairs_d.p, slots.data(), sizeof(int) * slots.size(),
                          hipMemcpyHostToDevice, c->st));
   MC_TRY(pair_launch(c, np, n, bfactor, box, wnoise, precision));
-  res.resize(3 * (size_t)np);
-  HIP_TRY(hipMemcpyAsync(res.data(), c->peaks.p, sizeof(double) * 3 * np, hipMemcpyDeviceToHost,
-                         c->st));
   if (boxmaps_host)
     HIP_TRY(hipMemcpyAsync(boxmaps_host, c->box.p, sizeof(float) * (size_t)np * box * box,
                            hipMemcpyDeviceToHost, c->st));
   HIP_TRY(hipStreamSynchronize(c->st));
+  res.assign(c->peaks.as<double>(), c->peaks.as<double>() + 3 * (size_t)np);
   return MC_OK;
 }
 
@@ -628,8 +651,9 @@ static int sharp_weights(mc_context_s* c, int n, float bfactor) {
     h[H + ky] = (float)std::exp(m * (double)yy * yy);
   }
   HIP_TRY(c->wk.ensure(sizeof(float) * h.size()));
+  // (h is written again only after the sharpness_eval that follows has
+  // synchronised the stream)
   HIP_TRY(hipMemcpyAsync(c->wk.p, h.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice, c->st));
-  HIP_TRY(hipStreamSynchronize(c->st));
   return MC_OK;
 }
 
@@ -648,10 +672,9 @@ static int sharpness_eval(mc_context_s* c, int base, int F, int sum, const std::
                                  slot(c, sum), c->wk.as<float>(), c->gpart.as<double2>(),
                                  c->gout.as<double2>(), c->st));
   }
-  std::vector<double> o(2 * (size_t)(F + 1));
-  HIP_TRY(hipMemcpyAsync(o.data(), c->gout.p, sizeof(double) * o.size(), hipMemcpyDeviceToHost, c->st));
   HIP_TRY(hipStreamSynchronize(c->st));
-  grad->assign(o.begin(), o.begin() + 2 * F);
+  const double* o = c->gout.as<double>();
+  grad->assign(o, o + 2 * F);
   *J = o[2 * F];
   return MC_OK;
 }
@@ -809,10 +832,8 @@ extern "C" int mc_find_peaks(mc_context ctx, const float* boxmaps, int npairs, i
                          hipMemcpyHostToDevice, ctx->st));
   HIP_TRY(mc::launch_find_peaks(ctx->box.as<float>(), npairs, box, n, wnoise,
                                 ctx->peaks.as<double>(), ctx->st));
-  std::vector<double> res(3 * (size_t)npairs);
-  HIP_TRY(hipMemcpyAsync(res.data(), ctx->peaks.p, sizeof(double) * res.size(),
-                         hipMemcpyDeviceToHost, ctx->st));
   HIP_TRY(hipStreamSynchronize(ctx->st));
+  const double* res = ctx->peaks.as<double>();
   for (int q = 0; q < npairs; q++) {
     if (b) {
       b[2 * q] = res[3 * q];
@@ -1428,9 +1449,6 @@ static int align_group(mc_context_s* c, std::vector<MovieRun*>& rs, bool use_gra
       double* md = c->means.as<double>() + mo;
       HIP_TRY(mc::launch_dc_gather(slot(c, r->base), c->spec_stride, r->F, 1.0 / ((double)n * n), md,
                                    c->st));
-      if (r->out->frame_mean)
-        HIP_TRY(hipMemcpyAsync(r->out->frame_mean, md, sizeof(double) * r->F, hipMemcpyDeviceToHost,
-                               c->st));
       mo += r->F;
     }
   }
@@ -1479,10 +1497,6 @@ static int align_group(mc_context_s* c, std::vector<MovieRun*>& rs, bool use_gra
   }
   MC_TRY(pairs_prepare(c, gs, L, slots));
   MC_TRY(pairs_launch(c, gs, L));
-  std::vector<double> res(3 * L.np);
-  if (L.np)
-    HIP_TRY(hipMemcpyAsync(res.data(), c->peaks.p, sizeof(double) * 3 * L.np, hipMemcpyDeviceToHost,
-                           c->st));
   HIP_TRY(hipEventRecord(ev[2], c->st));
   {
     size_t po = 0;
@@ -1494,9 +1508,12 @@ static int align_group(mc_context_s* c, std::vector<MovieRun*>& rs, bool use_gra
     }
     HIP_TRY(hipStreamSynchronize(c->st));
     po = 0;
+    const double* md = c->means.as<double>();
     for (MovieRun* r : rs) {
+      if (r->out->frame_mean) std::copy(md, md + r->F, r->out->frame_mean);
+      md += r->F;
       // 3. least squares, outlier rejection, least squares (DFAlign.cu:914-948)
-      MC_TRY(solve_drift(*r, res.data() + 3 * po));
+      MC_TRY(solve_drift(*r, c->peaks.as<double>() + 3 * po));
       po += r->P;
     }
   }
@@ -1558,10 +1575,6 @@ static int align_group(mc_context_s* c, std::vector<MovieRun*>& rs, bool use_gra
       gr.key = key;  // buffers uploaded for this set
       MC_TRY(round_launch(c, gs, rj, R));
     }
-    const size_t np = islots.size() / 2;
-    res.resize(3 * np);
-    HIP_TRY(hipMemcpyAsync(res.data(), c->peaks.p, sizeof(double) * 3 * np, hipMemcpyDeviceToHost,
-                           c->st));
     size_t po = 0;
     for (MovieRun* r : act) {
       if (r->out->iter_boxmaps)
@@ -1573,7 +1586,7 @@ static int align_group(mc_context_s* c, std::vector<MovieRun*>& rs, bool use_gra
     HIP_TRY(hipStreamSynchronize(c->st));
     po = 0;
     for (MovieRun* r : act) {
-      iter_update(*r, res.data() + 3 * po);
+      iter_update(*r, c->peaks.as<double>() + 3 * po);
       po += r->F;
     }
   }
