@@ -60,7 +60,7 @@ extern "C" const char* mc_version(void) { return "motioncorr1exp_amd 0.1 (gfx950
 
 // Transform sizes: any even size in [64, 8192], as cuFFT plans any size
 // (cufunc.cu:202-215).  Powers of two and 2^k * {3, 5, 15} from 768 have
-// Stockham plans; the others run as chirp-z transforms.
+// Stockham plans; the others run in mixed factors or as chirp-z transforms.
 static bool fft_size_ok(int n) { return n >= 64 && n <= 8192 && n % 2 == 0; }
 
 // ------------------------------------------------------- device buffers
