@@ -580,7 +580,7 @@ def main():
         ctx.kernel_timing(False)
         out["reference_geometry"] = {
             "workload": "the same movie at the reference's default square crop, n = %d "
-                        "(no -pad; two-level stage-1 transforms), itr 0" % rr["report"]["n"],
+                        "(no -pad; mixed-factor stage-1 transforms), itr 0" % rr["report"]["n"],
             "n": rr["report"]["n"], "movies_per_s": kr / dtr, "ms_per_movie": dtr * 1e3 / kr,
             "kernels_ms_per_movie": kernr}
         log("reference geometry n=%d: %.3f ms/movie %s" % (rr["report"]["n"], dtr * 1e3 / kr,
