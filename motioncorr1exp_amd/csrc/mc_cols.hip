@@ -29,6 +29,7 @@
 #include <algorithm>
 #include <atomic>
 
+#include "mc_cols_form.h"
 #include "mc_device.h"
 #include "mc_kernels.h"
 
@@ -455,27 +456,14 @@ static hipError_t cols_r(const float2* spectra, size_t spec_stride, const int2* 
                          const float* wxy, int n, int box, float2* tbuf, const float2* tw,
                          hipStream_t st) {
   static std::atomic<int> cache[16][17];
-  const int nw = (n / R0 + 63) / 64;
-  const size_t lds = (size_t)nw * ((R0 > 8 ? 8192 : 66 * 64) + TILES * 2048);
+  const int nw = cols_r_waves(n, R0);
+  const size_t lds = cols_r_lds(n, R0, TILES);
   return cols_launches(k_pair_cols_r<R0, TILES>, nw, lds, cache, npairs, n / 2 + 1,
                        [&](int grid, int kxb, int nkx) {
                          hipLaunchKernelGGL((k_pair_cols_r<R0, TILES>), dim3(grid), dim3(nw * 64), lds,
                                             st, spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf,
                                             tw, kxb, nkx);
                        });
-}
-
-// The radix of k_pair_cols_r at size n and the tiles of eight groups that the
-// box needs: the largest divisor whose tiles and waves the kernel holds (its
-// work per element falls with R0); 0: none, the chirp-z pass.
-static int cols_radix(int n, int box, int* tiles) {
-  for (int R0 : {16, 14, 12, 10, 8, 6}) {
-    const int t = (box + 8 * R0 - 1) / (8 * R0), waves = (n / R0 + 63) / 64;
-    if (n % R0 || t > (R0 > 8 ? 2 : 3) || waves > (t == 1 || R0 <= 8 ? 16 : 8)) continue;
-    *tiles = t;
-    return R0;
-  }
-  return 0;
 }
 
 hipError_t launch_pair_cols_fp32(const float2* spectra, size_t spec_stride, const int2* pairs,

@@ -67,3 +67,19 @@ def test_box_maps_match_fp64(ctx, n, box):
         worst = max(worst, float(np.abs(maps[q] - ref).max() / np.abs(ref).max()))
     print("n %d box %d: max error / max %.3g" % (n, box, worst), flush=True)
     assert worst < 2e-6
+
+
+@pytest.mark.parametrize("n,box", [(5766, 128), (7672, 144), (8170, 80), (8184, 129), (8184, 192)])
+def test_many_waves_and_tiles(ctx, n, box):
+    """Three tiles of 16 waves exceed the LDS and take the chirp-z pass (5766,
+    8184); 15 waves of three tiles (7672) and 13 of a wide exchange (8170) fit.
+    Two white spectra, one pair; reference and bound as above."""
+    rng = np.random.default_rng(n + box)
+    spec = rng.standard_normal((2, n, n + 2), np.float32)
+    ctx.set_spectra(spec)
+    _, _, maps = ctx.pair_shifts(np.array([(0, 1)], np.int32), 150.0, box, want_boxes=True)
+    a, b = spec.view(np.complex64)
+    ref = reference_box(a.astype(np.complex128), b.astype(np.complex128), n, 150.0, box)
+    worst = float(np.abs(maps[0] - ref).max() / np.abs(ref).max())
+    print("n %d box %d: max error / max %.3g" % (n, box, worst), flush=True)
+    assert worst < 2e-6
