@@ -478,7 +478,8 @@ hipError_t launch_pair_cols_fp32(const float2* spectra, size_t spec_stride, cons
     return cols64<8>(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, tw, st);
   }
   int tiles = 0;
-  switch (cols_radix(n, box, &tiles) * 4 + tiles) {
+  const int R0 = cols_radix(n, box, &tiles);
+  switch (R0 * 4 + tiles) {
 #define MC_COLS_R(R, T) \
   case R * 4 + T: return cols_r<R, T>(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, tw, st);
     MC_COLS_R(16, 1) MC_COLS_R(16, 2) MC_COLS_R(14, 1) MC_COLS_R(14, 2) MC_COLS_R(12, 1)
