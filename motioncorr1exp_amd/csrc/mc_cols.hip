@@ -396,20 +396,23 @@ __global__ __launch_bounds__(TILES == 1 || R0 <= 8 ? 1024 : 512, TILES == 1 || R
   }
 }
 
-// Resident workgroups of a persistent launch of nt threads with dynamic LDS,
-// asked once per kernel, device and workgroup size.
-template <class K> static int cols_grid(K kernel, int nw, size_t lds, std::atomic<int> (&cache)[16][17]) {
+// Resident workgroups of a persistent launch of nw waves with dynamic LDS, asked
+// once per kernel, device and workgroup size.  The kernel's LDS limit is always
+// set to the most that any size needs: a call with fewer waves does not lower it
+// for a grid that is in the cache.
+template <class K>
+static hipError_t cols_grid(K kernel, int nw, size_t lds, std::atomic<int> (&cache)[16][17], int* grid) {
   int dev = 0;
   (void)hipGetDevice(&dev);
   std::atomic<int>& c = cache[dev >= 0 && dev < 16 ? dev : 0][nw];
-  int g = c.load(std::memory_order_relaxed);
-  if (g <= 0) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    g = persistent_grid(kernel, nw * 64, lds);
-    c.store(g, std::memory_order_relaxed);
-  }
-  return g;
+  *grid = c.load(std::memory_order_relaxed);
+  if (*grid > 0) return hipSuccess;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)COLS_LDS_MAX);
+  if (e != hipSuccess) return e;
+  *grid = persistent_grid(kernel, nw * 64, lds);
+  c.store(*grid, std::memory_order_relaxed);
+  return hipSuccess;
 }
 
 // kx segments of a persistent column-pass launch: about 128 items per
@@ -425,7 +428,9 @@ int col_segments(int npairs, int H, int grid) {
 template <class K, class F>
 static hipError_t cols_launches(K kernel, int nw, size_t lds, std::atomic<int> (&cache)[16][17],
                                 int npairs, int H, F&& launch) {
-  const int grid = cols_grid(kernel, nw, lds, cache);
+  int grid = 0;
+  const hipError_t e = cols_grid(kernel, nw, lds, cache, &grid);
+  if (e != hipSuccess) return e;
   const int S = col_segments(npairs, H, grid);
   for (int s = 0; s < S; s++) {
     const int kxb = H * s / S, nkx = H * (s + 1) / S - kxb;

@@ -83,3 +83,14 @@ def test_many_waves_and_tiles(ctx, n, box):
     worst = float(np.abs(maps[0] - ref).max() / np.abs(ref).max())
     print("n %d box %d: max error / max %.3g" % (n, box, worst), flush=True)
     assert worst < 2e-6
+
+
+def test_more_waves_after_fewer(ctx):
+    """One kernel at eight waves (80 KB of LDS), one wave (10 KB) and eight again:
+    the map of the first call, bit for bit."""
+    got = []
+    for n in (8192, 128, 8192):
+        spec = np.random.default_rng(n).standard_normal((2, n, n + 2), np.float32)
+        ctx.set_spectra(spec)
+        got.append(ctx.pair_shifts(np.array([(0, 1)], np.int32), 150.0, 96, want_boxes=True)[2])
+    assert np.array_equal(got[0], got[2])
