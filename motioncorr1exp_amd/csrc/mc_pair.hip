@@ -486,8 +486,6 @@ hipError_t launch_pair_cols(const float2* spectra, size_t spec_stride, const int
       default: return hipErrorInvalidValue;
     }
   }
-  // boxes above 128 on multiples of 128: at multiples of 256 only, as ever
-  if (box > 128 && n % 128 == 0 && n % 256) return hipErrorInvalidValue;
   return launch_pair_cols_fp32(spectra, spec_stride, pairs, npairs, wxy, n, box, tbuf, st);
 }
 

@@ -94,3 +94,10 @@ def test_more_waves_after_fewer(ctx):
         ctx.set_spectra(spec)
         got.append(ctx.pair_shifts(np.array([(0, 1)], np.int32), 150.0, 96, want_boxes=True)[2])
     assert np.array_equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("n,box", [(384, 129), (384, 200), (1152, 256), (1920, 160)])
+def test_large_boxes_at_odd_multiples_of_128(ctx, n, box):
+    """Boxes above 128 at sizes that are a multiple of 128 and not of 256: the rows
+    start at n/2 - 128, a multiple of 64 there too."""
+    test_box_maps_match_fp64(ctx, n, box)
