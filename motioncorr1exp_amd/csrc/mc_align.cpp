@@ -637,6 +637,16 @@ static int shift_sum(mc_context_s* c, int base, int count, const std::vector<dou
   return MC_OK;
 }
 
+// Waits for the stream unless `done`: on every error return, so that no copy
+// reads host memory that its owner is about to free or to write again.
+struct SyncOnError {
+  hipStream_t st;
+  bool done = false;
+  ~SyncOnError() {
+    if (!done) (void)hipStreamSynchronize(st);
+  }
+};
+
 // Sharpness weights: wk[kx] = a_kx exp(-B kx^2/(2n^2)) (a = 1 at kx = 0 and
 // n/2, else 2), wk[n/2+1+ky] = exp(-B y'^2/(2n^2)).
 static int sharp_weights(mc_context_s* c, int n, float bfactor) {
@@ -652,7 +662,7 @@ static int sharp_weights(mc_context_s* c, int n, float bfactor) {
   }
   HIP_TRY(c->wk.ensure(sizeof(float) * h.size()));
   // (h is written again only after the sharpness_eval that follows has
-  // synchronised the stream)
+  // synchronised the stream, which it does on its error returns too)
   HIP_TRY(hipMemcpyAsync(c->wk.p, h.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice, c->st));
   return MC_OK;
 }
@@ -661,6 +671,7 @@ static int sharp_weights(mc_context_s* c, int n, float bfactor) {
 // `sum`; fs: 2F shifts (NaN: frame out).
 static int sharpness_eval(mc_context_s* c, int base, int F, int sum, const std::vector<double>& fs,
                           double* J, std::vector<double>* grad) {
+  SyncOnError sync{c->st};  // the weights' and the shifts' copies
   HIP_TRY(c->shifts.ensure(sizeof(double) * fs.size()));
   HIP_TRY(c->gpart.ensure(sizeof(double2) * mc::sharp_part_elems(F, c->n)));
   HIP_TRY(c->gout.ensure(sizeof(double2) * (F + 1)));
@@ -672,6 +683,7 @@ static int sharpness_eval(mc_context_s* c, int base, int F, int sum, const std::
                                  slot(c, sum), c->wk.as<float>(), c->gpart.as<double2>(),
                                  c->gout.as<double2>(), c->st));
   }
+  sync.done = true;
   HIP_TRY(hipStreamSynchronize(c->st));
   const double* o = c->gout.as<double>();
   grad->assign(o, o + 2 * F);
