@@ -69,14 +69,18 @@ MC_DEV ValIdx wave_first_max(ValIdx b) {
 // the points of the others (10 to 40 of the 4096 cells for box maps with a
 // peak, up to 100 for noise) are evaluated as in the full search, so the
 // result is the same bit for bit.  1e-10 sum |A| covers the rounding of T and
-// of the points (about 1e-14).  A map without a bound (NaN, infinities) or
-// without structure (constant) keeps all cells (330 us).
+// of the points (about 1e-14).  A map whose points are all zero (a blank frame) or
+// NaN is answered from the bound's sum alone.  A constant map keeps all cells: the
+// points are then evaluated in whole rows, with factors from registers, 100 us
+// against 320 cell by cell (15 maps; the line between the two lies at a quarter of
+// the cells, where both take about as long).
 // 96 x 96 maps: 22 us up to 256 pairs, 37 to 46 for noise; the full search took
 // 51 (40 pairs, four workgroups each and a launch to combine them), 70 (105)
 // and 106 (253).  What is left is latency: one wave issues an instruction in
 // about 6 clocks and no step has work for more than two waves per SIMD.
 constexpr int PEAK_NT = 512, PEAK_CELL = 8, PEAK_NCELL = 512 / PEAK_CELL;
 constexpr int PEAK_ROWS = 14;  // cell rows whose row sums are held at a time
+constexpr int PEAK_FULL = 1024;  // with more cells kept, all points in whole rows
 
 __global__ __launch_bounds__(PEAK_NT) void k_find_peaks(const float* __restrict__ boxmaps, int box,
                                                         int n, int wnoise, double* __restrict__ out) {
@@ -241,10 +245,14 @@ __global__ __launch_bounds__(PEAK_NT) void k_find_peaks(const float* __restrict_
   const int scale = 32;
   const int wns = scale * wnoise;
   const int ox = (box / 2 - offx) * scale, oy = (box / 2 - offy) * scale;
+  const double b2 = rs[0] + rs[1] + rs[2];
+  if (!(b2 > 0)) {  // every point is zero (b2 too), or NaN
+    if (tid == 0) peak_result(p, 0.0, 0x7fffffff, b2, offx, offy, box, n, out);
+    return;
+  }
   double bound[2][4], m0 = -1e300;
   {
     constexpr double h = PEAK_CELL / 2 * 2 * 3.14159265358979323846 / 512;
-    const double b2 = rs[0] + rs[1] + rs[2];
     const int c0 = PEAK_CELL * (l & 15);
 #pragma unroll
     for (int j = 0; j < 2; j++) {
@@ -303,7 +311,26 @@ __global__ __launch_bounds__(PEAK_NT) void k_find_peaks(const float* __restrict_
   __syncthreads();
   // 4. exact evaluation of the kept cells, first maximum
   ValIdx bb = {-1e300, 0x7fffffff};
+  auto row_sum = [&](int q, int kx) {
+    double2 h = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int ky = 0; ky < 16; ky++) {
+      const int yy = ky < 8 ? ky : ky - 16;
+      const double2 t = tw(yy * q);
+      const double2 g = G[ky][kx];
+      h.x += g.x * t.x - g.y * t.y;
+      h.y += g.x * t.y + g.y * t.x;
+    }
+    return h;
+  };
   unsigned long long rows = __ballot(keep[l] != 0);
+  int kept = 0;
+  if (rows == ~0ull) {
+    kept = __popcll(keep[l]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) kept += __shfl_xor(kept, o);
+  }
+  if (kept > PEAK_FULL) rows = 0;  // all points, below
   while (rows) {
     // the next (up to PEAK_ROWS) cell rows: row sums, then wave w takes row w of
     // each cell and 64 lanes the points of eight cells
@@ -314,17 +341,7 @@ __global__ __launch_bounds__(PEAK_NT) void k_find_peaks(const float* __restrict_
       const int s = i / (PEAK_CELL * 9), e = i - s * (PEAK_CELL * 9), dq = e / 9, kx = e - 9 * dq;
       unsigned long long t = todo;
       for (int x = 0; x < s; x++) t &= t - 1;
-      const int q = PEAK_CELL * (__ffsll((long long)t) - 1) - PEAK_CELL / 2 + dq;
-      double2 h = make_double2(0.0, 0.0);
-#pragma unroll
-      for (int ky = 0; ky < 16; ky++) {
-        const int yy = ky < 8 ? ky : ky - 16;
-        const double2 t = tw(yy * q);
-        const double2 g = G[ky][kx];
-        h.x += g.x * t.x - g.y * t.y;
-        h.y += g.x * t.y + g.y * t.x;
-      }
-      Hs[i] = h;
+      Hs[i] = row_sum(PEAK_CELL * (__ffsll((long long)t) - 1) - PEAK_CELL / 2 + dq, kx);
     }
     __syncthreads();
     for (int s = 0; s < nr; s++, todo &= todo - 1) {
@@ -356,6 +373,41 @@ __global__ __launch_bounds__(PEAK_NT) void k_find_peaks(const float* __restrict_
       }
     }
     __syncthreads();
+  }
+  if (kept > PEAK_FULL) {
+    // A thread takes the columns c0 + 128 j, whose factors stay in registers, in
+    // the rows q = tid / 128 mod 4.  (After the loop above: before it, this block
+    // cost the loop 2 us, 35 to 37 on 15 maps of noise.)
+    constexpr int NC = 4, QC = 56;  // a row sum per thread
+    static_assert(QC * 9 <= NT && QC <= PEAK_ROWS * PEAK_CELL && NT == NC * 128, "sums, rows of Hs, classes");
+    const int c0 = tid & 127;
+    double2 wc[NC][8];
+#pragma unroll
+    for (int j = 0; j < NC; j++)
+#pragma unroll
+      for (int kx = 1; kx < 9; kx++) wc[j][kx - 1] = tw(kx * (c0 + 128 * j));
+    for (int q0 = 0; q0 < 512; q0 += QC) {
+      if (tid < QC * 9) Hs[tid] = row_sum(q0 + tid / 9, tid % 9);
+      __syncthreads();
+      for (int qi = w >> 1; qi < min(QC, 512 - q0); qi += NC) {
+        const int q = q0 + qi;
+        const bool rowex = abs(q - oy) <= wns;
+        double2 hq[9];
+#pragma unroll
+        for (int kx = 0; kx < 9; kx++) hq[kx] = Hs[qi * 9 + kx];
+#pragma unroll
+        for (int j = 0; j < NC; j++) {
+          const int pp = c0 + 128 * j;
+          double u = hq[0].x;
+#pragma unroll
+          for (int kx = 1; kx < 9; kx++) u += hq[kx].x * wc[j][kx - 1].x - hq[kx].y * wc[j][kx - 1].y;
+          if (q == 0 && pp == 0) u0s = u;
+          // a thread's points come in row-major order
+          if (!(rowex && abs(pp - ox) <= wns) && u > bb.v) bb = ValIdx{u, q * 512 + pp};
+        }
+      }
+      __syncthreads();
+    }
   }
   bb = wave_first_max(bb);
   if (l == 0) {

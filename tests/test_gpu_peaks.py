@@ -71,3 +71,24 @@ def test_maps_without_a_maximum(ctx, o):
     m[0, 5, 7] = 100.0
     b, cc = ctx.find_peaks(m, N)
     assert (b[0] == -16).all() and np.isnan(cc[0])
+
+
+@pytest.mark.parametrize("wnoise", [-1, 3])
+@pytest.mark.parametrize("box", [16, 96])
+@pytest.mark.parametrize("kind", ["constant", "minus", "stripes", "inf"])
+def test_maps_that_keep_most_cells(ctx, o, kind, box, wnoise):
+    """Maps without a single maximum: every point ties up to rounding (1e-14 of the
+    value), so the value is compared and not the place; one map alone and twelve at
+    once give the same bits."""
+    y, x = np.mgrid[0:box, 0:box]
+    m = {"constant": np.full((box, box), 0.37), "minus": np.full((box, box), -2.5e4),
+         "stripes": np.cos(2 * np.pi * (6 * x + 3 * y) / 16), "inf": np.full((box, box), np.inf)}[kind]
+    m = np.repeat(m.astype(np.float32)[None], 12, axis=0)
+    b, cc = ctx.find_peaks(m, N, wnoise)
+    b1, cc1 = ctx.find_peaks(m[:1], N, wnoise)
+    assert (b == b1).all() and (cc.view(np.int64) == cc1.view(np.int64)).all()
+    if kind == "inf":
+        assert np.isnan(cc).all() and (b == -(box // 2)).all()
+    else:
+        occ = o.find_shift_box(m[0].astype(np.float64), N, wnoise)[2]
+        assert abs(cc[0] - occ) <= 1e-9 * abs(occ)
