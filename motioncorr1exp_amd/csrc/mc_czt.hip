@@ -1,8 +1,9 @@
 // mc_czt.hip -- transforms of the lengths that mc_mixed.hip has no factors for
-// (a prime above 127): Bluestein's chirp-z algorithm on the power-of-two LDS
-// Stockham engine of mc_device.h.  Stage 1 and the sum image at any even size
-// are dispatched here.  The reference plans cuFFT at any size
-// (cufunc.cu:202-215, called for nsamUnbin and nsam, DFAlign.cu:596,838).
+// (a prime above 127) or is slower at (mix_use, mc_mixed_form.h): Bluestein's
+// chirp-z algorithm on the power-of-two LDS Stockham engine of mc_device.h.
+// Stage 1 and the sum image at any even size are dispatched here.  The reference
+// plans cuFFT at any size (cufunc.cu:202-215, called for nsamUnbin and nsam,
+// DFAlign.cu:596,838).
 //
 // A length-L DFT with sign S, X_k = sum_m x_m e^{S 2 pi i m k/L}, is
 //   X_k = c_k sum_m (x_m c_m) h_{k-m},  c_j = e^{S i pi j^2/L}, h = conj(c),
@@ -29,6 +30,7 @@
 #include "mc_device.h"
 #include "mc_frames.h"
 #include "mc_kernels.h"
+#include "mc_mixed_form.h"
 
 namespace mc {
 
@@ -59,12 +61,6 @@ static std::complex<double> chirp(long long j, int L, int S) {
   const long long r = ((j % (2LL * L)) * (j % (2LL * L))) % (2LL * L);
   const double t = S * M_PI * (double)r / (double)L;
   return std::complex<double>(std::cos(t), std::sin(t));
-}
-
-int czt_len(int need) {
-  int M = 64;
-  while (M < need) M <<= 1;
-  return M;
 }
 
 float2* upload_table(const std::vector<float2>& h) {
@@ -606,7 +602,7 @@ hipError_t launch_frames_to_spectra_czt(const R2CGeom& g, int f0, int nframes, f
   const size_t rt_fstride = rt_frame_elems(g.n, g.nu);
   float* rs = g.pad_mode ? rowsum : nullptr;
   hipError_t e = hipErrorInvalidValue;
-  if (mix_size_ok(g.nu / 2)) {
+  if (mix_use(g.nu / 2, (long long)g.h * nframes)) {
     e = launch_rows_mix(g, f0, nframes, nkx, rt, rt_fstride, rs, st);
   } else {
     const BsTab* tr = bs_tables(g.nu / 2, -1);
@@ -625,7 +621,7 @@ hipError_t launch_frames_to_spectra_czt(const R2CGeom& g, int f0, int nframes, f
   }
   e = hipErrorInvalidValue;
   const float* fl = g.pad_mode ? fill : nullptr;
-  if (mix_size_ok(g.nu)) {
+  if (mix_use(g.nu, (long long)nkx * nframes)) {
     e = launch_cols_mix(g, nframes, nkx, rt, rt_fstride, fl, padP, spectra, spec_stride, st);
   } else {
     const BsTab* tc = bs_tables(g.nu, -1);
@@ -694,7 +690,7 @@ hipError_t launch_spectrum_to_image_czt(const float2* spec, int n, float scale, 
                                         size_t img_pitch, float2* tmp, hipStream_t st) {
   if (n < 64 || n > 8192 || n % 2) return hipErrorInvalidValue;
   hipError_t e = hipErrorInvalidValue;
-  if (mix_size_ok(n)) {
+  if (mix_use(n, n / 2 + 1)) {
     e = launch_cols_inv_mix(spec, n, tmp, st);
   } else {
     const BsTab* tc = bs_tables(n, 1);
@@ -706,7 +702,7 @@ hipError_t launch_spectrum_to_image_czt(const float2* spec, int n, float scale, 
     }
   }
   if (e != hipSuccess) return e;
-  if (mix_size_ok(n / 2)) return launch_c2r_rows_mix(tmp, n, scale, img, img_pitch, st);
+  if (mix_use(n / 2, n)) return launch_c2r_rows_mix(tmp, n, scale, img, img_pitch, st);
   const BsTab* tr = bs_tables(n / 2, 1);
   const float2* twn = twiddles(n);
   if (!tr || !twn) return hipErrorOutOfMemory;

@@ -81,16 +81,15 @@ hipError_t launch_fill(const float* rowsum, int nu, int h, int w, float* fill, i
 // Bluestein / chirp-z on power-of-two transforms (mc_czt.hip).  The stage-1
 // and sum-image entry points above dispatch to them by size; the pair
 // column pass computes only the box rows of each column inverse.
-int czt_len(int need);
 hipError_t launch_frames_to_spectra_czt(const R2CGeom& g, int f0, int nframes, float2* spectra,
                                         size_t spec_stride, float2* rt, float* rowsum,
                                         float* fill, const float2* padP, hipStream_t st);
 hipError_t launch_spectrum_to_image_czt(const float2* spec, int n, float scale, float* img,
                                         size_t img_pitch, float2* tmp, hipStream_t st);
-// Transforms of N = P Q with both factors in 7..127 (mc_mixed.hip).
+// Transforms of two to four factors in 2..127 (mc_mixed.hip), where mix_use
+// (mc_mixed_form.h) says so.
 float2* upload_table(const std::vector<float2>& h);  // device copy, nullptr on failure
 const float2* qp_twiddles(int Q, int P);  // e^{-2 pi i a k2/(Q P)} at k2 Q + a, a < Q, k2 < P
-bool mix_size_ok(int N);
 hipError_t launch_rows_mix(const R2CGeom& g, int f0, int nframes, int nkx, float2* rt,
                              size_t rt_fstride, float* rowsum, hipStream_t st);
 hipError_t launch_cols_mix(const R2CGeom& g, int nframes, int nkx, const float2* rt,

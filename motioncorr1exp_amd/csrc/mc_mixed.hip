@@ -30,11 +30,11 @@
 
 #include <algorithm>
 #include <cmath>
-#include <functional>
 
 #include "mc_device.h"
 #include "mc_frames.h"
 #include "mc_kernels.h"
+#include "mc_mixed_form.h"
 
 namespace mc {
 
@@ -516,39 +516,6 @@ __global__ __launch_bounds__(512, 4) void k_c2r_rows_mix(const float2* __restric
 }
 
 // ---------------------------------------------------------------- host part
-// Estimated clocks per element and SIMD of a level (issue of the vector ALU and
-// the matrix unit; measured sums of the parts).
-static double mix_cost(int F) {
-  static const double regs[17] = {0, 0, 11, 14, 13, 17, 16, 19, 16, 20, 19, 24, 18, 27, 21, 21, 18};
-  if (F <= 16) return regs[F] * 4 / 64;
-  const int mt = (F / 2 + 16) / 16, ks = (F / 2 + 4) / 4;
-  return (mt * ks * 128 + ks * 88 + mt * 400) / (16.0 * F);
-}
-
-// Cheapest factors of N in 2..127, two to four; 0: none.
-static int mix_factors(int N, int* F) {
-  double best = 1e30;
-  int m = 0, f[4];
-  std::function<void(int, int, int, double)> rec = [&](int rest, int lo, int i, double c) {
-    if (c >= best) return;
-    if (rest == 1) {
-      if (i < 2) return;
-      best = c;
-      m = i;
-      std::copy(f, f + i, F);
-      return;
-    }
-    if (i == 4) return;
-    for (int x = lo; x <= 127 && x <= rest; x++) {
-      if (rest % x) continue;
-      f[i] = x;
-      rec(rest / x, x, i + 1, c + mix_cost(x));
-    }
-  };
-  rec(N, 2, 0, 0.0);
-  return m;
-}
-
 // Plan of a transform of N elements for `items` of them.  The largest factor
 // goes first (its factors w_N are the long table), an even one last (padded to
 // odd distances), so that an odd product between them keeps the last level's
@@ -557,11 +524,10 @@ static int mix_factors(int N, int* F) {
 // with the first, 240 and 169 with the second; 4092: 161 and 133, 152 and 123;
 // other sizes of the workgroup leave the CU with fewer than 16 waves: 30 to 50%
 // slower), fewer items if that leaves less than two workgroups per CU.
-static bool mix_plan(int N, long long items, MixPlan* d, bool tables) {
+static bool mix_plan(int N, long long items, MixPlan* d) {
   int F[4];
   const int m = mix_factors(N, F);  // ascending
   if (!m) return false;
-  if (!tables) return true;
   std::reverse(F, F + m);
   for (int i = 1; i + 1 < m; i++)
     if (F[i] % 2 == 0 && F[m - 1] % 2) std::swap(F[i], F[m - 1]);
@@ -607,11 +573,6 @@ static bool mix_plan(int N, long long items, MixPlan* d, bool tables) {
   return true;
 }
 
-bool mix_size_ok(int N) {
-  MixPlan d;
-  return mix_plan(N, 1, &d, false);
-}
-
 template <class K, class... Args>
 static hipError_t mix_launch(K kernel, const MixPlan& d, int groups, hipStream_t st, Args... args) {
   if (d.lds > 64 * 1024) {
@@ -628,7 +589,7 @@ hipError_t launch_rows_mix(const R2CGeom& g, int f0, int nframes, int nkx, float
                            size_t rt_fstride, float* rowsum, hipStream_t st) {
   MixPlan d;
   const float2* twnu = twiddles(g.nu);
-  if (!mix_plan(g.nu / 2, (long long)g.h * nframes, &d, true) || !twnu) return hipErrorOutOfMemory;
+  if (!mix_plan(g.nu / 2, (long long)g.h * nframes, &d) || !twnu) return hipErrorOutOfMemory;
   return mix_launch(k_r2c_rows_mix, d, mix_groups(d, g.h) * nframes, st, g, d, f0, nkx, rt, rt_fstride,
                     rowsum, twnu);
 }
@@ -637,14 +598,14 @@ hipError_t launch_cols_mix(const R2CGeom& g, int nframes, int nkx, const float2*
                            size_t rt_fstride, const float* fill, const float2* padP,
                            float2* spectra, size_t spec_stride, hipStream_t st) {
   MixPlan d;
-  if (!mix_plan(g.nu, (long long)nkx * nframes, &d, true)) return hipErrorOutOfMemory;
+  if (!mix_plan(g.nu, (long long)nkx * nframes, &d)) return hipErrorOutOfMemory;
   return mix_launch(k_c2c_cols_mix, d, mix_groups(d, nkx) * nframes, st, rt, rt_fstride, d, nkx, g.h,
                     fill, padP, g.n, spectra, spec_stride);
 }
 
 hipError_t launch_cols_inv_mix(const float2* spec, int n, float2* tmp, hipStream_t st) {
   MixPlan d;
-  if (!mix_plan(n, n / 2 + 1, &d, true)) return hipErrorOutOfMemory;
+  if (!mix_plan(n, n / 2 + 1, &d)) return hipErrorOutOfMemory;
   return mix_launch(k_cols_inv_mix, d, mix_groups(d, n / 2 + 1), st, spec, d, tmp);
 }
 
@@ -652,7 +613,7 @@ hipError_t launch_c2r_rows_mix(const float2* tmp, int n, float scale, float* img
                                hipStream_t st) {
   MixPlan d;
   const float2* twn = twiddles(n);
-  if (!mix_plan(n / 2, n, &d, true) || !twn) return hipErrorOutOfMemory;
+  if (!mix_plan(n / 2, n, &d) || !twn) return hipErrorOutOfMemory;
   return mix_launch(k_c2r_rows_mix, d, mix_groups(d, n), st, tmp, d, scale, img, pitch, twn);
 }
 

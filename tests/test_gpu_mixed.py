@@ -90,3 +90,21 @@ def test_corrected_frames_of_every_type(dtype, nx, ny, kw, nu, n):
     err = np.abs(spec - ref).max() / np.abs(ref).max()
     print("%s %s: %.3g" % (np.dtype(dtype).name, kw, err), flush=True)
     assert err <= 1e-6
+
+
+@pytest.mark.parametrize("n,F", [(142, 2), (142, 32), (402, 2), (402, 10), (762, 2), (762, 5), (1010, 3)])
+def test_frames_on_both_sides_of_the_choice(n, F):
+    """Sizes with a large factor, which few frames take through the chirp-z
+    transform and many through mixed factors (mc_mixed_form.h)."""
+    rng = np.random.default_rng(n + F)
+    img = rng.standard_normal((F, n, n), np.float32)
+    c = mc.Context(0)
+    d = mc.DeviceArray(img)
+    c.load_frames(d, img.shape, np.float32, mc.default_params(F))
+    got = np.asarray(c.get_spectra(F, n)).view(np.complex64).reshape(F, n, n // 2 + 1)
+    c.close()
+    d.free()
+    ref = np.fft.rfft2(img.astype(np.float64))
+    err = np.abs(got - ref).max() / np.abs(ref).max()
+    print("n %d, %d frames: %.3g" % (n, F, err), flush=True)
+    assert err <= 1e-6
