@@ -564,8 +564,7 @@ def main():
 
     if not args.no_refgeom:
         # the reference's default geometry: square crop min(nx, ny) = 3710 =
-        # 2*5*7*53, no padding (stage 1 in two levels, 35 x 53 rows and 70 x 53
-        # columns; chirp-z for the image)
+        # 2*5*7*53, no padding (mixed-factor transforms)
         pr = dict(params, pad=0)
         step(pr)
         mc.check(L.mc_sync())

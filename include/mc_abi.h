@@ -73,9 +73,9 @@ int mc_mem_bin_d2d(float *dst, const float *src, int dst_n, int src_n);
 int mc_mem_bin_d2h(float *dst_host, const float *src, int dst_n, int src_n);
 /* GPUFFTPlan / GPUIFFTPlan (cufunc.cu:202-215): n x n in-place plans.
  * Supported n: any even size from 64 to 8192 (Stockham plans for powers of
- * two and 2^k * 3, 5 or 15; chirp-z transforms for the others, except the
- * forward transforms at 3710 and 4092, which run in two levels: 35 x 53 and
- * 70 x 53, 66 x 31 and 132 x 31). */
+ * two and 2^k * 3, 5 or 15; the others in mixed factors, or as chirp-z
+ * transforms where a prime factor exceeds 127 or a short transform has a large
+ * one). */
 int mc_fft_plan(mc_plan *plan, int n);
 int mc_ifft_plan(mc_plan *plan, int n);
 /* GPUFFT2d / GPUIFFT2d (cufunc.cu:223-233): unnormalised, in place. */
@@ -112,7 +112,7 @@ int mc_find_shift(const float *dsrc, int n, float *hboxmap, int box, float *sx, 
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): same arguments and results, but the box
  * copy and the peak record live in a fixed device array of the library
- * (MC_NOALLOC_MAX_BOX^2 floats + 256 bytes, one per GPU, held until the
+ * (MC_NOALLOC_MAX_BOX^2 floats + 24 bytes, one per GPU, held until the
  * process ends) and the call makes no allocation.  box > MC_NOALLOC_MAX_BOX
  * returns MC_ERR_ARG.  All calls on one GPU share the array: calls that
  * overlap on one GPU (several host threads) race. */

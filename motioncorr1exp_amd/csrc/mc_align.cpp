@@ -121,7 +121,7 @@ struct mc_context_s {
   // autotuned launch shapes (mc_autotune / mc_tune_load)
   struct Tune {
     int nu, n, dtype, box, precision;
-    int r2c, chunk, cols, rows;
+    int r2c, chunk;
   };
   std::vector<Tune> tunes;
   // resident spectra
@@ -481,12 +481,6 @@ static const mc_context_s::Tune* stage1_tune(const mc_context_s* c, int nu, int 
   return nullptr;
 }
 
-static const mc_context_s::Tune* pair_tune(const mc_context_s* c, int n, int box, int precision) {
-  for (const auto& t : c->tunes)
-    if (t.n == n && t.box == box && t.precision == precision) return &t;
-  return nullptr;
-}
-
 // Stage 1 for frames [first, first+count) of a buffer into slots [s0, ...).
 // variant / chunk < 0: the tuned shape for this geometry, else the default.
 static int run_stage1(mc_context_s* c, const void* frames, const mc_movie_desc* m,
@@ -569,7 +563,7 @@ static int load_frames(mc_context_s* c, const mc_movie_desc* m, const mc_params*
 }
 
 // Pair-stage buffers for np pairs (before any launch, outside graph capture).
-static int pair_reserve(mc_context_s* c, int np, int n, int box, int precision) {
+static int pair_reserve(mc_context_s* c, int np, int n, int box) {
   const int H = n / 2 + 1;
   HIP_TRY(c->pairs_d.ensure(sizeof(int) * 2 * (size_t)np));
   HIP_TRY(c->tbuf.ensure(sizeof(float2) * (size_t)np * H * box));
@@ -584,13 +578,10 @@ static int pair_reserve(mc_context_s* c, int np, int n, int box, int precision) 
 // Capturable.
 static int pair_launch(mc_context_s* c, int np, int n, float bfactor, int box, int wnoise,
                        int precision) {
-  const mc_context_s::Tune* tn = pair_tune(c, n, box, precision);
-  const int cols = tn ? tn->cols : mc::PAIR_COLS_AUTO;
   {
     KScope ks(c, MC_KT_PAIR_COLS);
     HIP_TRY(mc::launch_pair_cols(slot(c, 0), c->spec_stride, c->pairs_d.as<int2>(), np, n, bfactor,
-                                 box, c->tbuf.as<float2>(), precision, cols,
-                                 c->st));
+                                 box, c->tbuf.as<float2>(), precision, c->st));
   }
   {
     KScope ks(c, MC_KT_PAIR_ROWS);
@@ -610,7 +601,7 @@ static int pair_stage(mc_context_s* c, const std::vector<int>& slots, float bfac
                       int wnoise, int precision, std::vector<double>& res, float* boxmaps_host) {
   const int np = (int)slots.size() / 2;
   const int n = c->n;
-  MC_TRY(pair_reserve(c, np, n, box, precision));
+  MC_TRY(pair_reserve(c, np, n, box));
   HIP_TRY(hipMemcpyAsync(c->pairs_d.p, slots.data(), sizeof(int) * slots.size(),
                          hipMemcpyHostToDevice, c->st));
   MC_TRY(pair_launch(c, np, n, bfactor, box, wnoise, precision));
@@ -1242,7 +1233,6 @@ static void use_group(mc_context_s* c, const SizeGroup& g) {
 struct PairSpan {
   int gi = 0, np = 0;
   size_t po = 0, to = 0;
-  int cols = mc::PAIR_COLS_AUTO;
 };
 struct PairPlan {
   std::vector<PairSpan> sp;
@@ -1263,12 +1253,9 @@ static int pairs_prepare(mc_context_s* c, const std::vector<SizeGroup>& gs, Pair
     np += q.np;
     tel += (size_t)q.np * (n / 2 + 1) * L.box;
     gnp[q.gi] += q.np;
-    const mc_context_s::Tune* tn = pair_tune(c, n, L.box, L.precision);
-    q.cols = tn ? tn->cols : mc::PAIR_COLS_AUTO;
   }
-  for (size_t g = 0; g < gs.size(); g++) {
+  for (size_t g = 0; g < gs.size(); g++)
     part = std::max(part, mc::pair_rows_part_elems((int)gnp[g], gs[g].n, L.box));
-  }
   if (slots.size() != 2 * np) return set_err(MC_ERR_ARG, "pair spans cover %zu of %zu pairs", np, slots.size() / 2);
   L.np = np;
   HIP_TRY(c->pairs_d.ensure(sizeof(int) * 2 * std::max<size_t>(1, np)));
@@ -1281,8 +1268,8 @@ static int pairs_prepare(mc_context_s* c, const std::vector<SizeGroup>& gs, Pair
   return MC_OK;
 }
 
-// Column pass per span, then the row pass and the peak search per size group.  Results: peaks (3 doubles per pair, span
-// order) and box maps.  Capturable.
+// Column pass per span, then the row pass and the peak search per size group.
+// Results: peaks (3 doubles per pair, span order) and box maps.  Capturable.
 static int pairs_launch(mc_context_s* c, const std::vector<SizeGroup>& gs, const PairPlan& L) {
   const int box = L.box;
   {
@@ -1292,7 +1279,7 @@ static int pairs_launch(mc_context_s* c, const std::vector<SizeGroup>& gs, const
       const SizeGroup& g = gs[q.gi];
       HIP_TRY(mc::launch_pair_cols(c->spec.as<float2>() + g.off, g.stride,
                                    c->pairs_d.as<int2>() + q.po, q.np, g.n, L.bfactor, box,
-                                   c->tbuf.as<float2>() + q.to, L.precision, q.cols, c->st));
+                                   c->tbuf.as<float2>() + q.to, L.precision, c->st));
     }
   }
   // consecutive spans of one size group share a row-pass and a peak launch
@@ -1323,7 +1310,8 @@ static int pairs_launch(mc_context_s* c, const std::vector<SizeGroup>& gs, const
 // Graph of one align-to-sum round of a set of movies: the batched sums, the
 // pair column/row passes and the peak search, replayed while the set of
 // iterating movies is unchanged.  Only kernel launches are captured: the
-// shifts are uploaded and the peaks read back around each replay.
+// shifts are uploaded before each replay, and its kernels write the peaks to
+// pinned host memory.
 struct RoundGraph {
   hipGraphExec_t exec = nullptr;
   std::vector<int> key;
@@ -1394,9 +1382,9 @@ struct GroupTimes {
 // of any transform sizes, whose spectra fit together in device memory
 // (callers order them by size): stage 1 per movie into its size group's
 // region, then one pair stage over every pair of every movie (the column
-// pass per movie, row pass and peak search per size), the host drift model per movie, align-to-sum rounds over
-// the movies still iterating (one graph replay per round), and the final sum
-// per movie.
+// pass per movie, row pass and peak search per size), the host drift model per
+// movie, align-to-sum rounds over the movies still iterating (one graph replay
+// per round), and the final sum per movie.
 static int align_group(mc_context_s* c, std::vector<MovieRun*>& rs, bool use_graph,
                        GroupTimes* tm) {
   const int box = rs[0]->box, wnoise = rs[0]->wnoise;
@@ -1906,20 +1894,19 @@ extern "C" int mc_autotune(mc_context ctx, const mc_movie_desc* m, const mc_para
   }
   // ---- pair stage (spectra of the last stage-1 run are resident)
   std::vector<int> slots(r.pairs);
-  MC_TRY(pair_reserve(c, r.P, n, box, p->precision));
+  MC_TRY(pair_reserve(c, r.P, n, box));
   HIP_TRY(hipMemcpyAsync(c->pairs_d.p, slots.data(), sizeof(int) * slots.size(),
                          hipMemcpyHostToDevice, c->st));
-  const int bcol = mc::PAIR_COLS_AUTO, brow = mc::PAIR_ROWS_AUTO;
   if (p->precision == MC_PREC_FP32) {
     {  // one column and one row kernel per size: their times are reported
       float ms = 0;
       MC_TRY(time_min(c, reps, &ms, [&] {
         const hipError_t e = mc::launch_pair_cols(slot(c, 0), c->spec_stride,
                                                   c->pairs_d.as<int2>(), r.P, n, p->bfactor, box,
-                                                  c->tbuf.as<float2>(), p->precision, bcol, c->st);
+                                                  c->tbuf.as<float2>(), p->precision, c->st);
         return e == hipSuccess ? MC_OK : set_err(MC_ERR_DEVICE, "pair columns: %s", hipGetErrorString(e));
       }));
-      tr.ms_pair_cols[bcol] = ms;
+      tr.ms_pair_cols[0] = ms;
     }
     {
       float ms = 0;
@@ -1928,16 +1915,14 @@ extern "C" int mc_autotune(mc_context ctx, const mc_movie_desc* m, const mc_para
                                                   c->box.as<float>(), c->boxpart.as<float>(), c->st);
         return e == hipSuccess ? MC_OK : set_err(MC_ERR_DEVICE, "pair rows: %s", hipGetErrorString(e));
       }));
-      tr.ms_pair_rows[brow] = ms;
+      tr.ms_pair_rows[0] = ms;
     }
   }
   HIP_TRY(hipStreamSynchronize(c->st));
-  mc_context_s::Tune t{r.g.nsu, n, m->dtype, box, p->precision, bv, bc, bcol, brow};
+  mc_context_s::Tune t{r.g.nsu, n, m->dtype, box, p->precision, bv, bc};
   set_tune(c, t);
   tr.r2c_variant = bv;
   tr.chunk_frames = bc;
-  tr.pair_cols_variant = bcol;
-  tr.pair_rows_variant = brow;
   if (rep) *rep = tr;
   if (cache_path && *cache_path) {
     char arch[64];
@@ -1947,8 +1932,8 @@ extern "C" int mc_autotune(mc_context ctx, const mc_movie_desc* m, const mc_para
     if (!fp) return set_err(MC_ERR_IO, "cannot append to %s", cache_path);
     fprintf(fp,
             "{\"arch\": \"%s\", \"cus\": %d, \"nu\": %d, \"n\": %d, \"dtype\": %d, \"box\": %d, "
-            "\"precision\": %d, \"r2c\": %d, \"chunk\": %d, \"cols\": %d, \"rows\": %d}\n",
-            arch, cus, t.nu, t.n, t.dtype, t.box, t.precision, t.r2c, t.chunk, t.cols, t.rows);
+            "\"precision\": %d, \"r2c\": %d, \"chunk\": %d, \"cols\": 0, \"rows\": 0}\n",
+            arch, cus, t.nu, t.n, t.dtype, t.box, t.precision, t.r2c, t.chunk);
     fclose(fp);
   }
   return MC_OK;
@@ -1973,17 +1958,16 @@ extern "C" int mc_tune_load(mc_context ctx, const char* cache_path, int* loaded)
   int cnt = 0;
   while (fgets(line, sizeof line, fp)) {
     mc_context_s::Tune t;
-    int lc = 0;
+    int lc = 0, cols = 0, rows = 0;  // cols, rows: codes of former pair kernels, 0 to 3
     if (!strstr(line, want) || !json_int(line, "cus", &lc) || lc != cus) continue;
     if (json_int(line, "nu", &t.nu) && json_int(line, "n", &t.n) &&
         json_int(line, "dtype", &t.dtype) && json_int(line, "box", &t.box) &&
         json_int(line, "precision", &t.precision) && json_int(line, "r2c", &t.r2c) &&
-        json_int(line, "chunk", &t.chunk) && json_int(line, "cols", &t.cols) &&
-        json_int(line, "rows", &t.rows) && t.r2c >= 0 &&
+        json_int(line, "chunk", &t.chunk) && json_int(line, "cols", &cols) &&
+        json_int(line, "rows", &rows) && t.r2c >= 0 &&
         (t.r2c & (mc::R2C_COLS_P - 1)) < mc::R2C_VARIANTS &&
         (t.r2c >> mc::R2C_CPLAN_SHIFT) < mc::R2C_CPLANS &&
-        t.cols >= 0 && t.cols < mc::PAIR_COLS_VARIANTS && t.rows >= 0 &&
-        t.rows < mc::PAIR_ROWS_VARIANTS && t.chunk >= 0) {
+        cols >= 0 && cols < 4 && rows >= 0 && rows < 4 && t.chunk >= 0) {
       set_tune(ctx, t);  // later lines win
       cnt++;
     }

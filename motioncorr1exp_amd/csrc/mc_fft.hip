@@ -496,7 +496,7 @@ hipError_t launch_frames_to_spectra(const R2CGeom& g, int f0, int nframes, float
     MC_F2S(768) MC_F2S(1536) MC_F2S(3072) MC_F2S(6144)
     MC_F2S(1280) MC_F2S(2560) MC_F2S(5120) MC_F2S(1920) MC_F2S(3840)
 #undef MC_F2S
-    default:  // any other even size: chirp-z transforms (mc_czt.hip)
+    default:  // any other even size: mixed factors or chirp-z (mc_czt.hip)
       return launch_frames_to_spectra_czt(g, f0, nframes, spectra, spec_stride, rt, rowsum, fill,
                                           padP, st);
   }
@@ -639,7 +639,7 @@ hipError_t launch_spectrum_to_image(const float2* spec, int n, float scale, floa
     case 5120: return spectrum_to_image_t<5120>(spec, scale, img, img_pitch, tmp, st);
     case 1920: return spectrum_to_image_t<1920>(spec, scale, img, img_pitch, tmp, st);
     case 3840: return spectrum_to_image_t<3840>(spec, scale, img, img_pitch, tmp, st);
-    default:  // any other even size: chirp-z transforms (mc_czt.hip)
+    default:  // any other even size: mixed factors or chirp-z (mc_czt.hip)
       return launch_spectrum_to_image_czt(spec, n, scale, img, img_pitch, tmp, st);
   }
 }

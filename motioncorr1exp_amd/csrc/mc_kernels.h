@@ -77,10 +77,10 @@ hipError_t launch_frames_to_spectra(const R2CGeom& g, int f0, int nframes, float
 hipError_t launch_fill(const float* rowsum, int nu, int h, int w, float* fill, int nframes,
                        hipStream_t st);
 
-// Transforms of sizes without a Stockham plan (any even size in [64, 8192]):
-// Bluestein / chirp-z on power-of-two transforms (mc_czt.hip).  The stage-1
-// and sum-image entry points above dispatch to them by size; the pair
-// column pass computes only the box rows of each column inverse.
+// Transforms of sizes without a Stockham plan (any even size in [64, 8192]): in
+// mixed factors (mc_mixed.hip) or Bluestein / chirp-z on power-of-two transforms
+// (mc_czt.hip).  The stage-1 and sum-image entry points above dispatch to them by
+// size; the pair column pass computes only the box rows of each column inverse.
 hipError_t launch_frames_to_spectra_czt(const R2CGeom& g, int f0, int nframes, float2* spectra,
                                         size_t spec_stride, float2* rt, float* rowsum,
                                         float* fill, const float2* padP, hipStream_t st);
@@ -112,16 +112,13 @@ hipError_t launch_spectrum_to_image(const float2* spec, int n, float scale, floa
 // C[p][r][c] (row pass).  pairs: device int2 (a, b) indices into `spectra`
 // (frame slots of stride spec_stride); operand a is kept, b conjugated.
 // precision 0: FP32; 1: the first DFT stage of the column pass as FP16 hi/lo MFMA
-// products.  Each pass has one kernel per size (`variant` is one of the codes
-// that tuning files may hold; all run it).  The row pass splits the kx range over
-// workgroups, a count set by n alone, whose partial maps go to `part`
+// products.  Each pass has one kernel per size.  The row pass splits the kx range
+// over workgroups, a count set by n alone, whose partial maps go to `part`
 // (pair_rows_part_elems(npairs, n, box) floats) and are added in order.
-enum { PAIR_COLS_AUTO = 0, PAIR_COLS_VARIANTS = 4 };
-enum { PAIR_ROWS_AUTO = 0, PAIR_ROWS_VARIANTS = 4 };
 bool pair_form_supported(int precision, int n, int box);
 hipError_t launch_pair_cols(const float2* spectra, size_t spec_stride, const int2* pairs,
                             int npairs, int n, float bfactor, int box, float2* tbuf,
-                            int precision, int variant, hipStream_t st);
+                            int precision, hipStream_t st);
 // The FP32 column pass (mc_cols.hip; wxy: the weight table of mc_pair.hip), and
 // the kx segments of a persistent column-pass launch sequence.
 hipError_t launch_pair_cols_fp32(const float2* spectra, size_t spec_stride, const int2* pairs,

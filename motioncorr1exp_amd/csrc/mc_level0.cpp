@@ -32,7 +32,7 @@ static int l0_err(int code, const char* what, hipError_t e) {
   } while (0)
 
 // Any even size in [64, 8192]: Stockham plans for powers of two and
-// 2^k * {3, 5, 15}, chirp-z transforms otherwise.
+// 2^k * {3, 5, 15}, mixed factors or chirp-z transforms otherwise.
 static bool size_ok(int n) { return n >= 64 && n <= 8192 && n % 2 == 0; }
 
 struct mc_plan_s {

@@ -469,7 +469,7 @@ bool pair_form_supported(int precision, int n, int box) {
 
 hipError_t launch_pair_cols(const float2* spectra, size_t spec_stride, const int2* pairs,
                             int npairs, int n, float bfactor, int box, float2* tbuf,
-                            int precision, int variant, hipStream_t st) {
+                            int precision, hipStream_t st) {
   if (npairs <= 0) return hipSuccess;
   if (!pair_form_supported(precision, n, box)) return hipErrorInvalidValue;
   const float* wxy = weights(n, bfactor);

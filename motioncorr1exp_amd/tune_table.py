@@ -6,7 +6,7 @@ read back by mc_tune_load / Context.tune_load).
 Each geometry is tuned by mc_autotune on a synthetic movie of its shape
 generated in device memory (random-wave phantom, Poisson counts).  The
 default list covers the benchmark workloads: 3838x3710x40 float32 padded to
-4096 and at its default square crop (n = 3710, chirp-z stage 1); 4096x4096x24
+4096 and at its default square crop (n = 3710, mixed-factor stage 1); 4096x4096x24
 uint8 with 2x binning; uint8 movies padded to every
 canvas size of the batched form (1024 ... 4096); 512x512x10 float32.
 """
