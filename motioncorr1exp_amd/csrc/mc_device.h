@@ -405,10 +405,8 @@ MC_DEV void odd_dft(float2 (&x)[P], OUT&& out) {
 }
 
 // ---------------------------------------------------- Stockham stage plans
-// Lengths N = 2^k * m, m a product of distinct factors 3, 5, 7 and 11 (k = 0
-// included: no power-of-two stage).
-// Power-of-two plans are balanced; the odd factors add a radix-3, radix-5,
-// radix-7 and/or radix-11 stage after the plan of 2^k.
+// Lengths N = 2^k * m, m = 1, 3, 5 or 15.  Power-of-two plans are balanced; the
+// odd factors add a radix-3 and/or a radix-5 stage after the plan of 2^k.
 __host__ __device__ constexpr int ilog2c(int n) { return n <= 1 ? 0 : 1 + ilog2c(n / 2); }
 __host__ __device__ constexpr bool is_pow2c(int n) { return n > 0 && (n & (n - 1)) == 0; }
 __host__ __device__ constexpr int pow2_stage_count(int N) {
@@ -446,7 +444,7 @@ __host__ __device__ constexpr int r8_stage_radix(int N, int s) {
        : 8;
 }
 __host__ __device__ constexpr int plan_p2_count(int N, int P) {
-  return N == 1 ? 0 : P == 2 ? r8_stage_count(N) : pow2_stage_count(N);
+  return P == 2 ? r8_stage_count(N) : pow2_stage_count(N);
 }
 __host__ __device__ constexpr int plan_p2_radix(int N, int s, int P) {
   return P == 2 ? r8_stage_radix(N, s)
@@ -455,33 +453,19 @@ __host__ __device__ constexpr int plan_p2_radix(int N, int s, int P) {
 }
 __host__ __device__ constexpr int odd_part(int N) { return N % 2 ? N : odd_part(N / 2); }
 // Stages of a length N = 2^k * m under plan P: the power-of-two stages, then
-// one stage per odd factor of m, in the order 3, 5, 7, 11.
-__host__ __device__ constexpr int odd_factor(int k) {
-  return k == 0 ? 3 : (k == 1 ? 5 : (k == 2 ? 7 : 11));
-}
-__host__ __device__ constexpr int odd_radix_from(int m, int i, int k) {
-  return k > 3 ? 11
-       : m % odd_factor(k) != 0 ? odd_radix_from(m, i, k + 1)
-       : i == 0 ? odd_factor(k)
-                : odd_radix_from(m, i - 1, k + 1);
-}
-// the i-th of the factors 3, 5, 7, 11 that divide m
-__host__ __device__ constexpr int odd_radix(int m, int i) { return odd_radix_from(m, i, 0); }
+// one stage per odd factor of m, in the order 3, 5.
+__host__ __device__ constexpr int odd_radix(int m, int i) { return i == 0 && m % 3 == 0 ? 3 : 5; }
 __host__ __device__ constexpr int stage_count(int N, int P = 0) {
   return plan_p2_count(N / odd_part(N), P) + (odd_part(N) % 3 == 0 ? 1 : 0) +
-         (odd_part(N) % 5 == 0 ? 1 : 0) + (odd_part(N) % 7 == 0 ? 1 : 0) +
-         (odd_part(N) % 11 == 0 ? 1 : 0);
+         (odd_part(N) % 5 == 0 ? 1 : 0);
 }
 __host__ __device__ constexpr int stage_radix(int N, int s, int P = 0) {
   return s < plan_p2_count(N / odd_part(N), P)
              ? plan_p2_radix(N / odd_part(N), s, P)
              : odd_radix(odd_part(N), s - plan_p2_count(N / odd_part(N), P));
 }
-static_assert(stage_radix(70, 0) == 2 && stage_radix(70, 1) == 5 && stage_radix(70, 2) == 7 &&
-                  stage_radix(3840, 2) == 3 && stage_radix(3840, 3) == 5 &&
-                  stage_count(132) == 3 && stage_radix(132, 0) == 4 &&
-                  stage_radix(132, 1) == 3 && stage_radix(132, 2) == 11 &&
-                  stage_count(35) == 2 && stage_radix(35, 0) == 5 && stage_radix(35, 1) == 7,
+static_assert(stage_count(3840) == 4 && stage_radix(3840, 2) == 3 && stage_radix(3840, 3) == 5 &&
+                  stage_radix(1280, 2) == 5 && stage_radix(768, 2) == 3,
               "stage plans");
 // Table index modulo the table size (any size; a power of two masks).
 MC_DEV int tw_mod(int e, int ntw) { return (ntw & (ntw - 1)) == 0 ? (e & (ntw - 1)) : (e % ntw); }
