@@ -602,7 +602,7 @@ hipError_t launch_frames_to_spectra_czt(const R2CGeom& g, int f0, int nframes, f
   const size_t rt_fstride = rt_frame_elems(g.n, g.nu);
   float* rs = g.pad_mode ? rowsum : nullptr;
   hipError_t e = hipErrorInvalidValue;
-  if (mix_use(g.nu / 2, (long long)g.h * nframes)) {
+  if (mix_use(g.nu / 2, (long long)g.h * nframes, true)) {
     e = launch_rows_mix(g, f0, nframes, nkx, rt, rt_fstride, rs, st);
   } else {
     const BsTab* tr = bs_tables(g.nu / 2, -1);
@@ -621,7 +621,7 @@ hipError_t launch_frames_to_spectra_czt(const R2CGeom& g, int f0, int nframes, f
   }
   e = hipErrorInvalidValue;
   const float* fl = g.pad_mode ? fill : nullptr;
-  if (mix_use(g.nu, (long long)nkx * nframes)) {
+  if (mix_use(g.nu, (long long)nkx * nframes, true)) {
     e = launch_cols_mix(g, nframes, nkx, rt, rt_fstride, fl, padP, spectra, spec_stride, st);
   } else {
     const BsTab* tc = bs_tables(g.nu, -1);
@@ -690,7 +690,7 @@ hipError_t launch_spectrum_to_image_czt(const float2* spec, int n, float scale, 
                                         size_t img_pitch, float2* tmp, hipStream_t st) {
   if (n < 64 || n > 8192 || n % 2) return hipErrorInvalidValue;
   hipError_t e = hipErrorInvalidValue;
-  if (mix_use(n, n / 2 + 1)) {
+  if (mix_use(n, n / 2 + 1, false)) {
     e = launch_cols_inv_mix(spec, n, tmp, st);
   } else {
     const BsTab* tc = bs_tables(n, 1);
@@ -702,7 +702,7 @@ hipError_t launch_spectrum_to_image_czt(const float2* spec, int n, float scale, 
     }
   }
   if (e != hipSuccess) return e;
-  if (mix_use(n / 2, n)) return launch_c2r_rows_mix(tmp, n, scale, img, img_pitch, st);
+  if (mix_use(n / 2, n, false)) return launch_c2r_rows_mix(tmp, n, scale, img, img_pitch, st);
   const BsTab* tr = bs_tables(n / 2, 1);
   const float2* twn = twiddles(n);
   if (!tr || !twn) return hipErrorOutOfMemory;

@@ -61,17 +61,23 @@ inline int mix_factors(int N, int* F) {
 // longer of the two grows with its length M: 17 up to M = 512, 41 at 1024, 97 at
 // 2048 (1010 = 101 x 10, columns 12.8 against 11.4; 890 = 89 x 10, 10.7 against
 // 11.0), none above (1090 = 109 x 10: the whole transform 52 us against 61).  It
-// needs the whole chip from about 1800, 1600 and 800 transforms on (24 frames of
-// 762: stage 1 163 us against 224).  At M = 512 a factor of 97 or more is slower at
-// any count (254, 32 frames: 18.5 against 15.0).
-inline bool mix_use(int N, long long items) {
+// fills the chip at about 1400, 2000, 1600 and 800 transforms of M = 256, 512, 1024
+// and 2048, from where on its time steps up (24 frames of 762: stage 1 224 us
+// against 163).  At M = 512 a factor of 97 or more is slower at
+// any count (254, 32 frames: 18.5 against 15.0).  Factors up to 16 are the slower of
+// the two only at M = 512, up to 1000 transforms and forward (rows of 416 x 416
+// images, 16 x 13: one 7.4 us against 6.4, eight 9.3 against 15.8; back, within 0.5
+// us of each other).
+inline bool mix_use(int N, long long items, bool forward) {
   int F[4];
   const int m = mix_factors(N, F);
   if (!m) return false;
   const int big = F[m - 1], M = czt_len(2 * N - 1);
+  if (M == 512 && forward && items <= 1000) return false;
   if (big <= 16 || M > 2048) return true;
-  if (M <= 512) return big < 97 && items > 1800;
-  if (M <= 1024) return big < 41 || items > 1600;
+  if (M <= 256) return big < 97 && items > 1400;
+  if (M == 512) return big < 97 && items > 2000;
+  if (M == 1024) return big < 41 || items > 1600;
   return big < 97 || items > 800;
 }
 
