@@ -477,8 +477,10 @@ template <int NT, bool SUM>
 static hipError_t sharp_launch(const SharpPlan& p, const float2* spectra, size_t spec_stride,
                                int nframes, int n, const double2* shifts, float2* S,
                                const float* wk, double2* part, hipStream_t st) {
+  // the same limit at every call: a smaller launch of another thread does not
+  // lower it between this call and its launch
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_sharp<NT, SUM>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, p.lds);
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((k_sharp<NT, SUM>), dim3(p.nchunks, p.nb), dim3(NT), p.lds, st, spectra,
                      spec_stride, nframes, p.FB, n, shifts, S, wk, part);

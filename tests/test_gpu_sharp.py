@@ -38,3 +38,31 @@ def test_sum_value_and_gradient_match_oracle(n, F, skip):
     scale = 1e-5 * np.abs(og).max() if len(keep) > 1 else 4e-7 * oJ
     assert np.abs(g[keep] - og).max() <= scale
     assert (g[list(skip)] == 0).all()
+
+
+def test_two_threads_of_different_lds():
+    """Contexts on two threads whose sharpness launches need 81 and 36 KB of the same
+    kernel's LDS: the values of each alone, bit for bit."""
+    import threading
+
+    n, out, alone = 128, {}, {}
+    rng = np.random.default_rng(11)
+    specs = {F: np.fft.rfft2(rng.normal(0, 1, (F, n, n))).astype(np.complex64) for F in (38, 16)}
+    shift = {F: rng.normal(0, 1.5, (F, 2)) for F in specs}
+
+    def run(F, reps, to):
+        ctx = mc.Context(0)
+        ctx.set_spectra(specs[F].view(np.float32))
+        to[F] = [ctx.sharpness(shift[F], 150.0) for _ in range(reps)]
+        ctx.close()
+
+    for F in specs:
+        run(F, 1, alone)
+    threads = [threading.Thread(target=run, args=(F, 40, out)) for F in specs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for F in specs:
+        j, g = alone[F][0]
+        assert len(out[F]) == 40 and all(a == j and np.array_equal(b, g) for a, b in out[F])
