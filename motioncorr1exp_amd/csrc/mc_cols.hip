@@ -227,8 +227,8 @@ __global__ __launch_bounds__(512, NG > 8 ? 3 : 4) void k_pair_cols64(
 // the next power of two above n + box: 1854, box 96, 78 pairs: 0.36 ms against
 // 0.83; 3710, 253 pairs: 3.9 against 5.0 for its decimated pass (53 FFTs of 70
 // points with five barriers per item); 4092, 55 pairs: 0.99 against 1.20.
-// Columns that do not start on 64 bytes cost: each four lanes' 64 bytes then
-// span two lines (3696, 105 pairs: 1.17 ms; 3710: 1.63).
+// 105 pairs: 3696 (R0 = 16) 1.17 ms, 3710 (R0 = 14) 1.63; the radix and the columns
+// of 3710 that do not start on 64 bytes were not measured apart.
 template <int R0, int TILES>
 __global__ __launch_bounds__(TILES == 1 || R0 <= 8 ? 1024 : 512, TILES == 1 || R0 <= 8 ? 4 : 3) void k_pair_cols_r(
     const float2* __restrict__ spectra, size_t spec_stride, const int2* __restrict__ pairs,
